@@ -205,7 +205,7 @@ struct Runner {
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   DevBuf in;
   DevBuf lut_buf;   // gradient tables of the resident frame
-  DevBuf src_count, src_off, bounds, segs, seg_cmd, mat_cnt, mat_off, mat_pres, list_off, list, binned, cursor, scan_tmp, counters, cmd_tiles;
+  DevBuf src_count, src_off, bounds, segs, seg_cmd, mat_cnt, mat_off, mat_pres, list_off, list, binned, scan_tmp, counters, cmd_tiles;
   DevBuf tile_hdr, group_hdr, tile_px, list_style, band_buf, item_cnt, item_off, items;
   DevBuf cm_params, cm_acc, cm_feat, cm_pred, cm_act;
   DevBuf cmd_err;
@@ -235,7 +235,6 @@ struct Runner {
   hipGraphExec_t graph_exec = nullptr;
   FrameScratch graph_s{};
   void* graph_q[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
-  uint32_t* graph_cursor = nullptr;
   uint64_t graph_gen = ~0ull, graph_model = ~0ull;
   uint32_t graph_sched = ~0u, graph_wgs = ~0u;
   ~Runner() {
@@ -281,6 +280,8 @@ struct Runner {
     return ((uint64_t)ilog2_u64((uint64_t)f.n_tiles + 1) << 40) | ((uint64_t)ilog2_u64((uint64_t)f.n_cmds + 1) << 20) |
            (uint64_t)ilog2_u64((uint64_t)f.n_canvases + 1);
   }
+  // Workgroups per analytic tile on the GRID schedule.
+  uint32_t strips_for(uint32_t n_a) const;
   // Launches the render stage: the analytic tiles in the schedule in force
   // (`allow_queue` false: GRID), the box tile groups one workgroup each.
   uint32_t render_stage(FrameScratch& s, uint32_t n_a, uint32_t n_f, uint32_t n_s, uint32_t n_g, bool allow_queue,
@@ -707,8 +708,7 @@ uint32_t Runner::execute_pool(Stats& stats, uint32_t mode) {
       !items.reserve(std::max<size_t>(item_cap, 1) * sizeof(EdgeItem)) ||
       !bounds.reserve((size_t)f.n_cmds * sizeof(CmdBounds)) || !mat_cnt.reserve((n_mat + 1) * 4) ||
       !mat_off.reserve((n_mat + 1) * 4) || !mat_pres.reserve((n_mat + 1) * 4) || !list_off.reserve((n_mat + 1) * 4) ||
-      !list.reserve((n_mat + 1) * 16) || !list_style.reserve((n_mat + 1) * 4) || !cursor.reserve((n_mat + 1) * 4) ||
-      !scan_tmp.reserve(scan_words * 4) ||
+      !list.reserve((n_mat + 1) * 16) || !list_style.reserve((n_mat + 1) * 8) || !scan_tmp.reserve(scan_words * 4) ||
       !counters.reserve(64) || !cmd_tiles.reserve((size_t)f.n_cmds * 4) ||
       !tile_hdr.reserve((size_t)f.n_tiles * 16) || !group_hdr.reserve((size_t)f.n_groups * 32) ||
       !band_buf.reserve(((size_t)f.n_bands + 1) * 40) || !tile_px.reserve((size_t)f.n_tiles * 8) ||
@@ -741,7 +741,8 @@ uint32_t Runner::execute_pool(Stats& stats, uint32_t mode) {
   s.mat_pres = mat_pres.as<uint32_t>();
   s.list_off = list_off.as<uint32_t>();
   s.list_ent = list.as<uint4>();
-  s.list_style = list_style.as<uint32_t>();
+  s.list_cols = list_style.as<uint32_t>();
+  s.list_style = s.list_cols + (n_mat + 1);
   s.scan_tmp = scan_tmp.as<uint32_t>();
   s.pixels = counters.as<unsigned long long>();
   s.seg_cursor = counters.as<uint32_t>() + 2;
@@ -798,9 +799,10 @@ uint32_t Runner::execute_pool(Stats& stats, uint32_t mode) {
   scan_exclusive(s.mat_cnt, s.mat_off, n_mat, s.scan_tmp, stream);
   scan_exclusive(s.mat_pres, s.list_off, n_mat, s.scan_tmp, stream);
   launch_band_class(f, s, stream);
-  HIP_OK(hipMemcpyAsync(cursor.ptr, s.mat_off, (n_mat + 1) * 4, hipMemcpyDeviceToDevice, stream));
-  launch_bin_scatter(f, s, cap_segs, cursor.as<uint32_t>(), stream);
   launch_list_build(f, s, stream);
+  // the presence flags are used up: their memory holds the scatter cursors
+  launch_copy_u32(s.mat_pres, s.mat_off, n_mat + 1, stream);
+  launch_bin_scatter(f, s, cap_segs, s.mat_pres, stream);
 
   // One read-back before the render stage: a pool overflow ends the frame
   // here (nothing composited; the caller redoes it exactly), otherwise the
@@ -880,6 +882,18 @@ void Runner::resolve_schedule(uint32_t n_a, bool allow_queue, uint32_t& sched, u
   if (wgs < 1 || wgs > 4) wgs = 4;
 }
 
+// A tile's workgroup is a serial chain of its commands, so a frame of few
+// tiles is rendered with less than one pixel quad per thread: a tile split in
+// strips of 8 or 4 rows has two or four times the waves to hide latency with.
+// The strips repeat the walk over the band's segments, which costs more than
+// it hides once the tiles fill the chip.  Measured on 1000 polygons (render
+// stage ms for 1 / 2 / 4 strips): 64 tiles 1.17 / 0.82 / 0.73, 256 tiles
+// 1.01 / 0.82 / 0.89, 512 tiles 1.12 / 1.02 / 1.22, 1024 tiles
+// 1.33 / 1.47 / 1.94.
+uint32_t Runner::strips_for(uint32_t n_a) const {
+  return n_a * 2ull <= cus ? 4u : n_a <= cus * 2ull ? 2u : 1u;
+}
+
 uint32_t Runner::render_stage(FrameScratch& s, uint32_t n_a, uint32_t n_f, uint32_t n_s, uint32_t n_g, bool allow_queue,
                               Stats& stats) {
   uint32_t sched, wgs;
@@ -887,7 +901,7 @@ uint32_t Runner::render_stage(FrameScratch& s, uint32_t n_a, uint32_t n_f, uint3
   stats.schedule = sched;
   stats.queue_wgs = sched == BL_AMD_SCHEDULE_GRID ? 0u : wgs;
   if (sched == BL_AMD_SCHEDULE_GRID) {
-    launch_render(f, s, n_a, n_f, n_s, n_g, stream);
+    launch_render(f, s, n_a, strips_for(n_a), n_f, n_s, n_g, stream);
     return BL_AMD_SUCCESS;
   }
   const bool ordered = sched != BL_AMD_SCHEDULE_QUEUE;
@@ -915,7 +929,7 @@ uint32_t Runner::render_stage(FrameScratch& s, uint32_t n_a, uint32_t n_f, uint3
   if (ordered) launch_tile_queue(f, s, n_a, learned ? q_pred.as<float>() : nullptr, stream);
   const uint32_t grid = std::min<uint32_t>(n_a, std::max<uint32_t>(cus, 1) * wgs);
   launch_render_queue(f, s, grid, wgs, stream);
-  launch_render(f, s, 0, n_f, n_s, n_g, stream);
+  launch_render(f, s, 0, 1, n_f, n_s, n_g, stream);
   return BL_AMD_SUCCESS;
 }
 
@@ -948,7 +962,6 @@ uint32_t Runner::execute_exact(Stats& stats, ScratchArena* arena, const ExactPla
   s.mat_off = (uint32_t*)take(mat_off, (n_mat + 1) * 4);
   s.mat_pres = (uint32_t*)take(mat_pres, (n_mat + 1) * 4);
   s.list_off = (uint32_t*)take(list_off, (n_mat + 1) * 4);
-  uint32_t* cursor_p = (uint32_t*)take(cursor, (n_mat + 1) * 4);
   s.scan_tmp = (uint32_t*)take(scan_tmp, scan_words * 4);
   uint32_t* counters_p = (uint32_t*)take(counters, 64);
   s.cmd_tiles = (uint32_t*)take(cmd_tiles, (size_t)f.n_cmds * 4);
@@ -958,7 +971,7 @@ uint32_t Runner::execute_exact(Stats& stats, ScratchArena* arena, const ExactPla
   s.tile_px = (unsigned long long*)take(tile_px, (size_t)f.n_tiles * 8);
   s.cmd_err = (uint32_t*)take(cmd_err, (size_t)f.n_cmds * 4);
   if (!s.item_cnt || !s.item_off || !s.items || !s.src_count || !s.src_off || !s.bounds || !s.mat_cnt || !s.mat_off ||
-      !s.mat_pres || !s.list_off || !cursor_p || !s.scan_tmp || !counters_p || !s.cmd_tiles || !s.tile_hdr ||
+      !s.mat_pres || !s.list_off || !s.scan_tmp || !counters_p || !s.cmd_tiles || !s.tile_hdr ||
       !s.group_hdr || !s.band_nonsolid || !s.tile_px || !s.cmd_err)
     return kErrFit;
   s.band_tiles = s.band_nonsolid + (f.n_bands + 1);
@@ -1026,8 +1039,9 @@ uint32_t Runner::execute_exact(Stats& stats, ScratchArena* arena, const ExactPla
     s.seg_cmd = (uint32_t*)take(seg_cmd, (size_t)std::max<uint32_t>(known->n_segs, 1) * 4);
     s.binned = (DevSeg*)take(binned, (size_t)std::max<uint32_t>(known->n_binned, 1) * sizeof(DevSeg));
     s.list_ent = (uint4*)take(list, (size_t)std::max<uint32_t>(known->n_list, 1) * 16);
-    s.list_style = (uint32_t*)take(list_style, (size_t)std::max<uint32_t>(known->n_list, 1) * 4);
-    if (!s.segs || !s.seg_cmd || !s.binned || !s.list_ent || !s.list_style) return kErrOOM;
+    s.list_cols = (uint32_t*)take(list_style, (size_t)std::max<uint32_t>(known->n_list, 1) * 8);
+    if (!s.segs || !s.seg_cmd || !s.binned || !s.list_ent || !s.list_cols) return kErrOOM;
+    s.list_style = s.list_cols + std::max<uint32_t>(known->n_list, 1);
     resolve_schedule(known->n_atiles, true, g_sched, g_wgs);
     if (g_sched != BL_AMD_SCHEDULE_GRID) {
       const size_t n_a = known->n_atiles;
@@ -1043,12 +1057,11 @@ uint32_t Runner::execute_exact(Stats& stats, ScratchArena* arena, const ExactPla
       q_ptrs[3] = q_feat.ptr; q_ptrs[4] = q_pred.ptr; q_ptrs[5] = tm_params.ptr;
     }
     const bool same = graph_exec && graph_gen == gen && graph_sched == g_sched && graph_wgs == g_wgs &&
-                      graph_model == g_tile_model_version && graph_cursor == cursor_p &&
+                      graph_model == g_tile_model_version &&
                       memcmp(&graph_s, &s, sizeof(s)) == 0 && memcmp(graph_q, q_ptrs, sizeof(q_ptrs)) == 0;
     if (same) return run_graph();
     if (graph_exec) { (void)hipGraphExecDestroy(graph_exec); graph_exec = nullptr; }
     graph_s = s;
-    graph_cursor = cursor_p;
     memcpy(graph_q, q_ptrs, sizeof(q_ptrs));
     HIP_OK(hipStreamBeginCapture(stream, hipStreamCaptureModeRelaxed));
     capture.on = true;
@@ -1134,12 +1147,14 @@ uint32_t Runner::execute_exact(Stats& stats, ScratchArena* arena, const ExactPla
       return kErrDevice;
     s.binned = (DevSeg*)take(binned, (size_t)std::max<uint32_t>(n_binned, 1) * sizeof(DevSeg));
     s.list_ent = (uint4*)take(list, (size_t)std::max<uint32_t>(n_list, 1) * 16);
-    s.list_style = (uint32_t*)take(list_style, (size_t)std::max<uint32_t>(n_list, 1) * 4);
-    if (!s.binned || !s.list_ent || !s.list_style) return kErrFit;
+    s.list_cols = (uint32_t*)take(list_style, (size_t)std::max<uint32_t>(n_list, 1) * 8);
+    if (!s.binned || !s.list_ent || !s.list_cols) return kErrFit;
+    s.list_style = s.list_cols + std::max<uint32_t>(n_list, 1);
   }
-  launch_copy_u32(cursor_p, s.mat_off, n_mat + 1, stream);
-  launch_bin_scatter(f, s, n_segs, cursor_p, stream);
   launch_list_build(f, s, stream);
+  // the presence flags are used up: their memory holds the scatter cursors
+  launch_copy_u32(s.mat_pres, s.mat_off, n_mat + 1, stream);
+  launch_bin_scatter(f, s, n_segs, s.mat_pres, stream);
 
   // Stage 3: render.
   launch_render_setup(f, s, stream);

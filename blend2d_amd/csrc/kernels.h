@@ -49,8 +49,10 @@ struct FrameScratch {
   uint32_t* mat_off;       // n_mat + 1
   uint32_t* mat_pres;      // n_mat + 1
   uint32_t* list_off;      // n_mat + 1
-  uint4* list_ent;         // n_list: per listed (band, command) cell {command, tile-column range, binned offset, binned count}
-  uint32_t* list_style;    // n_list: style index of the entry's command
+  // Per listed (band, command) cell:
+  uint32_t* list_cols;     // n_list: tile-column range, first | last << 16
+  uint4* list_ent;         // n_list: {command, binned offset, binned count, kMeta* bits}
+  uint32_t* list_style;    // n_list: solid colour, or the style index of another kind of style
   DevSeg* binned;          // n_binned
   uint32_t* scan_tmp;      // scan_tmp_words(max n)
   unsigned long long* pixels;  // composited pixels (mask > 0), summed after render
@@ -92,6 +94,11 @@ struct FrameScratch {
   uint32_t* tile_cycles;   // <= n_tiles: logged wall-clock ticks per slot (null: not logged)
 };
 
+// What the compositor branches on, one word per list entry: CmdKind in bits
+// 0-1, then at these bits ExecOp (3), alpha (8), even-odd (1), FetchKind (3)
+// and the source format (2).
+constexpr uint32_t kMetaOp = 2, kMetaAlpha = 5, kMetaEvenOdd = 13, kMetaFetch = 14, kMetaFmt = 17;
+
 size_t scan_tmp_words(size_t n);
 void scan_exclusive(const uint32_t* in, uint32_t* out, size_t n, uint32_t* tmp, hipStream_t s);
 
@@ -116,7 +123,8 @@ void launch_cmd_tiles(const FrameDev& f, const FrameScratch& s, hipStream_t st);
 // start at zero (stats).
 void launch_band_class(const FrameDev& f, const FrameScratch& s, hipStream_t st);
 void launch_render_setup(const FrameDev& f, const FrameScratch& s, hipStream_t st);
-void launch_render(const FrameDev& f, const FrameScratch& s, uint32_t n_a, uint32_t n_f, uint32_t n_s, uint32_t n_g,
+// `strips`: workgroups per analytic tile (1, 2 or 4).
+void launch_render(const FrameDev& f, const FrameScratch& s, uint32_t n_a, uint32_t strips, uint32_t n_f, uint32_t n_s, uint32_t n_g,
                    hipStream_t st);
 void launch_render_stats(const FrameDev& f, const FrameScratch& s, hipStream_t st);
 // Work-queue form of the analytic-tile render: features of the (at most n_a)

@@ -5,8 +5,8 @@
 //            emit pass at prefix-scanned offsets).
 //   bin      per segment: count, scatter into (band, command) lists; per band
 //            a compacted, submission-ordered list of the commands touching it.
-//   render   one 256-thread workgroup per 64x16 tile: the destination tile is
-//            loaded once into registers (128-bit per lane), every command of
+//   render   one 256-thread workgroup per 64x16 tile (or strip of it): the
+//            destination is loaded once into registers, every command of
 //            the band is rasterized into LDS cells with LDS atomics, turned
 //            into coverage by a per-scanline DPP scan, fetched, composited
 //            in submission order, and the tile is stored once.
@@ -727,8 +727,15 @@ void launch_bin_scatter(const FrameDev& f, const FrameScratch& s, uint32_t n_seg
 }
 
 // Command lists of the bands: every present (band, command) cell becomes one
-// entry, in command order within its band, carrying what the render filter
-// and the record loads need (so they are one dependent load away).
+// entry, in command order within its band: the tile-column range (the render
+// filter reads only this), {command, binned offset, binned count, what the
+// compositor branches on}, and the colour of a solid style or the style index
+// of another, so a solid fill needs no command or style record at all.
+__device__ __forceinline__ uint32_t cmd_meta(const DevCmd& c, uint32_t fetch_kind) {
+  return c.kind | (c.op << kMetaOp) | (c.alpha << kMetaAlpha) | ((c.rule_mask == 0x1FFu ? 1u : 0u) << kMetaEvenOdd) |
+         (fetch_kind << kMetaFetch) | (c.src_fmt << kMetaFmt);
+}
+
 __global__ void k_list_build(FrameDev f, FrameScratch s, uint64_t n) {
   uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n || !s.mat_pres[i]) return;
@@ -741,8 +748,11 @@ __global__ void k_list_build(FrameDev f, FrameScratch s, uint64_t n) {
   const DevCanvas& cv = f.canvases[lo];
   const uint32_t cmd = cv.cmd_base + (uint32_t)((i - cv.mat_base) % cv.n_cmds);
   const uint32_t li = s.list_off[i];
-  s.list_ent[li] = make_uint4(cmd, s.cmd_tiles[cmd], s.mat_off[i], s.mat_cnt[i]);
-  s.list_style[li] = f.cmds[cmd].style;
+  const DevCmd& c = f.cmds[cmd];
+  const DevStyle& st = f.styles[c.style];
+  s.list_cols[li] = s.cmd_tiles[cmd];
+  s.list_ent[li] = make_uint4(cmd, s.mat_off[i], s.mat_cnt[i], cmd_meta(c, st.kind));
+  s.list_style[li] = st.kind == kFetchSolid ? st.solid : c.style;
 }
 
 void launch_list_build(const FrameDev& f, const FrameScratch& s, hipStream_t st) {
@@ -782,37 +792,54 @@ void launch_cmd_tiles(const FrameDev& f, const FrameScratch& s, hipStream_t st) 
 // Stage 3: render
 // ---------------------------------------------------------------------------
 
-// LDS cell buffer of one command in a tile: 16 rows x 64 cells, then one
-// backdrop word per row (the summed contributions of cells left of the tile).
-// Within a row the 16 groups of four cells are stored XOR-swizzled by the
-// row index, so the same cell column of different rows (the rows of one
+// LDS cell buffer of one command in a tile strip: its rows x 64 cells, then
+// one backdrop word per row (the summed contributions of cells left of the
+// tile).  Within a row the 16 groups of four cells are stored XOR-swizzled by
+// the row index, so the same cell column of different rows (the rows of one
 // steep edge, rasterized by neighbouring lanes) falls into different LDS
 // banks; a group stays four consecutive words, so the compositor still
 // reads a thread's four cells with one 128-bit load.
-constexpr int kCellWords = kTileH * kTileW + kTileH;
-constexpr int kBackdrop = kTileH * kTileW;
-
 __device__ __forceinline__ int cell_index(int row, int x) {
   return row * kTileW + ((((x >> 2) ^ row) & 15) << 2) + (x & 3);
 }
 
-__device__ __forceinline__ uint32_t calc_mask(uint32_t cov, uint32_t rule_mask, uint32_t alpha) {
-  uint32_t m = ((uint32_t)((int32_t)cov >> 9) & rule_mask) - 256u;
-  int32_t mi = (int32_t)m;
-  uint32_t a = (uint32_t)(mi < 0 ? -mi : mi);
-  a = a > 256u ? 256u : a;
-  return (a * alpha) >> 8;
+// Cross-lane moves on the VALU (DPP): lanes without a source keep `old`.
+template<int kCtrl, int kRowMask>
+__device__ __forceinline__ uint32_t dpp(uint32_t old, uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp((int)old, (int)v, kCtrl, kRowMask, 0xF, false);
 }
 
-__device__ __forceinline__ uint32_t row_excl_scan16(uint32_t v) {
-  const int q = threadIdx.x & 15;
-  uint32_t incl = v;
-#pragma unroll
-  for (int d = 1; d < 16; d <<= 1) {
-    uint32_t t = __shfl_up(incl, d, 16);
-    if (q >= d) incl += t;
-  }
-  return incl - v;
+// Inclusive prefix sum (maximum) within groups of W = 16, 32 or 64 lanes, all
+// lanes active: row shifts by 1, 2, 4 and 8, then the last lane of a row (of
+// 16) added to the next row, of the lower half to the upper.
+template<int W>
+__device__ __forceinline__ uint32_t lane_scan_add(uint32_t v) {
+  v += dpp<0x111, 0xF>(0u, v);
+  v += dpp<0x112, 0xF>(0u, v);
+  v += dpp<0x114, 0xF>(0u, v);
+  v += dpp<0x118, 0xF>(0u, v);
+  if (W >= 32) v += dpp<0x142, 0xA>(0u, v);
+  if (W >= 64) v += dpp<0x143, 0xC>(0u, v);
+  return v;
+}
+__device__ __forceinline__ uint32_t wave_scan_max(uint32_t v) {
+  v = max(v, dpp<0x111, 0xF>(0u, v));
+  v = max(v, dpp<0x112, 0xF>(0u, v));
+  v = max(v, dpp<0x114, 0xF>(0u, v));
+  v = max(v, dpp<0x118, 0xF>(0u, v));
+  v = max(v, dpp<0x142, 0xA>(0u, v));
+  v = max(v, dpp<0x143, 0xC>(0u, v));
+  return v;
+}
+// LDS written by lanes of this wave is visible to its other lanes after this
+// (a wave's LDS operations execute in order; the fence holds the compiler).
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+}
+__device__ __forceinline__ uint32_t lane_value(uint32_t v, uint32_t lane) {
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)lane);
 }
 
 // Per-command record staged in LDS for the render loop.
@@ -829,16 +856,9 @@ union RenderRec {
 constexpr int kRecWords = (int)(sizeof(RenderRecData) / 4);
 static_assert(sizeof(DevCmd) % 8 == 0, "DevStyle must stay 8-byte aligned in the record");
 
-// Commands rasterized together.  The segments of a batch's commands are
-// spread over all lanes of the workgroup, each command into its own LDS cell
-// buffer; after one barrier every thread composites its pixels through the
-// batch's commands in submission order.  Rasterization of different commands
-// is independent, so only the composite has to follow the command order.
-#ifndef B2AMD_RENDER_BATCH
-#define B2AMD_RENDER_BATCH 7
-#endif
-constexpr int kBatch = B2AMD_RENDER_BATCH;
-static_assert(kBatch >= 1 && kBatch * kRecWords <= 2 * kTileThreads, "two record words per thread");
+// Records staged together by the box compositor (double buffered).
+constexpr int kBatch = 7;
+static_assert(kBatch * kRecWords <= 2 * kTileThreads, "two record words per thread");
 
 // Word `w` of the record of command `cmd_i` (style index `style_i`).
 __device__ __forceinline__ uint32_t rec_word(const FrameDev& f, const FrameScratch& s, uint32_t cmd_i, uint32_t style_i, int w) {
@@ -856,45 +876,18 @@ __device__ __forceinline__ uint32_t batch_rec_word(const FrameDev& f, const Fram
   return rec_word(f, s, sel_cmd[kb + b], sel_style[kb + b], w);
 }
 
-// Inclusive prefix of the segment counts of the batch's `nb` commands.
-__device__ __forceinline__ void batch_prefix(const uint32_t* sel_cnt, uint32_t kb, uint32_t nb, uint32_t end[kBatch]) {
-  uint32_t acc = 0;
-#pragma unroll
-  for (int b = 0; b < kBatch; b++) {
-    acc += (uint32_t)b < nb ? sel_cnt[kb + b] : 0u;
-    end[b] = acc;
-  }
-}
-
-// Batch slot and in-command index of the batch's segment `j` (j < end[kBatch - 1]).
-__device__ __forceinline__ uint32_t batch_find(const uint32_t end[kBatch], uint32_t j, uint32_t* local) {
-  uint32_t b = 0, base = 0;
-#pragma unroll
-  for (int i = 0; i < kBatch - 1; i++) {
-    if (j >= end[i]) { b = (uint32_t)i + 1u; base = end[i]; }
-  }
-  *local = j - base;
-  return b;
-}
-
-// Tile rows one raster task covers (a task pays the rasterizer's set-up and
-// advance once for its rows).
-#ifndef B2AMD_ROWS_PER_TASK
-#define B2AMD_ROWS_PER_TASK 1
-#endif
-constexpr int kRowsPerTask = B2AMD_ROWS_PER_TASK;
-
-// First pass over one binned segment of an analytic fill: a segment right of
-// the tile is dropped; one left of it adds its signed vertical extent per
-// covered row to the backdrop; for one that reaches the tile the number of
-// raster tasks for the tile rows it covers is returned (raster_rows).
-__device__ __forceinline__ uint32_t seg_tile_rows(const DevSeg& g, uint32_t* cells, int X0, int Y0) {
+// First pass over one binned segment of an analytic fill, for the rows
+// [Y0, Y0 + rows) of a tile: a segment right of the tile is dropped; one left
+// of it adds its signed vertical extent per covered row to the backdrop; for
+// one that reaches the tile the number of rows it covers is returned, each a
+// raster task.
+__device__ __forceinline__ uint32_t seg_tile_rows(const DevSeg& g, uint32_t* backdrop, int X0, int Y0, int rows) {
   const int32_t x1 = g.x1 & 0x7FFFFFFF;
   const int32_t cmin = (g.x0 < x1 ? g.x0 : x1) >> 8;
   const int32_t cmax = (g.x0 < x1 ? x1 : g.x0) >> 8;
   int r0 = g.y0 >> 8, r1 = (g.y1 - 1) >> 8;
   if (r0 < Y0) r0 = Y0;
-  if (r1 > Y0 + kTileH - 1) r1 = Y0 + kTileH - 1;
+  if (r1 > Y0 + rows - 1) r1 = Y0 + rows - 1;
   if (cmin >= X0 + kTileW || r1 < r0) return 0u;
   if (cmax + 1 < X0) {
     // every cell of every row lies left of the tile: each row adds its y
@@ -903,28 +896,24 @@ __device__ __forceinline__ uint32_t seg_tile_rows(const DevSeg& g, uint32_t* cel
     for (int r = r0; r <= r1; r++) {
       const int lo_y = g.y0 > r * 256 ? g.y0 : r * 256;
       const int hi_y = g.y1 < (r + 1) * 256 ? g.y1 : (r + 1) * 256;
-      atomicAdd(&cells[kBackdrop + r - Y0], (uint32_t)(sgn * (hi_y - lo_y)) << 9);
+      atomicAdd(&backdrop[r - Y0], (uint32_t)ras::with_sign(hi_y - lo_y, sgn) << 9);
     }
     return 0u;
   }
-  return (uint32_t)((r1 - r0 + kRowsPerTask) / kRowsPerTask);
+  return (uint32_t)(r1 - r0 + 1);
 }
 
-// Rows `row` .. `row` + kRowsPerTask - 1 (within the tile) of a segment that
-// reaches the tile: the closed-form row emitter adds the cells inside the
-// tile and one backdrop value per row for the cells left of it.
-__device__ __forceinline__ void raster_rows(const DevSeg& g, uint32_t* cells, int X0, int Y0, int row) {
+// Row `r` of a segment that reaches the tile: the closed-form row emitter adds
+// the cells inside the tile and one backdrop value for the cells left of it.
+__device__ __forceinline__ void raster_row(const DevSeg& g, uint32_t* cells, uint32_t* backdrop, int X0, int Y0, int r) {
   ras::Edge e;
   if (!ras::edge_init(e, g.x0, g.y0, g.x1 & 0x7FFFFFFF, g.y1)) return;
   const int32_t sgn = g.x1 < 0 ? -1 : 1;
-  const int last = row + kRowsPerTask - 1 < e.row1 ? row + kRowsPerTask - 1 : e.row1;
-  for (int r = row; r <= last && r < Y0 + kTileH; r++) {
-    const int lr = r - Y0;
-    const uint32_t bd = ras::emit_row(e, r, X0, kTileW, sgn, [&](int32_t k, uint32_t v) {
-      if (v) atomicAdd(&cells[cell_index(lr, k)], v);
-    });
-    if (bd) atomicAdd(&cells[kBackdrop + lr], bd);
-  }
+  const int lr = r - Y0;
+  const uint32_t bd = ras::emit_row(e, r, X0, kTileW, sgn, [&](int32_t k, uint32_t v) {
+    if (v) atomicAdd(&cells[cell_index(lr, k)], v);
+  });
+  if (bd) atomicAdd(&backdrop[lr], bd);
 }
 
 // Destination pixels px .. px + 3 of a row (zero where outside the canvas).
@@ -1032,31 +1021,6 @@ __device__ __forceinline__ uint32_t composite4(const FrameDev& f, const DevCmd& 
   return n;
 }
 
-// The same with all four fetches issued before the first is used, so their
-// gradient-LUT / texel loads are in flight together (more registers).
-template<bool kDither>
-__device__ __forceinline__ uint32_t composite4_overlapped(const FrameDev& f, const DevCmd& c, const DevStyle& st,
-                                                          const pipe::Row& rs, int px, int w, bool a8,
-                                                          const uint32_t m[4], uint32_t d[4]) {
-  constexpr bool kSolid = false;
-  bool on[4];
-  uint32_t src[4];
-#pragma unroll
-  for (int k = 0; k < 4; k++) {
-    on[k] = m[k] && px + k < w;
-    src[k] = 0u;
-    if (on[k]) src[k] = kSolid ? st.solid : pipe::fetch<kDither>(st, rs, px + k, f.luts, f.images, c.src_fmt);
-  }
-  uint32_t n = 0;
-#pragma unroll
-  for (int k = 0; k < 4; k++) {
-    if (!on[k]) continue;
-    d[k] = a8 ? pipe::composite8(c.op, d[k], src[k] >> 24, m[k]) : pipe::composite32(c.op, d[k], src[k], m[k]);
-    n++;
-  }
-  return n;
-}
-
 // Workgroup -> tile.  Workgroups are dealt to the 8 XCDs round-robin; the
 // mapping gives each XCD a contiguous range of tiles, so the tiles of a band
 // (which read the same command lists, records and segments) share one L2.
@@ -1066,270 +1030,479 @@ __device__ __forceinline__ uint32_t xcd_tile(uint32_t wg, uint32_t n_tiles) {
   return (wg % kXcds) * per + wg / kXcds;
 }
 
-// One analytic tile (header `slot`): the whole workgroup rasterizes the
-// band's commands that reach the tile and composites them in order.
-template<bool kDither>
-__device__ __forceinline__ void render_tile(const FrameDev& f, const FrameScratch& s, uint32_t slot) {
-  __shared__ uint32_t cells[kBatch][kCellWords];
+// Analytic tiles.
+//
+// What bounds them: instruction issue.  Rasterization is one row of one
+// segment per lane, compositing a few dozen integer instructions per pixel and
+// command; a tile's destination is read and written once.  So the work is laid
+// out for few instructions per command and no waiting on memory in between:
+//
+//  - everything that belongs to a command is wave-uniform: its list entry
+//    arrives in a lane of the wave (63 selected entries at a time) and is read
+//    into scalar registers with v_readlane; branches on its kind, operator and
+//    style are scalar, other records are scalar loads;
+//  - cross-lane sums are DPP moves on the VALU, not LDS permutes;
+//  - pixels stay in registers as 16-bit pairs for the packed 16-bit
+//    instructions, and a wave with one mask for all its pixels under a solid
+//    colour forms the source terms once, in scalar registers;
+//  - a wave whose rows a command does not touch skips it after one look at its
+//    cells.
+//
+// Each thread holds N pixels of a row (4, 2 or 1), so a workgroup of four
+// waves covers 64 x 4N pixels: a whole 16-row tile, or a half or quarter strip
+// of it (see strips_for).
+//
+// Measured against records in LDS, permute scans and 64-bit divisions per row
+// (render stage, one workgroup per tile): 1024 glyph canvases 3.49 -> 1.86 ms
+// (VALU instructions 1177 -> 720 million, the VALU three quarters busy),
+// 10 000 gradient cubics at 1920x1080 4.60 -> 2.77, 2000 pattern shapes at
+// 3840x2160 2.04 -> 1.41, 32 canvases of uneven paths 4.22 -> 2.60, 1000
+// polygons at 512x512 2.17 -> 1.01 (0.82 in two strips).
+//
+// Commands rasterized together.  The segments of a batch's commands are
+// spread over all lanes of the workgroup, each command into its own LDS cell
+// buffer; after one barrier every wave composites its rows through the
+// batch's commands in submission order.  Rasterization of different commands
+// is independent, so only the composite has to follow the command order.
+constexpr uint32_t kTileBatch = 7;
+constexpr uint32_t kTileGroup = 64u / kTileBatch * kTileBatch;   // selected entries held by a wave
+
+// Masks of pixels px .. px + N - 1 of row y for a box fill (uniform command).
+template<int N>
+__device__ __forceinline__ void box_masks_n(const FrameDev& f, pipe::CPtr<DevCmd> c, uint32_t kind, uint32_t alpha, int y, int px,
+                                            uint32_t m[N]) {
+  const int bx0 = c->box[0], by0 = c->box[1], bx1 = c->box[2], by1 = c->box[3];
+  const bool row_in = y >= by0 && y < by1;
+  if (kind == kCmdBoxA) {
+#pragma unroll
+    for (int k = 0; k < N; k++) m[k] = (row_in && px + k >= bx0 && px + k < bx1) ? alpha : 0u;
+  }
+  else if (kind == kCmdBoxM) {
+    // FillMask with a VMaskA8 command (rendercommandprocsync_p.h:65-84,
+    // compopgeneric_p.h:165-183): byte x - x0 of the mask row, times the
+    // alpha below full alpha.  The view is exactly the box (host-checked), so
+    // every byte read lies in row y - y0 of the view.
+    const pipe::CPtr<DevImage> mi = pipe::cptr(f.images + c->box_mask[0]);
+    const pipe::GBytes row = pipe::global_bytes(mi->ptr) + (int64_t)(y - by0) * mi->stride - bx0;
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+      m[k] = 0u;
+      if (row_in && px + k >= bx0 && px + k < bx1) m[k] = row[px + k];
+    }
+    if (alpha < 255u) {
+#pragma unroll
+      for (int k = 0; k < N; k++) m[k] = pipe::div255(m[k] * alpha);
+    }
+  }
+  else {
+    const uint32_t top = c->box_mask[0], mid = c->box_mask[1], bot = c->box_mask[2];
+    const uint32_t rm = y == c->box_row_first ? top : y == c->box_row_last ? bot : mid;
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+      const int x = px + k;
+      const uint32_t sh = x == bx0 ? 0u : x == bx1 - 1 ? 16u : 8u;
+      m[k] = (row_in && x >= bx0 && x < bx1) ? (rm >> sh) & 0xFFu : 0u;
+    }
+  }
+}
+
+// One command's pixels: fetch and composite under masks m.
+template<int N, bool kDither>
+__device__ __forceinline__ void apply_n(const FrameDev& f, const FrameScratch& s, uint32_t meta, uint32_t cmd, uint32_t style,
+                                        bool a8, uint32_t ref_band_h, int y, int px, const uint32_t m[N], pipe::Px d[N]) {
+  const uint32_t op = (meta >> kMetaOp) & 7u, fetch = (meta >> kMetaFetch) & 7u;
+  constexpr int kPairs = (N + 1) / 2;
+  uint32_t src[N];
+  if (fetch == kFetchSolid) {
+    if (!a8 && op <= kOpSrcOver) {
+      const uint32_t m0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)m[0]);
+      uint32_t diff = m[0] ^ m0;
+#pragma unroll
+      for (int k = 1; k < N; k++) diff |= m[k] ^ m0;
+      if (__ballot(diff != 0u) == 0ull) {
+        pipe::composite32_flat<N>(op, d, style, m0);
+        return;
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < N; k++) src[k] = style;
+  }
+  else {
+    uint32_t any = m[0];
+#pragma unroll
+    for (int k = 1; k < N; k++) any |= m[k];
+#pragma unroll
+    for (int k = 0; k < N; k++) src[k] = 0u;
+    if (any) {
+      int row0 = 0;
+      const bool analytic = (meta & 3u) == kCmdAnalytic;
+      if (fetch == kFetchConic) row0 = analytic ? pipe::cptr(s.bounds + cmd)->min_y >> 8 : (int)pipe::cptr(f.cmds + cmd)->fetch_row0;
+      pipe::fetch_n<N, kDither>(pipe::cptr(f.styles + style), fetch, y, px, row0, analytic ? ref_band_h : 0u, f.luts, f.images,
+                                (meta >> kMetaFmt) & 3u, src);
+    }
+  }
+  if (a8) {
+    pipe::u16x2 da[kPairs], sa[kPairs], ma[kPairs];
+#pragma unroll
+    for (int k = 0; k < kPairs; k++) {
+      da[k] = d[k].rb;
+      const uint32_t k1 = 2 * k + 1 < N ? 2 * k + 1 : 2 * k;
+      sa[k] = pipe::u16x2{(uint16_t)(src[2 * k] >> 24), (uint16_t)(src[k1] >> 24)};
+      ma[k] = pipe::u16x2{(uint16_t)m[2 * k], (uint16_t)m[k1]};
+    }
+    pipe::composite8_n<kPairs>(op, da, sa, ma);
+#pragma unroll
+    for (int k = 0; k < kPairs; k++) d[k].rb = da[k];
+    return;
+  }
+  pipe::Px sp[N];
+#pragma unroll
+  for (int k = 0; k < N; k++) sp[k] = pipe::px_of(src[k]);
+  pipe::composite32_n<N>(op, d, sp, m, fetch >= kFetchPatternNN);
+}
+
+// Destination pixels px .. px + N - 1 of a row, as pairs (A8: neighbouring
+// pixels in d[k].rb); zero outside the canvas.
+template<int N>
+__device__ __forceinline__ void load_px(const uint8_t* rowp, int px, int w, bool a8, pipe::Px d[N]) {
+  uint32_t v[N];
+#pragma unroll
+  for (int k = 0; k < N; k++) v[k] = 0u;
+  if (a8) {
+    if (N == 4 && px + 3 < w && (((uintptr_t)(rowp + px)) & 3) == 0) {
+      const uint32_t b = *(const uint32_t*)(rowp + px);
+#pragma unroll
+      for (int k = 0; k < N; k++) v[k] = (b >> (8 * k)) & 0xFFu;
+    }
+    else {
+#pragma unroll
+      for (int k = 0; k < N; k++) if (px + k < w) v[k] = rowp[px + k];
+    }
+#pragma unroll
+    for (int k = 0; k < (N + 1) / 2; k++) d[k].rb = pipe::u16x2{(uint16_t)v[2 * k], (uint16_t)(2 * k + 1 < N ? v[2 * k + 1 < N ? 2 * k + 1 : 0] : 0u)};
+    return;
+  }
+  const uint32_t* r32 = (const uint32_t*)rowp;
+  if (N == 4 && px + 3 < w && (((uintptr_t)(r32 + px)) & 15) == 0) {
+    const uint4 q = *(const uint4*)(r32 + px);
+    const uint32_t u[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+    for (int k = 0; k < N; k++) v[k] = u[k];
+  }
+  else {
+#pragma unroll
+    for (int k = 0; k < N; k++) if (px + k < w) v[k] = r32[px + k];
+  }
+#pragma unroll
+  for (int k = 0; k < N; k++) d[k] = pipe::px_of(v[k]);
+}
+
+template<int N>
+__device__ __forceinline__ void store_px(uint8_t* rowp, int px, int w, bool a8, const pipe::Px d[N]) {
+  if (a8) {
+    uint32_t v[N];
+#pragma unroll
+    for (int k = 0; k < N; k++) v[k] = (pipe::as_u32(d[k / 2].rb) >> (16 * (k & 1))) & 0xFFu;
+    if (N == 4 && px + 3 < w && (((uintptr_t)(rowp + px)) & 3) == 0) {
+      uint32_t b = 0;
+#pragma unroll
+      for (int k = 0; k < N; k++) b |= v[k] << (8 * k);
+      *(uint32_t*)(rowp + px) = b;
+    }
+    else {
+#pragma unroll
+      for (int k = 0; k < N; k++) if (px + k < w) rowp[px + k] = (uint8_t)v[k];
+    }
+    return;
+  }
+  uint32_t* r32 = (uint32_t*)rowp;
+  uint32_t v[N];
+#pragma unroll
+  for (int k = 0; k < N; k++) v[k] = pipe::px_bits(d[k]);
+  if (N == 4 && px + 3 < w && (((uintptr_t)(r32 + px)) & 15) == 0) {
+    *(uint4*)(r32 + px) = make_uint4(v[0], v[1 % N], v[2 % N], v[3 % N]);
+  }
+  else {
+#pragma unroll
+    for (int k = 0; k < N; k++) if (px + k < w) r32[px + k] = v[k];
+  }
+}
+
+// Rows strip * 4N .. + 4N - 1 of the analytic tile with header `slot`: the
+// whole workgroup rasterizes the band's commands that reach the tile and
+// composites them in order.
+template<int N, bool kDither>
+__device__ __forceinline__ void render_tile(const FrameDev& f, const FrameScratch& s, uint32_t slot, uint32_t strip) {
+  constexpr int kRows = 4 * N, kLanes = kTileW / N;   // rows of the strip, lanes per row
+  constexpr int kCells = kRows * kTileW, kCellWords = kCells + kRows;
+  constexpr uint32_t kB = kTileBatch;
+  __shared__ __align__(16) uint32_t cells[kB][kCellWords];
+  // Row tasks, per wave: the segments that reach the strip, each with its
+  // first task index and batch slot, and the owners of the next 64 tasks.
+  __shared__ DevSeg task_seg[kTileThreads / 64][64];
+  __shared__ uint32_t task_meta[kTileThreads / 64][64];
+  __shared__ uint32_t task_own[kTileThreads / 64][64];
+  __shared__ uint8_t sel[kTileThreads];
+  __shared__ uint32_t sel_wave[kTileThreads / 64];
   const int t = threadIdx.x;
-  const uint4 th = s.tile_hdr[slot];
-  const DevCanvas cv = f.canvases[th.x];
-  const uint32_t lb = th.y, le = th.z;
-  const uint32_t tcol = th.w & 0xFFFFu;
-  const uint32_t band = th.w >> 16;
-  const uint32_t tile = cv.tile_base + band * cv.tiles_x + tcol;
+  const int lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const uint32_t* const hdr = (const uint32_t*)(s.tile_hdr + slot);
+  const pipe::CPtr<uint32_t> th = pipe::cptr(hdr);
+  const pipe::CPtr<DevCanvas> cv = pipe::cptr(f.canvases + th[0]);
+  const uint32_t lb = th[1], le = th[2];
+  const uint32_t tcol = th[3] & 0xFFFFu, band = th[3] >> 16;
+  const uint32_t tile = cv->tile_base + band * cv->tiles_x + tcol;
   // A pool overflow leaves the frame incomplete: nothing is composited and
   // the host redoes the frame with exact counting.
   if (s.flags && *s.flags) {
-    if (t == 0) s.tile_px[tile] = 0;
+    if (t == 0 && N == 4) s.tile_px[tile] = 0;
     return;
   }
   const int X0 = (int)tcol * kTileW;
-  const int Y0 = (int)band * kTileH;
+  const int Y0 = (int)band * kTileH + (int)strip * kRows;
+  const int w = (int)cv->w;
+  const bool a8 = cv->format == kFmtA8;
+  const uint32_t ref_band_h = cv->ref_band_h;
 
-  const int row = t >> 4;
-  const int q = t & 15;
+  const int row = wave * N + lane / kLanes;   // within the strip
+  const int q = lane % kLanes;
   const int y = Y0 + row;
-  const int px = X0 + q * 4;
-  const bool row_ok = y < (int)cv.h;
-  const bool a8 = cv.format == kFmtA8;
-
-  // zero LDS (each thread its own swizzled group of four cells)
-  const int grp = cell_index(row, q * 4);
+  const int px = X0 + q * N;
+  const bool row_ok = y < (int)cv->h;
+  // Lanes whose pixel k lies inside the canvas.  The others are composited
+  // like any (every fetch is safe at any position) but not counted or stored.
+  uint64_t inside[N];
 #pragma unroll
-  for (int b = 0; b < kBatch; b++) *(uint4*)&cells[b][grp] = make_uint4(0, 0, 0, 0);
-  for (int i = t; i < kBatch * kTileH; i += kTileThreads) cells[i / kTileH][kBackdrop + i % kTileH] = 0;
+  for (int k = 0; k < N; k++) inside[k] = __ballot(row_ok && px + k < w);
 
-  // load the destination tile
-  uint32_t d[4] = {0, 0, 0, 0};
-  uint8_t* rowp = (uint8_t*)cv.ptr + (int64_t)y * cv.stride;
-  if (row_ok) load4(rowp, px, (int)cv.w, a8, d);
+  // zero LDS (each thread its own swizzled group of cells)
+  const int grp = cell_index(row, q * N);
+#pragma unroll
+  for (uint32_t b = 0; b < kB; b++) {
+#pragma unroll
+    for (int k = 0; k < N; k++) cells[b][grp + k] = 0u;
+    if (q == 0) cells[b][kCells + row] = 0u;
+  }
 
-  const int lane = t & 63, wave = t >> 6;
+  // load the destination pixels
+  pipe::Px d[N];
+#pragma unroll
+  for (int k = 0; k < N; k++) d[k] = pipe::px_of(0u);
+  uint8_t* const rowp = (uint8_t*)cv->ptr + (int64_t)y * cv->stride;
+  if (row_ok) load_px<N>(rowp, px, w, a8, d);
+
   // Batch segment index of this thread in the first 256 of a batch: the
   // batch's segments are dealt to the four waves in turn, so every SIMD of
   // the CU takes part in rasterization.
   const uint32_t jt = ((uint32_t)lane << 2) | (uint32_t)wave;
   bool touched = false;
-  uint32_t npix = 0;
+  uint32_t npix = 0;   // composited pixels of the wave
 
   // The band's command list is filtered 256 entries at a time down to the
   // commands whose tile-column range holds this tile (ballot compaction,
-  // submission order kept); the filter also gathers, in parallel, each
-  // selected command's (band, command) cell extent and style index.
-  __shared__ uint32_t sel_cmd[kTileThreads], sel_off[kTileThreads], sel_cnt[kTileThreads], sel_style[kTileThreads];
-  __shared__ uint32_t sel_wave[kTileThreads / 64];
-  // Row tasks of the segments that reach the tile: the segment of each
-  // thread, and its first task index (low 12 bits) and batch slot (bits 12+).
-  __shared__ DevSeg task_seg[kTileThreads];
-  __shared__ uint16_t task_start[kTileThreads];
-  __shared__ uint32_t task_wave[kTileThreads / 64];
-  // Records (command, style, fill-row origin) of the batch being applied
-  // and of the next one (double buffer): the next batch's records and first
-  // 256 segments are loaded while the current batch is rasterized and
-  // composited, so the chain of dependent global loads is off the critical
-  // path.
-  __shared__ RenderRec rec[2][kBatch];
-
+  // submission order kept).
   for (uint32_t chunk = lb; chunk < le; chunk += kTileThreads) {
     const uint32_t li = chunk + (uint32_t)t;
-    uint4 ent = make_uint4(0, 0, 0, 0);
-    uint32_t style_i = 0;
     bool keep = false;
     if (li < le) {
-      ent = s.list_ent[li];
-      style_i = s.list_style[li];
-      keep = tcol >= (ent.y & 0xFFFFu) && tcol <= (ent.y >> 16);
+      const uint32_t cols = s.list_cols[li];
+      keep = tcol >= (cols & 0xFFFFu) && tcol <= (cols >> 16);
     }
     const uint64_t bal = __ballot(keep);
     if (lane == 0) sel_wave[wave] = (uint32_t)__popcll(bal);
-    __syncthreads();
+    __syncthreads();   // also: the previous chunk's selection is consumed
     uint32_t off = 0, n_sel = 0;
 #pragma unroll
-    for (int w = 0; w < kTileThreads / 64; w++) {
-      const uint32_t cw = sel_wave[w];
-      off += w < wave ? cw : 0u;
+    for (int v = 0; v < kTileThreads / 64; v++) {
+      const uint32_t cw = sel_wave[v];
+      off += v < wave ? cw : 0u;
       n_sel += cw;
     }
-    if (keep) {
-      const uint32_t slot = off + (uint32_t)__popcll(bal & ((1ull << lane) - 1ull));
-      sel_cmd[slot] = ent.x;
-      sel_off[slot] = ent.z;
-      sel_cnt[slot] = ent.w;
-      sel_style[slot] = style_i;
-    }
+    if (keep) sel[off + (uint32_t)__popcll(bal & ((1ull << lane) - 1ull))] = (uint8_t)t;
     __syncthreads();
-    if (n_sel == 0) continue;   // uniform; sel_wave is rewritten only after the next chunk's ballot
+    n_sel = (uint32_t)__builtin_amdgcn_readfirstlane((int)n_sel);
 
-    // first batch of the chunk: records and first segments
-    DevSeg pre_seg{0, 0, 0, 0};
-    uint32_t pre_b = 0;
-    {
-      const uint32_t nb = n_sel < (uint32_t)kBatch ? n_sel : (uint32_t)kBatch;
-      uint32_t end[kBatch];
-      batch_prefix(sel_cnt, 0, nb, end);
-      if (t < (int)nb * kRecWords) rec[0][t / kRecWords].w[t % kRecWords] = batch_rec_word(f, s, sel_cmd, sel_style, 0, t);
-      if (t + kTileThreads < (int)nb * kRecWords) {
-        const int gw = t + kTileThreads;
-        rec[0][gw / kRecWords].w[gw % kRecWords] = batch_rec_word(f, s, sel_cmd, sel_style, 0, gw);
+    for (uint32_t g0 = 0; g0 < n_sel; g0 += kTileGroup) {
+      // up to kTileGroup selected entries, one per lane
+      const uint32_t gn = min(n_sel - g0, kTileGroup);
+      uint4 ent = make_uint4(0u, 0u, 0u, 0u);
+      uint32_t style = 0;
+      if ((uint32_t)lane < gn) {
+        const uint32_t i = chunk + sel[g0 + (uint32_t)lane];
+        ent = s.list_ent[i];
+        style = s.list_style[i];
       }
-      if (jt < end[kBatch - 1]) {
-        uint32_t loc;
-        pre_b = batch_find(end, jt, &loc);
-        pre_seg = s.binned[sel_off[pre_b] + loc];
-      }
-    }
-    __syncthreads();
+      const uint32_t incl = lane_scan_add<64>(ent.z);      // segments up to and with this entry
+      const uint32_t delta = ent.y - (incl - ent.z);       // binned index of group segment j: delta + j
 
-    for (uint32_t kb = 0, bi = 0; kb < n_sel; kb += kBatch, bi++) {
-      const int cur = (int)(bi & 1u);
-      const uint32_t nb = n_sel - kb < (uint32_t)kBatch ? n_sel - kb : (uint32_t)kBatch;
-      uint32_t end[kBatch];
-      batch_prefix(sel_cnt, kb, nb, end);
-      const uint32_t total = end[kBatch - 1];
-      const DevSeg seg = pre_seg;
-      const uint32_t seg_b = pre_b;
-
-      // prefetch the next batch
-      const uint32_t kn = kb + kBatch;
-      const bool has_next = kn < n_sel;
-      uint32_t pw0 = 0, pw1 = 0;
-      int nwn = 0;
-      if (has_next) {
-        const uint32_t nbn = n_sel - kn < (uint32_t)kBatch ? n_sel - kn : (uint32_t)kBatch;
-        nwn = (int)nbn * kRecWords;
-        if (t < nwn) pw0 = batch_rec_word(f, s, sel_cmd, sel_style, kn, t);
-        if (t + kTileThreads < nwn) pw1 = batch_rec_word(f, s, sel_cmd, sel_style, kn, t + kTileThreads);
-        uint32_t endn[kBatch];
-        batch_prefix(sel_cnt, kn, nbn, endn);
-        pre_seg = DevSeg{0, 0, 0, 0};
-        pre_b = 0;
-        if (jt < endn[kBatch - 1]) {
-          uint32_t loc;
-          pre_b = batch_find(endn, jt, &loc);
-          pre_seg = s.binned[sel_off[kn + pre_b] + loc];
+      // the batch's segment `j` (of `total`, the first being group segment
+      // `base`): its batch slot and record
+      auto find = [&](uint32_t kb, uint32_t nb, uint32_t base, uint32_t j, DevSeg& g) -> uint32_t {
+        uint32_t b = 0;
+#pragma unroll
+        for (uint32_t i = 0; i + 1 < kB; i++) {
+          const uint32_t end = i + 1 < nb ? lane_value(incl, kb + i) - base : 0xFFFFFFFFu;
+          b += j >= end ? 1u : 0u;
         }
-      }
+        const uint32_t at = (uint32_t)__shfl((int)delta, (int)(kb + b), 64) + base + j;
+        g = s.binned[at];
+        return b;
+      };
+      // (every lane calls it, so the shuffle sees all lanes; lanes past the
+      // batch's segments look at its first one and drop it)
+      auto batch_n = [&](uint32_t kb) { return min(gn - kb, kB); };
+      auto batch_base = [&](uint32_t kb) { return kb ? lane_value(incl, kb - 1u) : 0u; };
+      auto batch_total = [&](uint32_t kb) { return lane_value(incl, kb + batch_n(kb) - 1u) - batch_base(kb); };
+      DevSeg pre{0, 0, 0, 0};
+      uint32_t pre_b = 0;
+      uint32_t total = batch_total(0);
+      if (total) pre_b = find(0, batch_n(0), 0u, jt < total ? jt : 0u, pre);
 
-      // Rasterize the batch.  Segments left of the tile add their row
-      // covers to the backdrop; every segment that reaches the tile becomes
-      // one task per tile row it covers, so a lane's serial cell walk is one
-      // row long and the rows are spread over all lanes.
-      for (uint32_t rb = 0; rb < total; rb += kTileThreads) {
-        const uint32_t j = rb + jt;
-        DevSeg g = seg;
-        uint32_t gb = seg_b;
-        if (rb) {
-          g = DevSeg{0, 0, 0, 0};
-          gb = 0;
-          if (j < total) {
-            uint32_t loc;
-            gb = batch_find(end, j, &loc);
-            g = s.binned[sel_off[kb + gb] + loc];
+      for (uint32_t kb = 0; kb < gn; kb += kB) {
+        const uint32_t nb = batch_n(kb), base = batch_base(kb);
+        const uint32_t tot = total;
+        const DevSeg seg = pre;
+        const uint32_t seg_b = pre_b;
+        // the next batch's first segments are on their way while this batch
+        // is rasterized and composited
+        if (kb + kB < gn) {
+          total = batch_total(kb + kB);
+          if (total) pre_b = find(kb + kB, batch_n(kb + kB), batch_base(kb + kB), jt < total ? jt : 0u, pre);
+        }
+
+        // Rasterize the batch.  Segments left of the tile add their row
+        // covers to the backdrop; every segment that reaches the strip
+        // becomes one task per row it covers, so a lane's serial cell walk
+        // is one row long.  A wave's tasks are its own segments': no barrier.
+        for (uint32_t rb = 0; rb < tot; rb += kTileThreads) {
+          const uint32_t j = rb + jt;
+          DevSeg g = seg;
+          uint32_t gb = seg_b;
+          if (rb) gb = find(kb, nb, base, j < tot ? j : 0u, g);
+          const uint32_t rows = j < tot ? seg_tile_rows(g, &cells[gb][kCells], X0, Y0, kRows) : 0u;
+          const uint32_t tend = lane_scan_add<64>(rows);
+          const uint32_t n_tasks = lane_value(tend, 63u);
+          if (n_tasks == 0) continue;
+          const uint32_t first = tend - rows;
+          if (rows) {
+            task_seg[wave][lane] = g;
+            task_meta[wave][lane] = first | (gb << 16);
+          }
+          uint32_t carry = 0;   // owner of the task before this window, + 1
+          for (uint32_t k0 = 0; k0 < n_tasks; k0 += 64) {
+            // owner of each task of the window: the last segment whose first
+            // task is at or before it
+            task_own[wave][lane] = 0u;
+            wave_sync();
+            if (rows && first - k0 < 64u) task_own[wave][first - k0] = (uint32_t)lane + 1u;
+            wave_sync();
+            const uint32_t own = max(wave_scan_max(task_own[wave][lane]), carry);
+            carry = lane_value(own, 63u);
+            const uint32_t k = k0 + (uint32_t)lane;
+            if (k < n_tasks) {
+              const uint32_t o = own - 1u;
+              const DevSeg og = task_seg[wave][o];
+              const uint32_t tm = task_meta[wave][o];
+              const int r0 = (og.y0 >> 8) > Y0 ? (og.y0 >> 8) : Y0;
+              uint32_t* cb = cells[tm >> 16];
+              raster_row(og, cb, cb + kCells, X0, Y0, r0 + (int)(k - (tm & 0xFFFFu)));
+            }
+            wave_sync();
           }
         }
-        const uint32_t rows = j < total ? seg_tile_rows(g, cells[gb], X0, Y0) : 0u;
-        uint32_t incl = rows;
-#pragma unroll
-        for (int dd = 1; dd < 64; dd <<= 1) {
-          const uint32_t v = __shfl_up(incl, dd, 64);
-          if (lane >= dd) incl += v;
-        }
-        if (lane == 63) task_wave[wave] = incl;
-        if (rows) task_seg[t] = g;
-        __syncthreads();
-        uint32_t before = 0, n_tasks = 0;
-#pragma unroll
-        for (int w = 0; w < kTileThreads / 64; w++) {
-          const uint32_t cw = task_wave[w];
-          before += w < wave ? cw : 0u;
-          n_tasks += cw;
-        }
-        task_start[t] = (uint16_t)((before + incl - rows) | (gb << 12));
-        __syncthreads();
-        for (uint32_t k = (uint32_t)t; k < n_tasks; k += kTileThreads) {
-          // owner: the last thread whose first task index is <= k
-          int o = 0;
-#pragma unroll
-          for (int step = kTileThreads / 2; step > 0; step >>= 1)
-            if ((uint32_t)(task_start[o + step] & 0xFFFu) <= k) o += step;
-          const uint32_t ts = task_start[o];
-          const DevSeg og = task_seg[o];
-          const int r0 = (og.y0 >> 8) > Y0 ? (og.y0 >> 8) : Y0;
-          raster_rows(og, cells[ts >> 12], X0, Y0, r0 + kRowsPerTask * (int)(k - (ts & 0xFFFu)));
-        }
-        __syncthreads();   // cells complete (and task arrays free for the next round)
-      }
+        if (tot) __syncthreads();   // cells complete
 
-      // composite the batch's commands in order
-      for (uint32_t b = 0; b < nb; b++) {
-        const DevCmd& c = rec[cur][b].r.cmd;
-        uint32_t m[4] = {0, 0, 0, 0};
-
-        if (c.kind == kCmdAnalytic) {
-          uint32_t* cb = cells[b];
-          uint4 cv4 = *(uint4*)&cb[grp];
-          uint32_t bdv = cb[kBackdrop + row];
-          *(uint4*)&cb[grp] = make_uint4(0, 0, 0, 0);
-          uint32_t sum = cv4.x + cv4.y + cv4.z + cv4.w;
-          uint32_t base = (256u << 9) + bdv + row_excl_scan16(sum);
-          // every lane of the row has read the backdrop before the scan
-          if (q == 0) cb[kBackdrop + row] = 0;
-          uint32_t c0 = base + cv4.x, c1 = c0 + cv4.y, c2 = c1 + cv4.z, c3 = c2 + cv4.w;
-          m[0] = calc_mask(c0, c.rule_mask, c.alpha);
-          m[1] = calc_mask(c1, c.rule_mask, c.alpha);
-          m[2] = calc_mask(c2, c.rule_mask, c.alpha);
-          m[3] = calc_mask(c3, c.rule_mask, c.alpha);
-        }
-        else {
-          box_masks4(f, c, y, px, m);
-        }
-
-        if (row_ok && (m[0] | m[1] | m[2] | m[3]) != 0) {
+        // composite the batch's commands in order
+        for (uint32_t b = 0; b < nb; b++) {
+          const uint32_t p = kb + b;
+          const uint32_t meta = lane_value(ent.w, p);
+          const uint32_t alpha = (meta >> kMetaAlpha) & 0xFFu;
+          uint32_t m[N];
+          if ((meta & 3u) == kCmdAnalytic) {
+            if (lane_value(ent.z, p) == 0u) continue;
+            uint32_t* cb = cells[b];
+            uint32_t c[N];
+#pragma unroll
+            for (int k = 0; k < N; k++) c[k] = cb[grp + k];
+            const uint32_t bd = cb[kCells + row];
+            uint32_t any = c[0];
+#pragma unroll
+            for (int k = 1; k < N; k++) any |= c[k];
+            const uint64_t has = __ballot(any != 0u);
+            if ((has | __ballot(bd != 0u)) == 0ull) continue;   // nothing covers the wave's rows
+            uint32_t cov = bd;
+            if (has) {
+              uint32_t sum = c[0];
+#pragma unroll
+              for (int k = 1; k < N; k++) sum += c[k];
+              cov += lane_scan_add<kLanes>(sum) - sum;
+#pragma unroll
+              for (int k = 0; k < N; k++) cb[grp + k] = 0u;
+            }
+            if (q == 0) cb[kCells + row] = 0u;
+            // coverage (cov / 512, rounded down) to mask: its magnitude up
+            // to 256, folded into [0, 256] first under the even-odd rule
+            if ((meta >> kMetaEvenOdd) & 1u) {
+#pragma unroll
+              for (int k = 0; k < N; k++) {
+                cov += c[k];
+                const int32_t v = (((int32_t)cov >> 9) + 256 & 0x1FF) - 256;
+                m[k] = __umul24((uint32_t)(v < 0 ? -v : v), alpha) >> 8;
+              }
+            }
+            else {
+#pragma unroll
+              for (int k = 0; k < N; k++) {
+                cov += c[k];
+                const int32_t v = (int32_t)cov >> 9;
+                m[k] = __umul24(min((uint32_t)max(v, -v), 256u), alpha) >> 8;
+              }
+            }
+          }
+          else {
+            box_masks_n<N>(f, pipe::cptr(f.cmds + lane_value(ent.x, p)), meta & 3u, alpha, y, px, m);
+          }
+          uint32_t n = 0;
+#pragma unroll
+          for (int k = 0; k < N; k++) n += (uint32_t)__popcll(__ballot(m[k] != 0u) & inside[k]);
+          if (n == 0) continue;
+          npix += n;
           touched = true;
-          const DevStyle& st = rec[cur][b].r.style;
-          const int fill_row0 = (c.kind == kCmdAnalytic) ? (rec[cur][b].r.min_y >> 8) : (int)c.fetch_row0;
-          const pipe::Row rs = pipe::row_setup(st, y, fill_row0, c.kind == kCmdAnalytic ? cv.ref_band_h : 0u);
-          npix += composite4_overlapped<kDither>(f, c, st, rs, px, (int)cv.w, a8, m, d);
+          apply_n<N, kDither>(f, s, meta, lane_value(ent.x, p), lane_value(style, p), a8, ref_band_h, y, px, m, d);
         }
+        if (tot) __syncthreads();   // cells cleared
       }
-      if (has_next) {
-        if (t < nwn) rec[cur ^ 1][t / kRecWords].w[t % kRecWords] = pw0;
-        if (t + kTileThreads < nwn) {
-          const int gw = t + kTileThreads;
-          rec[cur ^ 1][gw / kRecWords].w[gw % kRecWords] = pw1;
-        }
-      }
-      __syncthreads();   // next records visible; cells cleared; these records no longer read
     }
   }
 
-  // Composited-pixel statistics: one value per tile, summed by k_sum_u64.
+  // Composited-pixel statistics: one value per tile, summed by k_sum_u64
+  // (strips add to their tile's, which k_tile_setup zeroed).
   __shared__ uint32_t wave_px[kTileThreads / 64];
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) npix += __shfl_xor(npix, o, 64);
   if (lane == 0) wave_px[wave] = npix;
   __syncthreads();
   if (t == 0) {
     unsigned long long tp = 0;
 #pragma unroll
-    for (int w = 0; w < kTileThreads / 64; w++) tp += wave_px[w];
-    s.tile_px[tile] = tp;
+    for (int v = 0; v < kTileThreads / 64; v++) tp += wave_px[v];
+    if (N == 4) s.tile_px[tile] = tp;
+    else if (tp) atomicAdd(&s.tile_px[tile], tp);
   }
 
-  if (!touched || !row_ok) return;
-  store4(rowp, px, (int)cv.w, a8, d);
+  if (touched && row_ok) store_px<N>(rowp, px, w, a8, d);
 }
 
 // Four workgroups per CU: LDS (7 cell buffers) and the register budget are
-// sized for it.  One workgroup per analytic tile, XCD-contiguous.
-template<bool kDither>
+// sized for it.  One workgroup per analytic tile or strip, XCD-contiguous.
+template<int N, bool kDither>
 __global__ __launch_bounds__(kTileThreads, 4) void k_render(FrameDev f, FrameScratch s, uint32_t n) {
-  const uint32_t slot = xcd_tile(blockIdx.x, n);
+  constexpr uint32_t kStrips = 4 / N;
+  const uint32_t unit = xcd_tile(blockIdx.x, n * kStrips);
+  const uint32_t slot = unit / kStrips;
   // uniform: padding workgroups of the XCD mapping, and (when n is an upper
   // bound) slots past the analytic tiles
   if (slot >= n || slot >= s.tile_off[f.n_bands]) return;
-  render_tile<kDither>(f, s, slot);
+  render_tile<N, kDither>(f, s, slot, unit % kStrips);
 }
 
 // The same tiles drained from a work queue by a persistent grid: every
@@ -1351,11 +1524,11 @@ __global__ __launch_bounds__(kTileThreads, kOcc) void k_render_queue(FrameDev f,
     if (i >= total) break;   // uniform
     const uint32_t slot = s.queue ? s.queue[i] : i;
     if constexpr (!kLog) {
-      render_tile<kDither>(f, s, slot);
+      render_tile<4, kDither>(f, s, slot, 0);
     }
     else {
       const long long c0 = wall_clock64();
-      render_tile<kDither>(f, s, slot);
+      render_tile<4, kDither>(f, s, slot, 0);
       __syncthreads();
       if (threadIdx.x == 0) {
         s.tile_cycles[slot] = (uint32_t)min((long long)0xFFFFFFFF, wall_clock64() - c0);
@@ -1392,22 +1565,22 @@ __global__ __launch_bounds__(256) void k_tile_features(FrameDev f, FrameScratch 
   const uint32_t tcol = th.w & 0xFFFFu, band = th.w >> 16;
   uint32_t c[12] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};   // n, segs, segs_left, lin, rad, con, pat, solid, box, op, -, max
   for (uint32_t li = th.y + lane; li < th.z; li += 64) {
-    const uint4 ent = s.list_ent[li];
-    const uint32_t lo = ent.y & 0xFFFFu, hi = ent.y >> 16;
+    const uint32_t cols = s.list_cols[li];
+    const uint32_t lo = cols & 0xFFFFu, hi = cols >> 16;
     if (tcol < lo || tcol > hi) continue;
-    const DevCmd& cmd = f.cmds[ent.x];
-    const uint32_t kind = f.styles[s.list_style[li]].kind;
+    const uint4 ent = s.list_ent[li];
+    const uint32_t kind = (ent.w >> kMetaFetch) & 7u;
     c[0] += 1u;
-    c[1] += ent.w;
-    c[2] += lo < tcol ? ent.w : 0u;
+    c[1] += ent.z;
+    c[2] += lo < tcol ? ent.z : 0u;
     c[3] += kind == kFetchLinear;
     c[4] += kind == kFetchRadial;
     c[5] += kind == kFetchConic;
     c[6] += kind >= kFetchPatternNN;
     c[7] += kind == kFetchSolid;
-    c[8] += cmd.kind != kCmdAnalytic;
-    c[9] += cmd.op != kOpSrcOver;
-    c[11] = ent.w > c[11] ? ent.w : c[11];
+    c[8] += (ent.w & 3u) != kCmdAnalytic;
+    c[9] += ((ent.w >> kMetaOp) & 7u) != kOpSrcOver;
+    c[11] = ent.z > c[11] ? ent.z : c[11];
   }
 #pragma unroll
   for (int k = 0; k < 12; k++) {
@@ -1433,7 +1606,7 @@ __global__ __launch_bounds__(256) void k_tile_features(FrameDev f, FrameScratch 
   o[11] = cv.format == kFmtA8 ? 1.0f : 0.0f;
   o[12] = (float)rows / (float)kTileH;
   o[13] = (float)cols / (float)kTileW;
-  o[14] = log2f(1.0f + (float)((c[0] + kBatch - 1) / kBatch));
+  o[14] = log2f(1.0f + (float)((c[0] + kTileBatch - 1) / kTileBatch));
   o[15] = log2f(1.0f + (float)c[11]);
 }
 
@@ -1548,6 +1721,7 @@ __global__ void k_tile_setup(FrameDev f, FrameScratch s) {
   const uint32_t local = i - cv.tile_base;
   const uint32_t band = local / cv.tiles_x, col = local % cv.tiles_x;
   const uint32_t gb = cv.band_base + band;
+  s.tile_px[i] = 0;
   if (!s.band_tiles[gb]) return;
   const uint64_t row_base = cv.mat_base + (uint64_t)band * cv.n_cmds;
   s.tile_hdr[s.tile_off[gb] + col] = make_uint4(lo, s.list_off[row_base], s.list_off[row_base + cv.n_cmds], col | (band << 16));
@@ -1660,13 +1834,13 @@ __device__ __forceinline__ void render_box(const FrameDev& f, const FrameScratch
 
   for (uint32_t chunk = lb; chunk < le; chunk += kTileThreads) {
     const uint32_t li = chunk + (uint32_t)t;
-    uint4 ent = make_uint4(0, 0, 0, 0);
-    uint32_t style_i = 0;
+    uint32_t cmd_i = 0, style_i = 0;
     bool keep = false;
     if (li < le) {
-      ent = s.list_ent[li];
-      style_i = s.list_style[li];
-      keep = (ent.y & 0xFFFFu) <= tc1 && (ent.y >> 16) >= tc0;
+      const uint32_t cols = s.list_cols[li];
+      cmd_i = s.list_ent[li].x;
+      style_i = f.cmds[cmd_i].style;
+      keep = (cols & 0xFFFFu) <= tc1 && (cols >> 16) >= tc0;
     }
     const uint64_t bal = __ballot(keep);
     if (lane == 0) sel_wave[wave] = (uint32_t)__popcll(bal);
@@ -1680,7 +1854,7 @@ __device__ __forceinline__ void render_box(const FrameDev& f, const FrameScratch
     }
     if (keep) {
       const uint32_t slot = off + (uint32_t)__popcll(bal & ((1ull << lane) - 1ull));
-      sel_cmd[slot] = ent.x;
+      sel_cmd[slot] = cmd_i;
       sel_style[slot] = style_i;
     }
     __syncthreads();
@@ -1856,7 +2030,7 @@ __global__ __launch_bounds__(kTileThreads, 8) void k_render_box_fast(FrameDev f,
     if ((uint32_t)t < nc) {
       const DevCmd& c = f.cmds[s.list_ent[chunk + t].x];
       rec[t] = FastBoxRec{c.box[0], c.box[1], c.box[2], c.box[3], c.alpha | (c.op << 8),
-                          f.styles[s.list_style[chunk + t]].solid};
+                          s.list_style[chunk + t]};
     }
     __syncthreads();
     for (uint32_t k = 0; k < nc; k++) {
@@ -1943,13 +2117,25 @@ void launch_render_setup(const FrameDev& f, const FrameScratch& s, hipStream_t s
   hipLaunchKernelGGL(k_group_setup, dim3((f.n_groups + 255) / 256), dim3(256), 0, st, f, s);
 }
 
-void launch_render(const FrameDev& f, const FrameScratch& s, uint32_t n_a, uint32_t n_f, uint32_t n_s, uint32_t n_g,
+void launch_render(const FrameDev& f, const FrameScratch& s, uint32_t n_a, uint32_t strips, uint32_t n_f, uint32_t n_s, uint32_t n_g,
                    hipStream_t st) {
   if (!f.n_tiles) return;
   // frames with dithered gradients take the instances that carry the dither
   // path; the others leave it out
-  if (n_a && f.dither) hipLaunchKernelGGL(k_render<true>, dim3((n_a + kXcds - 1) / kXcds * kXcds), dim3(kTileThreads), 0, st, f, s, n_a);
-  else if (n_a) hipLaunchKernelGGL(k_render<false>, dim3((n_a + kXcds - 1) / kXcds * kXcds), dim3(kTileThreads), 0, st, f, s, n_a);
+  if (n_a) {
+    const uint32_t units = n_a * strips;
+    const dim3 grid((units + kXcds - 1) / kXcds * kXcds), block(kTileThreads);
+    if (strips == 4) {
+      if (f.dither) hipLaunchKernelGGL((k_render<1, true>), grid, block, 0, st, f, s, n_a);
+      else hipLaunchKernelGGL((k_render<1, false>), grid, block, 0, st, f, s, n_a);
+    }
+    else if (strips == 2) {
+      if (f.dither) hipLaunchKernelGGL((k_render<2, true>), grid, block, 0, st, f, s, n_a);
+      else hipLaunchKernelGGL((k_render<2, false>), grid, block, 0, st, f, s, n_a);
+    }
+    else if (f.dither) hipLaunchKernelGGL((k_render<4, true>), grid, block, 0, st, f, s, n_a);
+    else hipLaunchKernelGGL((k_render<4, false>), grid, block, 0, st, f, s, n_a);
+  }
   if (n_f) hipLaunchKernelGGL(k_render_box_fast, dim3((n_f + kXcds - 1) / kXcds * kXcds), dim3(kTileThreads), 0, st, f, s, n_f);
   if (n_s) hipLaunchKernelGGL(k_render_box_solid, dim3((n_s + kXcds - 1) / kXcds * kXcds), dim3(kTileThreads), 0, st, f, s, n_s);
   if (n_g && f.dither) hipLaunchKernelGGL(k_render_box<true>, dim3((n_g + kXcds - 1) / kXcds * kXcds), dim3(kTileThreads), 0, st, f, s, n_g);

@@ -39,81 +39,70 @@
 namespace b2amd {
 namespace ras {
 
-// floor(n / d) for d > 0.  Below 2^53 the quotient comes from the correctly
-// rounded double division: with Q = n / d < 2^53 / d the rounding error is
-// at most 2^-53 * Q < 1 / d, while a non-integral Q lies at least 1 / d away
-// from every integer, so truncating the rounded quotient gives floor(Q).
-// The 24.8 coordinates the rasterizer sees keep every dividend far below
-// 2^53; the integer division stays as the exact path for anything larger.
-B2AMD_HD uint64_t udiv_floor(uint64_t n, uint64_t d) {
-  if (n < (1ull << 53)) return (uint64_t)__builtin_trunc((double)n / (double)d);
-  return n / d;
+// 1 / d to within two units in the last place, d > 0.
+B2AMD_HD double recip(int32_t d) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const double x = (double)d;
+  double r = __builtin_amdgcn_rcp(x);
+  r = __builtin_fma(r, __builtin_fma(-x, r, 1.0), r);
+  return __builtin_fma(r, __builtin_fma(-x, r, 1.0), r);
+#else
+  return 1.0 / (double)d;
+#endif
 }
 
-// Coordinates beyond this magnitude never come out of the edge builder for a
-// canvas (it clips to the canvas in 24.8); an edge carrying one is ignored.
-constexpr int32_t kCoordLimit = 1 << 30;
+// floor(n / d) for an integral n, 0 <= n < 2^49, and inv = recip(d).  The
+// exact (n + 1/2) / d lies at least 1 / (2 d) away from every integer, and
+// the computed product is off by less than 2^-50 of itself (two ulps of inv
+// and one rounding): less than 1 / (2 d) while n < 2^49, so truncating it
+// gives the floor.  The dividends here stay below 2^24 * 2^24 + 2^24.
+B2AMD_HD int32_t div_floor(double n, double inv) { return (int32_t)((n + 0.5) * inv); }
 
+// A line moving left is handled as its mirror image (x -> -x) moving right:
+// the reference starts a cell right of a boundary point when moving right and
+// left of it when moving left, and measures the area from the other side, so
+// the two directions are exact mirror images.
 struct Edge {
-  int32_t x0, y0, x1, y1;  // 24.8, y0 < y1
-  int32_t dx, dy;          // |x1 - x0|, y1 - y0
-  int32_t dir;             // +1: x grows downwards (or constant), -1: x shrinks
+  int32_t x0, y0, x1, y1;  // 24.8, y0 < y1, x0 <= x1 (mirrored when `left`)
+  int32_t dx, dy;          // x1 - x0, y1 - y0
+  bool left;               // x shrinks downwards
   int32_t row0, row1;      // first and last pixel row it touches
-  int32_t top0;            // start y within row0 (0..255)
-  int32_t bot1;            // end y within row1 (1..256)
-  bool one_column;         // vertical, or within one cell: one cell column, constant area factor
   bool steep;              // dy >= dx: at most one column crossing per row
 };
 
-// Returns false for edges that add nothing (horizontal) or that no clipped
-// geometry can produce.
+// Returns false for edges that add nothing (horizontal).  Coordinates lie
+// within the canvas, at most 65535 pixels a side: the edge builder clips.
 B2AMD_HD bool edge_init(Edge& e, int32_t x0, int32_t y0, int32_t x1, int32_t y1) {
   if (y0 >= y1) return false;
-  if (x0 < -kCoordLimit || x0 > kCoordLimit || x1 < -kCoordLimit || x1 > kCoordLimit ||
-      y0 < -kCoordLimit || y1 > kCoordLimit)
-    return false;
-  e.x0 = x0; e.y0 = y0; e.x1 = x1; e.y1 = y1;
-  e.dir = x1 < x0 ? -1 : 1;
-  e.dx = x1 < x0 ? x0 - x1 : x1 - x0;
+  e.left = x1 < x0;
+  e.x0 = e.left ? -x0 : x0; e.y0 = y0;
+  e.x1 = e.left ? -x1 : x1; e.y1 = y1;
+  e.dx = e.x1 - e.x0;
   e.dy = y1 - y0;
   e.row0 = y0 >> 8;
   e.row1 = (y1 - 1) >> 8;
-  e.top0 = y0 & 255;
-  e.bot1 = ((y1 - 1) & 255) + 1;
-  e.one_column = (x0 >> 8) == (x1 >> 8) && (e.row0 == e.row1 || e.dx == 0);
   e.steep = e.dy >= e.dx;
   return true;
 }
 
-// x where the edge crosses the row boundary y = 256 k, row0 < k <= row1.
-B2AMD_HD int32_t x_at_row_boundary(const Edge& e, int32_t k) {
-  const uint64_t t = (uint64_t)(int64_t)(256 * (int64_t)k - e.y0);
-  const uint64_t q = udiv_floor(t * (uint64_t)e.dx + (uint64_t)(e.dy - (e.dy >> 1)), (uint64_t)e.dy);
-  return e.x0 + e.dir * (int32_t)q;
+// x where the edge crosses the row boundary y = 256 k, row0 < k <= row1;
+// inv_dy = recip(e.dy).
+B2AMD_HD int32_t x_at_row_boundary(const Edge& e, double inv_dy, int32_t k) {
+  const uint32_t half = (uint32_t)(uint64_t)(e.dy - (e.dy >> 1));
+  return e.x0 + div_floor(__builtin_fma((double)(256 * k - e.y0), (double)e.dx, (double)half), inv_dy);
 }
 
-// Crossings of consecutive column boundaries in the direction of travel:
-// the boundary at distance `dist` from x0 is crossed at y0 + q, and each
-// next boundary is 256 further.
-struct ColumnWalk {
-  uint64_t q, rem;          // quotient and remainder of dist * dy + ceil(dx / 2) by dx
-  uint64_t lift, lift_rem;  // the same of 256 * dy
-  uint64_t dx;
-  B2AMD_HD void start(const Edge& e, uint64_t dist) {
-    dx = (uint64_t)e.dx;
-    const uint64_t num = dist * (uint64_t)e.dy + (dx - (dx >> 1));
-    q = udiv_floor(num, dx);
-    rem = num - q * dx;
-    const uint64_t step = 256u * (uint64_t)e.dy;
-    lift = udiv_floor(step, dx);
-    lift_rem = step - lift * dx;
-  }
-  B2AMD_HD void next() {
-    q += lift;
-    rem += lift_rem;
-    if (rem >= dx) { q++; rem -= dx; }
-  }
-};
+// Product of two values below 2^23 in magnitude that fits 32 bits.
+B2AMD_HD int32_t mul_small(int32_t a, int32_t b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __mul24(a, b);
+#else
+  return a * b;
+#endif
+}
+
+// v * sgn for sgn = +1 or -1.
+B2AMD_HD int32_t with_sign(int32_t v, int32_t sgn) { return (v ^ (sgn >> 31)) - (sgn >> 31); }
 
 // Row `r` (row0 <= r <= row1) of edge `e`, with cover sign `sgn` (+1 or -1),
 // against a tile whose pixel columns are [x_left, x_left + width): calls
@@ -121,101 +110,63 @@ struct ColumnWalk {
 // backdrop, the cover << 9 of the row's cells left of the tile.
 template<typename Sink>
 B2AMD_HD uint32_t emit_row(const Edge& e, int32_t r, int32_t x_left, int32_t width, int32_t sgn, Sink&& sink) {
-  const int32_t ytop = r == e.row0 ? e.top0 : 0;
-  const int32_t ybot = r == e.row1 ? e.bot1 : 256;
-  const int32_t x_end = x_left + width;   // first column right of the tile
-
-  // One cell: cover over the row, area factor fsum.
-  auto single = [&](int32_t c, int32_t fsum) -> uint32_t {
-    const int32_t cover = sgn * (ybot - ytop);
-    if (c < x_left) return (uint32_t)cover << 9;
-    if (c < x_end) {
-      const int32_t area = cover * fsum;
-      sink(c - x_left, ((uint32_t)cover << 9) - (uint32_t)area);
-      if (c + 1 < x_end) sink(c + 1 - x_left, (uint32_t)area);
-    }
-    return 0u;
-  };
-
-  if (e.one_column) return single(e.x0 >> 8, (e.x0 & 255) + (e.x1 & 255));
-
-  const int32_t xe = r == e.row0 ? e.x0 : x_at_row_boundary(e, r);
-  const int32_t xx = r == e.row1 ? e.x1 : x_at_row_boundary(e, r + 1);
-  const int32_t run = e.dir > 0 ? xx - xe : xe - xx;   // >= 0
-
-  // Entry cell and entry offset: moving right a point on a boundary starts
-  // the cell right of it, moving left the cell left of it (offset 256).
-  int32_t ce, fe;
-  if (e.dir > 0) { ce = xe >> 8; fe = xe & 255; }
-  else { ce = (xe - 1) >> 8; fe = ((xe - 1) & 255) + 1; }
-  if (e.dir > 0 ? fe + run <= 256 : fe - run >= 0) return single(ce, e.dir > 0 ? 2 * fe + run : 2 * fe - run);
-
-  // Several cells, ce to cx in the direction of travel.
-  const int32_t cx = e.dir > 0 ? (xx - 1) >> 8 : xx >> 8;
-  const int32_t fx = e.dir > 0 ? ((xx - 1) & 255) + 1 : xx & 255;
-  const int32_t lo = e.dir > 0 ? ce : cx, hi = e.dir > 0 ? cx : ce;
-  if (hi < x_left) return (uint32_t)(sgn * (ybot - ytop)) << 9;
-  if (lo >= x_end) return 0u;
-
-  // In-tile cells in the direction of travel: first k0, last k1.
-  const int32_t k0 = e.dir > 0 ? (ce > x_left ? ce : x_left) : (ce < x_end - 1 ? ce : x_end - 1);
-  const int32_t k1 = e.dir > 0 ? (cx < x_end - 1 ? cx : x_end - 1) : (cx > x_left ? cx : x_left);
-  // Crossing y of the boundary a cell is entered through, row-relative.
   const int32_t row_y = 256 * r;
-  auto rel = [&](uint64_t q) -> int32_t {
-    const int32_t y = e.y0 + (int32_t)q;
+  const int32_t ytop = r == e.row0 ? e.y0 - row_y : 0;
+  const int32_t ybot = r == e.row1 ? e.y1 - row_y : 256;
+  // the tile's cells in the direction of travel: [w0, w1]
+  const int32_t w0 = e.left ? -(x_left + width) : x_left, w1 = w0 + width - 1;
+
+  const double inv_dy = recip(e.dy);
+  const int32_t xt = x_at_row_boundary(e, inv_dy, r), xb = x_at_row_boundary(e, inv_dy, r + 1);
+  const int32_t xe = r == e.row0 ? e.x0 : xt;
+  const int32_t xx = r == e.row1 ? e.x1 : xb;
+
+  // First and last cell, entry and exit offset in them.  A point on a
+  // boundary starts the cell right of it and ends the cell left of it.
+  const int32_t ce = xe >> 8, cx = (xx - 1) >> 8 > ce ? (xx - 1) >> 8 : ce;
+  const int32_t fe = xe & 255, fx = xx - (cx << 8);
+  if (cx < w0 || ce > w1) return (cx < w0) != e.left ? (uint32_t)with_sign(ybot - ytop, sgn) << 9 : 0u;
+  const int32_t k0 = ce > w0 ? ce : w0, k1 = cx < w1 ? cx : w1;   // the cells inside the tile
+
+  // Crossing y of a column boundary, row-relative.
+  auto rel = [&](int32_t q) -> int32_t {
+    const int32_t y = e.y0 + q;
     return e.steep ? (y & 255) : y - row_y;
   };
-  ColumnWalk walk;
-  int32_t y_in;
-  if (k0 == ce) {
-    y_in = ytop;
-    // the next boundary: right of ce / left of ce
-    const int32_t m = e.dir > 0 ? ce + 1 : ce;
-    walk.start(e, (uint64_t)(int64_t)(e.dir > 0 ? 256 * (int64_t)m - e.x0 : e.x0 - 256 * (int64_t)m));
+  // Dividend of the crossing of the boundary that cell k0 is left through;
+  // each next boundary adds 256 dy.
+  double inv_dx = 0.0, num = 0.0, step = 0.0;
+  int32_t y_in = ytop;
+  if (ce != cx) {
+    inv_dx = recip(e.dx);
+    step = 256.0 * (double)e.dy;
+    num = __builtin_fma((double)(256 * (k0 + 1) - e.x0), (double)e.dy, (double)(e.dx - (e.dx >> 1)));
+    // entered through the tile edge: the crossing one boundary earlier
+    if (k0 != ce) y_in = rel(div_floor(num - step, inv_dx));
   }
-  else {
-    // entered through the tile edge: the left edge x_left moving right, the
-    // right edge x_end moving left
-    const int32_t m = e.dir > 0 ? k0 : k0 + 1;
-    walk.start(e, (uint64_t)(int64_t)(e.dir > 0 ? 256 * (int64_t)m - e.x0 : e.x0 - 256 * (int64_t)m));
-    y_in = rel(walk.q);
-    walk.next();
-  }
-  // Backdrop: cells left of the tile telescope to the y interval they span.
+  // Cells left of the tile telescope to the y interval they span: the first
+  // ones moving right, the last ones moving left.
   uint32_t backdrop = 0;
-  if (lo < x_left) {
-    // moving right they are the first cells (ytop .. y_in of the first tile
-    // cell), moving left the last ones (the crossing at x_left .. ybot)
-    if (e.dir > 0) backdrop = (uint32_t)(sgn * (y_in - ytop)) << 9;
-  }
-  int32_t carry = 0;   // moving right: area the previous tile cell passes into this one
-  for (int32_t k = k0;; k += e.dir) {
+  if (!e.left) backdrop = (uint32_t)with_sign(y_in - ytop, sgn) << 9;
+  // A cell adds cover * 512 - area to itself and area to the cell on its
+  // right, the area measured from its left side; in the direction of travel
+  // that is one value per boundary: what the cell before it passes on plus
+  // what this cell adds on that side.
+  int32_t carry = 0;
+  for (int32_t k = k0; k <= k1; k++) {
     const bool last = k == cx;
-    const int32_t y_out = last ? ybot : rel(walk.q);
-    const int32_t f_in = k == ce ? fe : (e.dir > 0 ? 0 : 256);
-    const int32_t f_out = last ? fx : (e.dir > 0 ? 256 : 0);
-    const int32_t cover = sgn * (y_out - y_in);
-    const int32_t area = cover * (f_in + f_out);
-    const uint32_t own = ((uint32_t)cover << 9) - (uint32_t)area;
-    if (e.dir > 0) {
-      sink(k - x_left, own + (uint32_t)carry);
-      carry = area;
-    }
-    else {
-      // moving left, the cell right of this one was visited just before
-      sink(k - x_left, own);
-      if (k + 1 < x_end) sink(k + 1 - x_left, (uint32_t)area);
-    }
-    if (k == k1) {
-      if (e.dir > 0 && k + 1 < x_end) sink(k + 1 - x_left, (uint32_t)carry);
-      // moving left past the tile: the rest of the row lies left of it
-      if (e.dir < 0 && !last) backdrop = (uint32_t)(sgn * (ybot - y_out)) << 9;
-      break;
-    }
+    const int32_t y_out = last ? ybot : rel(div_floor(num, inv_dx));
+    const int32_t cover = with_sign(y_out - y_in, sgn);
+    const int32_t area = mul_small(cover, (k == ce ? fe : 0) + (last ? fx : 256));
+    const int32_t cell = (e.left ? -k : k) - x_left;
+    if ((uint32_t)cell < (uint32_t)width) sink(cell, (uint32_t)(carry + cover * 512 - area));
+    carry = area;
     y_in = y_out;
-    walk.next();
+    num += step;
   }
+  const int32_t cell = (e.left ? -(k1 + 1) : k1 + 1) - x_left;
+  if ((uint32_t)cell < (uint32_t)width) sink(cell, (uint32_t)carry);
+  if (e.left && cx > w1) backdrop = (uint32_t)with_sign(ybot - y_in, sgn) << 9;
   return backdrop;
 }
 
