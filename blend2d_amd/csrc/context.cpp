@@ -183,6 +183,58 @@ DeviceQueue& device_queue() {
   return *q;
 }
 
+// Read-back of images through pinned memory: the device rows come over as they
+// lie (padding included) in chunks of whole rows, and each chunk is copied into
+// the caller's rows while the next one is on its way.  hipMemcpy2D into
+// pageable memory takes 5-7 us a row instead: a 129 x 229 A8 image 1.57 ms
+// against 0.02, 1920 x 1080 PRGB32 7.7 ms against 0.4-0.9.  Shared by all threads,
+// two fixed chunks, kept until the process ends.
+struct Downloader {
+  static constexpr size_t kChunk = (size_t)1 << 20;   // an image row is at most 256 KB
+  std::mutex mu;
+  uint8_t* pinned = nullptr;
+  hipEvent_t done[2] = {nullptr, nullptr};
+  bool init() {
+    if (!pinned && hipHostMalloc((void**)&pinned, 2 * kChunk, hipHostMallocDefault) != hipSuccess) { pinned = nullptr; return false; }
+    for (hipEvent_t& e : done)
+      if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) { e = nullptr; return false; }
+    return true;
+  }
+  // Rows of `row` bytes from device memory (rows `src_stride` apart) to host
+  // memory (rows `dst_stride` apart), behind the work of the null stream as
+  // hipMemcpy is.
+  hipError_t copy(void* dst, size_t dst_stride, const void* src, size_t src_stride, size_t row, size_t rows) {
+    std::lock_guard<std::mutex> lock(mu);
+    if (!init()) return hipMemcpy2D(dst, dst_stride, src, src_stride, row, rows, hipMemcpyDeviceToHost);
+    const size_t per = std::max<size_t>(1, kChunk / src_stride), n = (rows + per - 1) / per;
+    auto issue = [&](size_t c) -> hipError_t {
+      const size_t r0 = c * per, k = std::min(per, rows - r0);
+      // the last row ends with its pixels
+      const hipError_t e = hipMemcpyAsync(pinned + (c & 1) * kChunk, (const uint8_t*)src + r0 * src_stride,
+                                          (k - 1) * src_stride + row, hipMemcpyDeviceToHost, nullptr);
+      return e != hipSuccess ? e : hipEventRecord(done[c & 1], nullptr);
+    };
+    hipError_t err = issue(0);
+    for (size_t c = 0; c < n && err == hipSuccess; c++) {
+      if (c + 1 < n && (err = issue(c + 1)) != hipSuccess) break;
+      if ((err = hipEventSynchronize(done[c & 1])) != hipSuccess) break;
+      const size_t r0 = c * per, k = std::min(per, rows - r0);
+      const uint8_t* from = pinned + (c & 1) * kChunk;
+      uint8_t* to = (uint8_t*)dst + r0 * dst_stride;
+      if (dst_stride == row && src_stride == row) memcpy(to, from, k * row);
+      else
+        for (size_t r = 0; r < k; r++) memcpy(to + r * dst_stride, from + r * src_stride, row);
+    }
+    if (err != hipSuccess) (void)hipStreamSynchronize(nullptr);   // copies already issued write the chunks
+    return err;
+  }
+};
+
+Downloader& downloader() {
+  static Downloader* d = new Downloader();
+  return *d;
+}
+
 // Slices of one caller-owned device region, 256-byte aligned, handed out in
 // order; used instead of the runner's grow-only buffers by the execution
 // that allocates nothing.
@@ -2103,7 +2155,8 @@ BLAmdResult bl_amd_image_upload(BLAmdImage* img, const void* pixels, intptr_t st
 BLAmdResult bl_amd_image_download(const BLAmdImage* img, void* pixels, intptr_t stride) {
   if (!img || !pixels) return kErrInvalid;
   const size_t row = (size_t)img->w * (img->format == BL_AMD_FORMAT_A8 ? 1 : 4);
-  if (hipMemcpy2D(pixels, (size_t)stride, img->dptr, (size_t)img->stride, row, (size_t)img->h, hipMemcpyDeviceToHost) != hipSuccess)
+  if (stride < (intptr_t)row || stride > INT32_MAX) return kErrDevice;   // as hipMemcpy2D refuses them
+  if (downloader().copy(pixels, (size_t)stride, img->dptr, (size_t)img->stride, row, (size_t)img->h) != hipSuccess)
     return kErrDevice;
   return BL_AMD_SUCCESS;
 }
