@@ -89,15 +89,16 @@ struct FrameHost {
   std::vector<Stop> lut_stops;
   uint64_t lut_entries = 0;
   bool dither = false;   // some style samples a dithered gradient
-  // upper bound of the edge work items of `src`: 1 per line, 3 per quad, 8 per cubic
+  // upper bound of the monotonic pieces of `src`: 1 per line, 3 per quad, 8 per cubic
   uint64_t items = 0;
+  uint32_t boxes = 0;    // box fills among the commands
   std::vector<DevImage> images;
   // Host only: per command, the rendering call (counted from begin()) that
   // recorded it, so errors found on the device name their call.
   std::vector<uint64_t> cmd_call;
   void clear() {
     canvases.clear(); cmds.clear(); xforms.clear(); src.clear(); vtx.clear();
-    styles.clear(); lut_jobs.clear(); lut_stops.clear(); lut_entries = 0; dither = false; items = 0; images.clear();
+    styles.clear(); lut_jobs.clear(); lut_stops.clear(); lut_entries = 0; dither = false; items = 0; boxes = 0; images.clear();
     cmd_call.clear();
   }
 };
@@ -167,7 +168,7 @@ struct DeviceQueue {
     if (!stream && hipStreamCreateWithFlags(&stream, hipStreamNonBlocking) != hipSuccess) { stream = nullptr; return false; }
     if (!ev0 && hipEventCreate(&ev0) != hipSuccess) { ev0 = nullptr; return false; }
     if (!ev1 && hipEventCreate(&ev1) != hipSuccess) { ev1 = nullptr; return false; }
-    if (!host_readback && hipHostMalloc((void**)&host_readback, 256, hipHostMallocDefault) != hipSuccess) { host_readback = nullptr; return false; }
+    if (!host_readback && hipHostMalloc((void**)&host_readback, 1024, hipHostMallocDefault) != hipSuccess) { host_readback = nullptr; return false; }
     int dev = 0, n_cu = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n_cu <= 0)
@@ -257,8 +258,8 @@ struct Runner {
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   DevBuf in;
   DevBuf lut_buf;   // gradient tables of the resident frame
-  DevBuf src_count, src_off, bounds, segs, seg_cmd, mat_cnt, mat_off, mat_pres, list_off, list, binned, scan_tmp, counters, cmd_tiles;
-  DevBuf tile_hdr, group_hdr, tile_px, list_style, band_buf, item_cnt, item_off, items;
+  DevBuf bounds, cmd_bin, segs, seg_cmd, clip, mat_cnt, mat_off, mat_pres, list_off, list, binned, scan_tmp, counters;
+  DevBuf tile_hdr, group_hdr, list_style, band_buf;
   DevBuf cm_params, cm_acc, cm_feat, cm_pred, cm_act;
   DevBuf cmd_err;
   // Tile work queue: queue, bucket counters + head, keys, features,
@@ -279,7 +280,7 @@ struct Runner {
   struct ExactPlan {
     bool valid = false;
     uint64_t gen = 0;
-    uint32_t n_segs = 0, some_failed = 0, n_binned = 0, n_list = 0;
+    uint32_t n_segs = 0, seg_stride = 0, clip_stride = 0, some_failed = 0, n_binned = 0, n_list = 0;
     uint32_t n_atiles = 0, n_fgroups = 0, n_sgroups = 0, n_ggroups = 0;
   } plan;
   // The captured replay and what it was captured with (buffers, frame,
@@ -302,7 +303,7 @@ struct Runner {
   bool resident = false;
   FrameDev f{};
   uint64_t n_src = 0;
-  uint32_t item_cap = 0;   // upper bound of edge work items: lines + 3 per quad + 8 per cubic
+  uint32_t item_cap = 0;   // upper bound of monotonic pieces: lines + 3 per quad + 8 per cubic
   uint32_t bands_max = 0;
   uint32_t max_bands() const { return bands_max; }
   uint64_t frame_bytes = 0, lut_bytes = 0, image_bytes = 0;
@@ -353,6 +354,12 @@ struct Runner {
   uint32_t execute_exact(Stats& stats, ScratchArena* arena = nullptr, const ExactPlan* known = nullptr);
   // The schedule the analytic tiles of this frame run with.
   void resolve_schedule(uint32_t n_a, bool allow_queue, uint32_t& sched, uint32_t& wgs) const;
+  // The buffers whose sizes the resident frame alone fixes, each from
+  // take(own buffer, bytes); false when one could not be had.
+  template<typename Take> bool frame_scratch(FrameScratch& s, Take&& take);
+  // The clip list: every piece of a small frame, a quarter of the sources of
+  // a large one to begin with, or as many as it was grown to.
+  bool reserve_clip(FrameScratch& s);
   // 0 done, 1 pool overflow (redo exactly), otherwise an error
   uint32_t execute_pool(Stats& stats, uint32_t mode);
   bool model_views(cm::FrameModel& m);
@@ -366,6 +373,9 @@ struct Runner {
     const double up = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     if (r) return r;
     r = execute(stats);
+    // every execution ends with a synchronization, which also frees the
+    // staging memory for the next upload; one that failed may not have
+    if (r && resident) (void)hipStreamSynchronize(stream);
     stats.merge_ms = merge_ms;
     stats.upload_ms = up;
     stats.pack_ms = pack_ms;
@@ -523,6 +533,7 @@ uint32_t Runner::upload(const std::vector<FrameHost*>& parts) {
   PartBase tot{0, 0, 0, 0, 0, 0, 0, 0, 0};
   uint64_t n_src_total = 0;
   uint64_t n_items_max = 0;
+  uint32_t n_boxes = 0;
   bool dither = false;
   for (size_t k = 0; k < parts.size(); k++) {
     const FrameHost& fh = *parts[k];
@@ -542,6 +553,7 @@ uint32_t Runner::upload(const std::vector<FrameHost*>& parts) {
     tot.images += fh.images.size();
     n_src_total += fh.src.size();
     n_items_max += fh.items;
+    n_boxes += fh.boxes;
   }
 
   uint64_t n_mat = 0;
@@ -652,9 +664,6 @@ uint32_t Runner::upload(const std::vector<FrameHost*>& parts) {
   if (tot.jobs)
     launch_gradient_luts((const lut::Job*)(in.as<uint8_t>() + off[kSecJobs]), (const Stop*)(in.as<uint8_t>() + off[kSecStops]),
                          (uint32_t)tot.jobs, lut_buf.as<uint32_t>(), stream);
-  // the staging memory is reused by the next upload
-  HIP_OK(hipStreamSynchronize(stream));
-
   const uint8_t* base = in.as<uint8_t>();
   f = FrameDev{};
   f.canvases = (const DevCanvas*)(base + off[kSecCanvases]); f.n_canvases = (uint32_t)canvases.size();
@@ -669,6 +678,7 @@ uint32_t Runner::upload(const std::vector<FrameHost*>& parts) {
   f.n_tiles = n_tiles;
   f.n_groups = n_groups;
   f.n_bands = band_base;
+  f.n_boxes = n_boxes;
   f.n_mat = n_mat;
   f.tol_sq = kToleranceSq;
   n_src = n_src_total;
@@ -748,77 +758,75 @@ uint32_t Runner::execute(Stats& stats) {
   return execute_exact(stats);
 }
 
+template<typename Take>
+bool Runner::frame_scratch(FrameScratch& s, Take&& take) {
+  memset(&s, 0, sizeof(s));
+  const size_t n_mat = f.n_mat, nb = (size_t)f.n_bands + 1;
+  s.counters = (uint32_t*)take(counters, kCounterWords * 4);
+  s.bounds = (CmdBounds*)take(bounds, (size_t)f.n_cmds * sizeof(CmdBounds));
+  s.cmd_bin = (CmdBin*)take(cmd_bin, (size_t)f.n_cmds * sizeof(CmdBin));
+  s.mat_cnt = (uint32_t*)take(mat_cnt, (n_mat + 1) * 4);
+  s.mat_off = (uint32_t*)take(mat_off, (n_mat + 1) * 4);
+  s.mat_pres = (uint32_t*)take(mat_pres, (n_mat + 1) * 4);
+  s.list_off = (uint32_t*)take(list_off, (n_mat + 1) * 4);
+  s.scan_tmp = (uint32_t*)take(scan_tmp, scan_tmp_words() * 4);
+  s.tile_hdr = (uint4*)take(tile_hdr, (size_t)f.n_tiles * 16);
+  s.group_hdr = (uint4*)take(group_hdr, (size_t)f.n_groups * 32);
+  s.band_nonsolid = (uint32_t*)take(band_buf, nb * 24);
+  s.cmd_err = (uint32_t*)take(cmd_err, (size_t)f.n_cmds * 4);
+  if (!s.counters || !s.bounds || !s.cmd_bin || !s.mat_cnt || !s.mat_off || !s.mat_pres || !s.list_off || !s.scan_tmp || !s.tile_hdr ||
+      !s.group_hdr || !s.band_nonsolid || !s.cmd_err)
+    return false;
+  s.band_slow = s.band_nonsolid + nb;
+  s.tile_off = s.band_slow + nb;
+  s.fgroup_off = s.tile_off + nb;
+  s.sgroup_off = s.fgroup_off + nb;
+  s.ggroup_off = s.sgroup_off + nb;
+  s.err_any = s.counters + kCounterErr;
+  s.seg_cursor = s.counters + kCounterCursors;
+  s.seg_regions = 1;
+  return true;
+}
+
+bool Runner::reserve_clip(FrameScratch& s) {
+  const uint64_t want = s.seg_regions == 1 ? item_cap : n_src < 65536 ? 2ull * item_cap : (n_src / 4 + 1024);
+  if (!clip.reserve(std::max<uint64_t>(want, 1) * sizeof(ClipItem))) return false;
+  s.clip = clip.as<ClipItem>();
+  s.clip_stride = (uint32_t)(std::min<size_t>(clip.cap / sizeof(ClipItem), 0x7FFFF000u) / s.seg_regions);
+  return true;
+}
+
 // Pool mode: segment and bin buffers are sized ahead of time (from the cost
-// model's predictions or from the last exact frame) and the edge builder
-// runs once, without the counting pass and without host round trips in
-// between; any overflow is detected at the end of the frame.
+// model's predictions or from the last exact frame), and any overflow is
+// detected before the frame is composited.
 uint32_t Runner::execute_pool(Stats& stats, uint32_t mode) {
   auto t0 = std::chrono::steady_clock::now();
   const uint64_t n_mat = f.n_mat;
-  size_t scan_words = scan_tmp_words(std::max<size_t>({(size_t)n_src, (size_t)n_mat, (size_t)f.n_bands}) + 1);
-  if (!item_cnt.reserve((n_src + 1) * 4) || !item_off.reserve((n_src + 1) * 4) ||
-      !items.reserve(std::max<size_t>(item_cap, 1) * sizeof(EdgeItem)) ||
-      !bounds.reserve((size_t)f.n_cmds * sizeof(CmdBounds)) || !mat_cnt.reserve((n_mat + 1) * 4) ||
-      !mat_off.reserve((n_mat + 1) * 4) || !mat_pres.reserve((n_mat + 1) * 4) || !list_off.reserve((n_mat + 1) * 4) ||
-      !list.reserve((n_mat + 1) * 16) || !list_style.reserve((n_mat + 1) * 8) || !scan_tmp.reserve(scan_words * 4) ||
-      !counters.reserve(64) || !cmd_tiles.reserve((size_t)f.n_cmds * 4) ||
-      !tile_hdr.reserve((size_t)f.n_tiles * 16) || !group_hdr.reserve((size_t)f.n_groups * 32) ||
-      !band_buf.reserve(((size_t)f.n_bands + 1) * 40) || !tile_px.reserve((size_t)f.n_tiles * 8) ||
-      !cmd_err.reserve((size_t)f.n_cmds * 4))
-    return kErrOOM;
-
   FrameScratch s;
-  memset(&s, 0, sizeof(s));
-  s.tile_hdr = tile_hdr.as<uint4>();
-  s.group_hdr = group_hdr.as<uint4>();
-  s.band_nonsolid = band_buf.as<uint32_t>();
-  s.band_tiles = s.band_nonsolid + (f.n_bands + 1);
-  s.band_sgroups = s.band_tiles + (f.n_bands + 1);
-  s.band_ggroups = s.band_sgroups + (f.n_bands + 1);
-  s.tile_off = s.band_ggroups + (f.n_bands + 1);
-  s.sgroup_off = s.tile_off + (f.n_bands + 1);
-  s.ggroup_off = s.sgroup_off + (f.n_bands + 1);
-  s.band_slow = s.ggroup_off + (f.n_bands + 1);
-  s.band_fgroups = s.band_slow + (f.n_bands + 1);
-  s.fgroup_off = s.band_fgroups + (f.n_bands + 1);
-  s.tile_px = tile_px.as<unsigned long long>();
-  s.item_cnt = item_cnt.as<uint32_t>();
-  s.item_off = item_off.as<uint32_t>();
-  s.items = items.as<EdgeItem>();
-  s.cmd_err = cmd_err.as<uint32_t>();
-  s.err_any = counters.as<uint32_t>() + 4;
-  s.bounds = bounds.as<CmdBounds>();
-  s.mat_cnt = mat_cnt.as<uint32_t>();
-  s.mat_off = mat_off.as<uint32_t>();
-  s.mat_pres = mat_pres.as<uint32_t>();
-  s.list_off = list_off.as<uint32_t>();
+  if (!frame_scratch(s, [](DevBuf& own, size_t bytes) -> void* { return own.reserve(bytes) ? own.ptr : nullptr; }) ||
+      !list.reserve((n_mat + 1) * 16) || !list_style.reserve((n_mat + 1) * 8))
+    return kErrOOM;
   s.list_ent = list.as<uint4>();
   s.list_cols = list_style.as<uint32_t>();
   s.list_style = s.list_cols + (n_mat + 1);
-  s.scan_tmp = scan_tmp.as<uint32_t>();
-  s.pixels = counters.as<unsigned long long>();
-  s.seg_cursor = counters.as<uint32_t>() + 2;
-  s.flags = counters.as<uint32_t>() + 3;
-  s.cmd_tiles = cmd_tiles.as<uint32_t>();
+  s.flags = s.counters + kCounterFlags;
+  s.seg_regions = edge_plan(f.n_src).regions;
+  if (!reserve_clip(s)) return kErrOOM;
 
-  launch_fill_u32(counters.as<uint32_t>(), 0u, 5, stream);
-  launch_fill_u32(s.cmd_err, 0u, f.n_cmds, stream);
-  launch_init_bounds(s.bounds, f.n_cmds, stream);
+  launch_frame_init(f, s, true, stream);
 
-  launch_edge_items(f, s, stream);
-
-  // Pool sizes: the emitter writes segments densely (exact slots per item).
+  // Pool sizes.
   uint64_t want_segs, want_bins;
   if (mode == kSizeLearned) {
     cm::FrameModel m;
     if (!model_views(m)) return kErrOOM;
     cm::launch_features(f, m, stream);
     cm::launch_infer_frame(f, m, stream);
-    HIP_OK(hipMemcpyAsync(host_readback + 4, m.totals, 16, hipMemcpyDeviceToHost, stream));
+    HIP_OK(hipMemcpyAsync(host_readback + 64, m.totals, 16, hipMemcpyDeviceToHost, stream));
     HIP_OK(hipStreamSynchronize(stream));
     stats.syncs++;
     uint64_t tot[2];
-    memcpy(tot, host_readback + 4, 16);
+    memcpy(tot, host_readback + 64, 16);
     stats.pred_segs = tot[0];
     stats.pred_bins = tot[1];
     want_segs = tot[0] + tot[0] / 4 + 1024;
@@ -828,87 +836,66 @@ uint32_t Runner::execute_pool(Stats& stats, uint32_t mode) {
     want_segs = hist_segs + hist_segs / 4 + 1024;
     want_bins = hist_bins + hist_bins / 4 + 1024;
   }
-  // (the cursor may run past the capacity by up to the slots of the
-  // allocations that fail, so the capacity stays below 2^31)
+  // (a cursor may run past its region's end by what did not fit, so the
+  // capacity stays below 2^31)
   if (want_segs > 0x7FFFF000ull || want_bins > 0xFFFFF000ull) return 1;
-  if (!segs.reserve(want_segs * sizeof(DevSeg)) || !seg_cmd.reserve(want_segs * 4) || !binned.reserve(want_bins * sizeof(DevSeg)))
+  if (!segs.reserve(want_segs * sizeof(DevSeg)) || !seg_cmd.reserve(want_segs * 8) || !binned.reserve(want_bins * sizeof(DevSeg)))
     return kErrOOM;
-  const uint32_t cap_segs = (uint32_t)std::min<size_t>(std::min(segs.cap / sizeof(DevSeg), seg_cmd.cap / 4), 0x7FFFF000ull);
+  const uint32_t cap_segs = (uint32_t)std::min<size_t>(std::min(segs.cap / sizeof(DevSeg), seg_cmd.cap / 8), 0x7FFFF000ull);
   const uint32_t cap_bins = (uint32_t)std::min<size_t>(binned.cap / sizeof(DevSeg), 0xFFFFF000ull);
   s.segs = segs.as<DevSeg>();
   s.seg_cmd = seg_cmd.as<uint32_t>();
+  s.seg_rank = s.seg_cmd + cap_segs;
+  s.seg_stride = cap_segs / s.seg_regions;
   s.binned = binned.as<DevSeg>();
   s.binned_cap = cap_bins;
 
-  launch_edges_pool(f, s, cap_segs, item_cap, stream);
-#ifdef B2AMD_EMU_TRACE
-  fprintf(stderr, "pool: cap_segs %u cursor %u flags %u want %llu\n", cap_segs, counters.as<uint32_t>()[2], counters.as<uint32_t>()[3], (unsigned long long)want_segs);
-#endif
-  launch_cmd_tiles(f, s, stream);
-  launch_fill_u32(s.mat_cnt, 0u, n_mat + 1, stream);
-  launch_bin_count(f, s, cap_segs, stream);
-  launch_presence(f, s, stream);
-  scan_exclusive(s.mat_cnt, s.mat_off, n_mat, s.scan_tmp, stream);
-  scan_exclusive(s.mat_pres, s.list_off, n_mat, s.scan_tmp, stream);
-  launch_band_class(f, s, stream);
-  launch_list_build(f, s, stream);
-  // the presence flags are used up: their memory holds the scatter cursors
-  launch_copy_u32(s.mat_pres, s.mat_off, n_mat + 1, stream);
-  launch_bin_scatter(f, s, cap_segs, s.mat_pres, stream);
+  launch_edges(f, s, stream);
+  launch_bin_count(f, s, want_segs, stream);
+  launch_scans(f, s, stream);
+  launch_setup(f, s, stream);
+  launch_bin_scatter(f, s, want_segs, stream);
 
   // One read-back before the render stage: a pool overflow ends the frame
   // here (nothing composited; the caller redoes it exactly), otherwise the
   // tile and tile-group counts size the render grids exactly (upper-bound
   // grids of a frame with a million tiles spend milliseconds launching
   // workgroups that exit at once).
-  uint32_t n_atiles = 0, n_fgroups = 0, n_sgroups = 0, n_ggroups = 0;
-  HIP_OK(hipMemcpyAsync(host_readback + 3, s.flags, 4, hipMemcpyDeviceToHost, stream));
-  if (f.n_tiles) {
-    HIP_OK(hipMemcpyAsync(host_readback + 12, s.tile_off + f.n_bands, 4, hipMemcpyDeviceToHost, stream));
-    HIP_OK(hipMemcpyAsync(host_readback + 13, s.sgroup_off + f.n_bands, 4, hipMemcpyDeviceToHost, stream));
-    HIP_OK(hipMemcpyAsync(host_readback + 14, s.ggroup_off + f.n_bands, 4, hipMemcpyDeviceToHost, stream));
-    HIP_OK(hipMemcpyAsync(host_readback + 15, s.fgroup_off + f.n_bands, 4, hipMemcpyDeviceToHost, stream));
-  }
+  launch_report(s, host_readback, stream);
   HIP_OK(hipStreamSynchronize(stream));
   stats.syncs++;
-  if (host_readback[3]) {
+  if (host_readback[kCounterFlags]) {
     stats.total_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     stats.sizing = mode;
     return 1;
   }
-  if (f.n_tiles) {
-    n_atiles = host_readback[12];
-    n_sgroups = host_readback[13];
-    n_ggroups = host_readback[14];
-    n_fgroups = host_readback[15];
-    if (n_atiles > f.n_tiles || (uint64_t)n_fgroups + n_sgroups + n_ggroups > f.n_groups) return kErrDevice;
-  }
+  const uint32_t n_atiles = host_readback[kCounterTiles], n_fgroups = host_readback[kCounterTiles + 1];
+  const uint32_t n_sgroups = host_readback[kCounterTiles + 2], n_ggroups = host_readback[kCounterTiles + 3];
+  if (n_atiles > f.n_tiles || (uint64_t)n_fgroups + n_sgroups + n_ggroups > f.n_groups) return kErrDevice;
 
-  launch_render_setup(f, s, stream);
   HIP_OK(hipEventRecord(ev0, stream));
   if (uint32_t r = render_stage(s, n_atiles, n_fgroups, n_sgroups, n_ggroups, true, stats)) return r;
   stats.render_kernels = (n_atiles ? 1u : 0u) | (n_sgroups ? 2u : 0u) | (n_ggroups ? 4u : 0u) | (n_fgroups ? 8u : 0u);
   HIP_OK(hipEventRecord(ev1, stream));
-  launch_render_stats(f, s, stream);
-  HIP_OK(hipMemcpyAsync(host_readback, counters.ptr, 20, hipMemcpyDeviceToHost, stream));
-  HIP_OK(hipMemcpyAsync(host_readback + 8, s.mat_off + n_mat, 4, hipMemcpyDeviceToHost, stream));
+  launch_report(s, host_readback, stream);
   HIP_OK(hipStreamSynchronize(stream));
   stats.syncs++;
   if (hipError_t e_ = hipGetLastError(); e_ != hipSuccess) { report_hip("kernel launch", e_, __LINE__); return kErrDevice; }
   auto t1 = std::chrono::steady_clock::now();
   stats.total_ms = std::chrono::duration<double, std::milli>(t1 - t0).count();
   stats.sizing = mode;
-  if (host_readback[3]) return 1;
-  if (uint32_t r = read_failures(s, host_readback[4])) return r;
+  if (host_readback[kCounterFlags]) return 1;
+  uint64_t n_segs = 0, pixels;
+  for (uint32_t r = 0; r < s.seg_regions; r++) n_segs += host_readback[kReportCursors + r];
+  memcpy(&pixels, host_readback + kReportPixels, 8);
+  stats.binned = host_readback[kCounterBinned];
+  if (uint32_t r = read_failures(s, host_readback[kCounterErr])) return r;
 
   float ms = 0.f;
   (void)hipEventElapsedTime(&ms, ev0, ev1);
-  uint64_t pixels;
-  memcpy(&pixels, host_readback, 8);
   stats.cmds = f.n_cmds;
   stats.src = n_src;
-  stats.segs = std::min(host_readback[2], cap_segs);   // slots taken, unused chunk tails included
-  stats.binned = host_readback[8];
+  stats.segs = n_segs;
   stats.tiles = f.n_tiles;
   stats.pixels = pixels;
   stats.frame_bytes = frame_bytes;
@@ -985,9 +972,10 @@ uint32_t Runner::render_stage(FrameScratch& s, uint32_t n_a, uint32_t n_f, uint3
   return BL_AMD_SUCCESS;
 }
 
-// Exact sizing: counting pass of the edge builder, scan, read-back, emit;
-// bin count, scans, read-back, scatter.  Two host round trips read back the
-// sizes the next stage allocates (segment count, binned count).
+// Exact sizing: the edge builder writes into the segment buffer the runner has
+// and counts what it needs; after the read-back the buffer is grown and the
+// pass repeated if it did not fit (a first frame of curves).  The second
+// read-back sizes the binned segments and the command lists.
 uint32_t Runner::execute_exact(Stats& stats, ScratchArena* arena, const ExactPlan* known) {
   stats = Stats{};
   auto t0 = std::chrono::steady_clock::now();
@@ -1000,43 +988,24 @@ uint32_t Runner::execute_exact(Stats& stats, ScratchArena* arena, const ExactPla
     if (arena) return arena->take(bytes);
     return own.reserve(bytes) ? own.ptr : nullptr;
   };
-
-  size_t scan_words = scan_tmp_words(std::max<size_t>({(size_t)n_src, (size_t)item_cap, (size_t)n_mat, (size_t)f.n_bands}) + 1);
   FrameScratch s;
-  memset(&s, 0, sizeof(s));
-  s.item_cnt = (uint32_t*)take(item_cnt, (n_src + 1) * 4);
-  s.item_off = (uint32_t*)take(item_off, (n_src + 1) * 4);
-  s.items = (EdgeItem*)take(items, std::max<size_t>(item_cap, 1) * sizeof(EdgeItem));
-  s.src_count = (uint32_t*)take(src_count, ((size_t)item_cap + 1) * 4);
-  s.src_off = (uint32_t*)take(src_off, ((size_t)item_cap + 1) * 4);
-  s.bounds = (CmdBounds*)take(bounds, (size_t)f.n_cmds * sizeof(CmdBounds));
-  s.mat_cnt = (uint32_t*)take(mat_cnt, (n_mat + 1) * 4);
-  s.mat_off = (uint32_t*)take(mat_off, (n_mat + 1) * 4);
-  s.mat_pres = (uint32_t*)take(mat_pres, (n_mat + 1) * 4);
-  s.list_off = (uint32_t*)take(list_off, (n_mat + 1) * 4);
-  s.scan_tmp = (uint32_t*)take(scan_tmp, scan_words * 4);
-  uint32_t* counters_p = (uint32_t*)take(counters, 64);
-  s.cmd_tiles = (uint32_t*)take(cmd_tiles, (size_t)f.n_cmds * 4);
-  s.tile_hdr = (uint4*)take(tile_hdr, (size_t)f.n_tiles * 16);
-  s.group_hdr = (uint4*)take(group_hdr, (size_t)f.n_groups * 32);
-  s.band_nonsolid = (uint32_t*)take(band_buf, ((size_t)f.n_bands + 1) * 40);
-  s.tile_px = (unsigned long long*)take(tile_px, (size_t)f.n_tiles * 8);
-  s.cmd_err = (uint32_t*)take(cmd_err, (size_t)f.n_cmds * 4);
-  if (!s.item_cnt || !s.item_off || !s.items || !s.src_count || !s.src_off || !s.bounds || !s.mat_cnt || !s.mat_off ||
-      !s.mat_pres || !s.list_off || !s.scan_tmp || !counters_p || !s.cmd_tiles || !s.tile_hdr ||
-      !s.group_hdr || !s.band_nonsolid || !s.tile_px || !s.cmd_err)
-    return kErrFit;
-  s.band_tiles = s.band_nonsolid + (f.n_bands + 1);
-  s.band_sgroups = s.band_tiles + (f.n_bands + 1);
-  s.band_ggroups = s.band_sgroups + (f.n_bands + 1);
-  s.tile_off = s.band_ggroups + (f.n_bands + 1);
-  s.sgroup_off = s.tile_off + (f.n_bands + 1);
-  s.ggroup_off = s.sgroup_off + (f.n_bands + 1);
-  s.band_slow = s.ggroup_off + (f.n_bands + 1);
-  s.band_fgroups = s.band_slow + (f.n_bands + 1);
-  s.fgroup_off = s.band_fgroups + (f.n_bands + 1);
-  s.pixels = (unsigned long long*)counters_p;
-  s.err_any = counters_p + 4;
+  if (!frame_scratch(s, take)) return kErrFit;
+  // the arena is small: one region wastes none of it
+  if (!arena) s.seg_regions = edge_plan(f.n_src).regions;
+  auto take_clip = [&](uint64_t stride) -> bool {
+    s.clip = (ClipItem*)take(clip, (size_t)std::max<uint64_t>(stride * s.seg_regions, 1) * sizeof(ClipItem));
+    s.clip_stride = (uint32_t)stride;
+    return s.clip != nullptr;
+  };
+  // The segment buffer with regions of `stride` slots.
+  auto take_segs = [&](uint64_t stride) -> bool {
+    const size_t slots = (size_t)std::max<uint64_t>(stride * s.seg_regions, 1);
+    s.segs = (DevSeg*)take(segs, slots * sizeof(DevSeg));
+    s.seg_cmd = (uint32_t*)take(seg_cmd, slots * 8);   // commands, then numbers
+    s.seg_rank = s.seg_cmd + slots;
+    s.seg_stride = (uint32_t)stride;
+    return s.segs && s.seg_cmd;
+  };
 
   // Graph replay: every buffer is taken now (the counts are known), the
   // render stage's queue buffers and the tile model are made ready, and the
@@ -1058,16 +1027,14 @@ uint32_t Runner::execute_exact(Stats& stats, ScratchArena* arena, const ExactPla
     HIP_OK(hipEventRecord(ev0, stream));
     HIP_OK(hipGraphLaunch(graph_exec, stream));
     HIP_OK(hipEventRecord(ev1, stream));
-    HIP_OK(hipMemcpyAsync(host_readback + 2, s.pixels, 8, hipMemcpyDeviceToHost, stream));
-    HIP_OK(hipMemcpyAsync(host_readback + 4, s.err_any, 4, hipMemcpyDeviceToHost, stream));
     HIP_OK(hipStreamSynchronize(stream));
     stats.syncs++;
     if (hipError_t e_ = hipGetLastError(); e_ != hipSuccess) { report_hip("graph launch", e_, __LINE__); return kErrDevice; }
-    if (uint32_t r = read_failures(s, host_readback[4])) return r;
+    uint64_t pixels;
+    memcpy(&pixels, host_readback + kReportPixels, 8);
+    if (uint32_t r = read_failures(s, host_readback[kCounterErr])) return r;
     float ms = 0.f;
     (void)hipEventElapsedTime(&ms, ev0, ev1);
-    uint64_t pixels;
-    memcpy(&pixels, host_readback + 2, 8);
     stats.cmds = f.n_cmds;
     stats.src = n_src;
     stats.segs = known->n_segs;
@@ -1087,12 +1054,11 @@ uint32_t Runner::execute_exact(Stats& stats, ScratchArena* arena, const ExactPla
     return BL_AMD_SUCCESS;
   };
   if (graph) {
-    s.segs = (DevSeg*)take(segs, (size_t)std::max<uint32_t>(known->n_segs, 1) * sizeof(DevSeg));
-    s.seg_cmd = (uint32_t*)take(seg_cmd, (size_t)std::max<uint32_t>(known->n_segs, 1) * 4);
+    if (!take_segs(known->seg_stride) || !take_clip(known->clip_stride)) return kErrOOM;
     s.binned = (DevSeg*)take(binned, (size_t)std::max<uint32_t>(known->n_binned, 1) * sizeof(DevSeg));
     s.list_ent = (uint4*)take(list, (size_t)std::max<uint32_t>(known->n_list, 1) * 16);
     s.list_cols = (uint32_t*)take(list_style, (size_t)std::max<uint32_t>(known->n_list, 1) * 8);
-    if (!s.segs || !s.seg_cmd || !s.binned || !s.list_ent || !s.list_cols) return kErrOOM;
+    if (!s.binned || !s.list_ent || !s.list_cols) return kErrOOM;
     s.list_style = s.list_cols + std::max<uint32_t>(known->n_list, 1);
     resolve_schedule(known->n_atiles, true, g_sched, g_wgs);
     if (g_sched != BL_AMD_SCHEDULE_GRID) {
@@ -1125,46 +1091,66 @@ uint32_t Runner::execute_exact(Stats& stats, ScratchArena* arena, const ExactPla
     cm::launch_features(f, model, stream);
   }
 
-  // Stage 1: edges (work items; count, scan, emit).
-  launch_fill_u32(counters_p, 0u, 5, stream);
-  launch_fill_u32(s.cmd_err, 0u, f.n_cmds, stream);
-  launch_init_bounds(s.bounds, f.n_cmds, stream);
-  launch_edge_items(f, s, stream);
-  launch_edges(f, s, true, item_cap, stream);
-  launch_cmd_tiles(f, s, stream);
-  // A frame of box fills only has no edges: no counting round trip.
-  uint32_t n_segs = 0;
+  // Stage 1: edges.
+  uint32_t n_segs = 0, max_region = 0, max_clip = 0;
   bool some_failed = false;
   if (graph) {
-    if (n_src) scan_exclusive(s.src_count, s.src_off, item_cap, s.scan_tmp, stream);
+    launch_frame_init(f, s, true, stream);
+    launch_edges(f, s, stream);
     n_segs = known->n_segs;
     some_failed = known->some_failed != 0;
   }
   else {
-    if (n_src) {
-      scan_exclusive(s.src_count, s.src_off, item_cap, s.scan_tmp, stream);
-      HIP_OK(hipMemcpyAsync(host_readback, s.src_off + item_cap, 4, hipMemcpyDeviceToHost, stream));
-      HIP_OK(hipMemcpyAsync(host_readback + 5, s.err_any, 4, hipMemcpyDeviceToHost, stream));
+    // room for three segments per monotonic piece to begin with (an arena
+    // only counts first)
+    uint64_t stride = arena || !n_src ? 0 : std::min<uint64_t>(3ull * item_cap + 1024, 0x7FFFF000ull) / s.seg_regions;
+    if (arena) {
+      if (n_src && !take_clip(item_cap)) return kErrFit;
+    }
+    else {
+      if (!take_segs(stride) || (n_src && !reserve_clip(s))) return kErrOOM;
+      if (n_src) {   // all that the buffers hold
+        const size_t slots = std::min<size_t>({segs.cap / sizeof(DevSeg), seg_cmd.cap / 8, (size_t)0x7FFFF000u});
+        s.seg_rank = s.seg_cmd + slots;
+        s.seg_stride = (uint32_t)(slots / s.seg_regions);
+      }
+    }
+    launch_frame_init(f, s, true, stream);
+    while (n_src) {   // a frame of box fills only has no edges: no round trip
+      launch_edges(f, s, stream);
+      launch_report(s, host_readback, stream);
       HIP_OK(hipStreamSynchronize(stream));
       stats.syncs++;
-      n_segs = host_readback[0];
+      uint64_t total = 0;
+      max_region = max_clip = 0;
+      for (uint32_t r = 0; r < s.seg_regions; r++) {
+        total += host_readback[kReportCursors + r];
+        max_region = std::max(max_region, host_readback[kReportCursors + r]);
+        max_clip = std::max(max_clip, host_readback[kReportClip + r]);
+      }
+      // segments of failed commands are not binned
+      some_failed = host_readback[kCounterErr] != 0;
+      if (total >= 0x80000000ull) return kErrDevice;
+      n_segs = (uint32_t)total;
+      if (max_clip > s.clip_stride) {
+        // more pieces cross the clip box than the list holds: their segments
+        // are not counted yet
+        if (!take_clip(max_clip)) return kErrFit;
+        launch_frame_init(f, s, true, stream);
+        continue;
+      }
+      if (max_region > s.seg_stride || arena) {
+        if (!take_segs(max_region)) return kErrFit;
+        launch_frame_init(f, s, true, stream);
+        launch_edges(f, s, stream);
+      }
+      break;
     }
-    // segments of failed commands are not binned
-    some_failed = n_src && host_readback[5];
-    if (n_segs >= 0x80000000u) return kErrDevice;
-    s.segs = (DevSeg*)take(segs, (size_t)std::max<uint32_t>(n_segs, 1) * sizeof(DevSeg));
-    s.seg_cmd = (uint32_t*)take(seg_cmd, (size_t)std::max<uint32_t>(n_segs, 1) * 4);
-    if (!s.segs || !s.seg_cmd) return kErrFit;
   }
-  launch_edges(f, s, false, item_cap, stream);
 
   // Stage 2: binning.
-  launch_fill_u32(s.mat_cnt, 0u, n_mat + 1, stream);
   launch_bin_count(f, s, n_segs, stream);
-  launch_presence(f, s, stream);
-  scan_exclusive(s.mat_cnt, s.mat_off, n_mat, s.scan_tmp, stream);
-  scan_exclusive(s.mat_pres, s.list_off, n_mat, s.scan_tmp, stream);
-  launch_band_class(f, s, stream);
+  launch_scans(f, s, stream);
   uint32_t n_binned, n_list, n_atiles, n_sgroups, n_ggroups, n_fgroups;
   if (graph) {
     n_binned = known->n_binned;
@@ -1175,22 +1161,15 @@ uint32_t Runner::execute_exact(Stats& stats, ScratchArena* arena, const ExactPla
     n_fgroups = known->n_fgroups;
   }
   else {
-    HIP_OK(hipMemcpyAsync(host_readback, s.mat_off + n_mat, 4, hipMemcpyDeviceToHost, stream));
-    HIP_OK(hipMemcpyAsync(host_readback + 1, s.list_off + n_mat, 4, hipMemcpyDeviceToHost, stream));
-    if (f.n_tiles) {
-      HIP_OK(hipMemcpyAsync(host_readback + 12, s.tile_off + f.n_bands, 4, hipMemcpyDeviceToHost, stream));
-      HIP_OK(hipMemcpyAsync(host_readback + 13, s.sgroup_off + f.n_bands, 4, hipMemcpyDeviceToHost, stream));
-      HIP_OK(hipMemcpyAsync(host_readback + 14, s.ggroup_off + f.n_bands, 4, hipMemcpyDeviceToHost, stream));
-      HIP_OK(hipMemcpyAsync(host_readback + 15, s.fgroup_off + f.n_bands, 4, hipMemcpyDeviceToHost, stream));
-    }
+    launch_report(s, host_readback, stream);
     HIP_OK(hipStreamSynchronize(stream));
     stats.syncs++;
-    n_binned = host_readback[0];
-    n_list = host_readback[1];
-    n_atiles = f.n_tiles ? host_readback[12] : 0u;
-    n_sgroups = f.n_tiles ? host_readback[13] : 0u;
-    n_ggroups = f.n_tiles ? host_readback[14] : 0u;
-    n_fgroups = f.n_tiles ? host_readback[15] : 0u;
+    n_binned = host_readback[kCounterBinned];
+    n_list = host_readback[kCounterList];
+    n_atiles = host_readback[kCounterTiles];
+    n_fgroups = host_readback[kCounterTiles + 1];
+    n_sgroups = host_readback[kCounterTiles + 2];
+    n_ggroups = host_readback[kCounterTiles + 3];
     if (n_atiles > f.n_tiles || (uint64_t)n_fgroups + n_sgroups + n_ggroups > f.n_groups) return kErrDevice;
     // every edge segment crosses at least one band and at most all of them;
     // the command lists hold at most one entry per (band, command) cell
@@ -1203,18 +1182,15 @@ uint32_t Runner::execute_exact(Stats& stats, ScratchArena* arena, const ExactPla
     if (!s.binned || !s.list_ent || !s.list_cols) return kErrFit;
     s.list_style = s.list_cols + std::max<uint32_t>(n_list, 1);
   }
-  launch_list_build(f, s, stream);
-  // the presence flags are used up: their memory holds the scatter cursors
-  launch_copy_u32(s.mat_pres, s.mat_off, n_mat + 1, stream);
-  launch_bin_scatter(f, s, n_segs, s.mat_pres, stream);
+  launch_setup(f, s, stream);
+  launch_bin_scatter(f, s, n_segs, stream);
 
   // Stage 3: render.
-  launch_render_setup(f, s, stream);
   if (!graph) HIP_OK(hipEventRecord(ev0, stream));
   if (uint32_t r = render_stage(s, n_atiles, n_fgroups, n_sgroups, n_ggroups, !arena, stats)) return r;
   stats.render_kernels = (n_atiles ? 1u : 0u) | (n_sgroups ? 2u : 0u) | (n_ggroups ? 4u : 0u) | (n_fgroups ? 8u : 0u);
   if (!graph) HIP_OK(hipEventRecord(ev1, stream));
-  launch_render_stats(f, s, stream);
+  launch_report(s, host_readback, stream);
   if (graph) {
     hipGraph_t g = nullptr;
     capture.on = false;
@@ -1228,10 +1204,8 @@ uint32_t Runner::execute_exact(Stats& stats, ScratchArena* arena, const ExactPla
     graph_model = g_tile_model_version;
     return run_graph();
   }
-  HIP_OK(hipMemcpyAsync(host_readback + 2, s.pixels, 8, hipMemcpyDeviceToHost, stream));
-  HIP_OK(hipMemcpyAsync(host_readback + 4, s.err_any, 4, hipMemcpyDeviceToHost, stream));
   if (collect && !arena) {
-    cm::launch_actuals(f, s, model, n_segs, stream);
+    cm::launch_actuals(f, s, model, max_region, stream);
     const size_t nc = f.n_cmds;
     std::vector<float> feat(nc * cm::kIn);
     std::vector<uint32_t> act(2 * std::max<size_t>(nc, 1));
@@ -1251,10 +1225,12 @@ uint32_t Runner::execute_exact(Stats& stats, ScratchArena* arena, const ExactPla
   HIP_OK(hipStreamSynchronize(stream));
   stats.syncs++;
   if (hipError_t e_ = hipGetLastError(); e_ != hipSuccess) { report_hip("kernel launch", e_, __LINE__); return kErrDevice; }
+  uint64_t pixels;
+  memcpy(&pixels, host_readback + kReportPixels, 8);
   // (the arena execution is a replay: its failures were reported by the
   // flush that uploaded the frame, and it keeps no host-side list)
   if (!arena)
-    if (uint32_t r = read_failures(s, host_readback[4])) return r;
+    if (uint32_t r = read_failures(s, host_readback[kCounterErr])) return r;
   if (collect_tiles && !arena) {
     tile_x.assign((size_t)n_atiles * 16, 0.0f);
     std::vector<uint32_t> ticks((size_t)n_atiles * 2);
@@ -1275,6 +1251,8 @@ uint32_t Runner::execute_exact(Stats& stats, ScratchArena* arena, const ExactPla
     plan.valid = true;
     plan.gen = gen;
     plan.n_segs = n_segs;
+    plan.seg_stride = max_region;
+    plan.clip_stride = max_clip;
     plan.some_failed = some_failed ? 1u : 0u;
     plan.n_binned = n_binned;
     plan.n_list = n_list;
@@ -1287,8 +1265,6 @@ uint32_t Runner::execute_exact(Stats& stats, ScratchArena* arena, const ExactPla
   (void)hipEventElapsedTime(&ms, ev0, ev1);
   auto t1 = std::chrono::steady_clock::now();
 
-  uint64_t pixels;
-  memcpy(&pixels, host_readback + 2, 8);
   stats.cmds = f.n_cmds;
   stats.src = n_src;
   stats.segs = n_segs;
@@ -1588,12 +1564,13 @@ CmdXform fixed_xform(const BLAmdContext* c) {
   x.m10 = c->user.m10 * 256.0; x.m11 = c->user.m11 * 256.0;
   x.m20 = c->user.m20 * 256.0; x.m21 = c->user.m21 * 256.0;
   x.scale_only = transform_type(c->user) <= kTTScale ? 1u : 0u;
-  x.pad = 0;
+  x.canvas_size = (uint32_t)c->target->w | ((uint32_t)c->target->h << 16);
   return x;
 }
 
 uint32_t push_cmd(BLAmdContext* c, const DevCmd& cmd, const CmdXform* xf) {
   c->frame.cmds.push_back(cmd);
+  if (cmd.kind != kCmdAnalytic) c->frame.boxes++;
   c->frame.cmd_call.push_back(c->call_seq ? c->call_seq - 1 : 0);
   if (xf) c->frame.xforms.push_back(*xf);
   else c->frame.xforms.push_back(CmdXform{});

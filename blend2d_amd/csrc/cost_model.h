@@ -50,7 +50,7 @@ struct FrameModel {
 
 void launch_features(const FrameDev& f, const FrameModel& m, hipStream_t st);
 void launch_infer_frame(const FrameDev& f, const FrameModel& m, hipStream_t st);
-void launch_actuals(const FrameDev& f, const FrameScratch& s, const FrameModel& m, uint32_t n_segs, hipStream_t st);
+void launch_actuals(const FrameDev& f, const FrameScratch& s, const FrameModel& m, uint32_t n_region, hipStream_t st);
 
 // Generic MLP entry points (training / tests).
 void launch_mlp_forward(const float* X, uint32_t n, const float* params, float* Y, hipStream_t st);

@@ -275,19 +275,15 @@ void launch_infer_frame(const FrameDev& f, const FrameModel& m, hipStream_t st) 
   if (f.n_cmds) hipLaunchKernelGGL(k_infer_frame, dim3((f.n_cmds + 255) / 256), dim3(256), 0, st, f, m);
 }
 
-// Exact per-command counts of a frame that ran the counting pass (the
-// training targets).
-__global__ void k_actual_segs(FrameDev f, FrameScratch s, FrameModel m, uint32_t n_segs) {
-  uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n_segs) return;
-  atomicAdd(&m.actual_segs[s.seg_cmd[i]], 1u);
-}
-
-__global__ void k_actual_bins(FrameDev f, FrameScratch s, FrameModel m, uint32_t n_segs) {
-  uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n_segs) return;
-  const DevSeg g = s.segs[i];
-  const uint32_t cmd = s.seg_cmd[i];
+// Exact per-command counts of an executed frame (the training targets): one
+// grid row per region of the segment buffer.
+__global__ void k_actuals(FrameDev f, FrameScratch s, FrameModel m) {
+  const uint32_t r = blockIdx.y, i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= s.seg_stride || i >= s.seg_cursor[r * kCursorStep]) return;
+  const size_t at = (size_t)r * s.seg_stride + i;
+  const DevSeg g = s.segs[at];
+  const uint32_t cmd = s.seg_cmd[at];
+  atomicAdd(&m.actual_segs[cmd], 1u);
   const DevCanvas& cv = f.canvases[f.cmds[cmd].canvas];
   int b0 = (g.y0 >> 8) / kTileH, b1 = ((g.y1 - 1) >> 8) / kTileH;
   b0 = b0 < 0 ? 0 : b0;
@@ -295,9 +291,9 @@ __global__ void k_actual_bins(FrameDev f, FrameScratch s, FrameModel m, uint32_t
   if (b1 >= b0) atomicAdd(&m.actual_bins[cmd], (uint32_t)(b1 - b0 + 1));
 }
 
-void launch_actuals(const FrameDev& f, const FrameScratch& s, const FrameModel& m, uint32_t n_segs, hipStream_t st) {
-  if (n_segs) hipLaunchKernelGGL(k_actual_segs, dim3((n_segs + 255) / 256), dim3(256), 0, st, f, s, m, n_segs);
-  if (n_segs) hipLaunchKernelGGL(k_actual_bins, dim3((n_segs + 255) / 256), dim3(256), 0, st, f, s, m, n_segs);
+// `n_region`: an upper bound of the segments of one region.
+void launch_actuals(const FrameDev& f, const FrameScratch& s, const FrameModel& m, uint32_t n_region, hipStream_t st) {
+  if (n_region) hipLaunchKernelGGL(k_actuals, dim3((n_region + 255) / 256, s.seg_regions), dim3(256), 0, st, f, s, m);
 }
 
 // ---------------------------------------------------------------------------

@@ -89,7 +89,7 @@ struct SrcSeg {
 struct CmdXform {
   double m00, m01, m10, m11, m20, m21;
   uint32_t scale_only;   // transform type <= SCALE: x*m00+m20, y*m11+m21
-  uint32_t pad;
+  uint32_t canvas_size;  // width | height << 16 of the command's canvas (the clip box)
 };
 
 struct DevCmd {

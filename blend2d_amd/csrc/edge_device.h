@@ -251,7 +251,9 @@ struct Builder {
     for (int i = 1; i < m.n - 1; i++) { m.p[i].x = dclamp(m.p[i].x, l.x, f.x); m.p[i].y = dclamp(m.p[i].y, f.y, l.y); }
   }
   __device__ __forceinline__ bool is_flat(const Mono& m) const {
-    if (invalid & kFailTooManySegments) return true;
+    return (invalid & kFailTooManySegments) || flat_enough(m, tol_sq);
+  }
+  __device__ __forceinline__ static bool flat_enough(const Mono& m, double tol_sq) {
     double value, limit;
     if (m.n == 3) {
       P v1 = psub(m.p[1], m.p[0]);
@@ -282,6 +284,20 @@ struct Builder {
       s.p012 = pmid(s.p01, s.p12);
       s.p123 = pmid(s.p12, s.p23);
       s.p0123 = pmid(s.p012, s.p123);
+    }
+  }
+  // Splits `m`: it becomes its left half, `right` receives the other (a quad's
+  // end point in both of the last two places).
+  __device__ __forceinline__ static void halves(Mono& m, P right[4]) {
+    const P p01 = pmid(m.p[0], m.p[1]), p12 = pmid(m.p[1], m.p[2]), p012 = pmid(p01, p12);
+    if (m.n == 3) {
+      right[0] = p012; right[1] = p12; right[2] = m.p[2]; right[3] = m.p[2];
+      m.p[1] = p01; m.p[2] = p012; m.p[3] = p012;
+    }
+    else {
+      const P p23 = pmid(m.p[2], m.p[3]), p123 = pmid(p12, p23), p0123 = pmid(p012, p123);
+      right[0] = p0123; right[1] = p123; right[2] = p23; right[3] = m.p[3];
+      m.p[1] = p01; m.p[2] = p012; m.p[3] = p0123;
     }
   }
   __device__ __forceinline__ static P step_mid(const Mono& m, const Step& s) { return m.n == 3 ? s.p012 : s.p0123; }
@@ -548,8 +564,9 @@ RTL_AddLine:
     return n;
   }
 
-  __device__ int split_quad(const P* cv, P* out) {
-    double ts[3];
+  // Parameters a quad is cut at to become monotonic, then 1; 0 when it needs
+  // no cut.  `ts` holds 3.
+  __device__ static int cuts_quad(const P* cv, double* ts) {
     int n = 0;
     P num{cv[0].x - cv[1].x, cv[0].y - cv[1].y};
     P den{cv[0].x - cv[1].x * 2.0 + cv[2].x, cv[0].y - cv[1].y * 2.0 + cv[2].y};
@@ -558,34 +575,41 @@ RTL_AddLine:
     double t1 = dmax(ex.x, ex.y);
     ts[n] = t0; n += (int)((t0 > 0.0) & (t0 < 1.0));
     ts[n] = t1; n += (int)((t1 > dmax(t0, 0.0)) & (t1 < 1.0));
-    if (n == 0) { out[0] = cv[0]; out[1] = cv[1]; out[2] = cv[2]; return 1; }
-    ts[n++] = 1.0;
+    if (n) ts[n++] = 1.0;
+    return n;
+  }
+  // The piece from t_cut to t; `at` is the previous piece's end point.
+  __device__ __forceinline__ static void piece_quad(const P* cv, double t_cut, double t, bool final, P at, P* out) {
     P v1 = psub(cv[1], cv[0]);
     P v2 = psub(cv[2], cv[1]);
     P qa = psub(v2, v1);
     P qb{v1.x + v1.x, v1.y + v1.y};
     P qc = cv[0];
-    P last = cv[2];
-    out[0] = cv[0];
-    int i = 0, pieces = 0;
+    double dt = (t - t_cut) * 0.5;
+    P cp{(qa.x * (t * 2.0) + qb.x) * dt, (qa.y * (t * 2.0) + qb.y) * dt};
+    P tp{(qa.x * t + qb.x) * t + qc.x, (qa.y * t + qb.y) * t + qc.y};
+    if (final) tp = cv[2];
+    out[0] = at;
+    out[1] = P{tp.x - cp.x, tp.y - cp.y};
+    out[2] = tp;
+  }
+  __device__ int split_quad(const P* cv, P* out) {
+    double ts[3];
+    const int n = cuts_quad(cv, ts);
+    if (n == 0) { out[0] = cv[0]; out[1] = cv[1]; out[2] = cv[2]; return 1; }
+    P at = cv[0];
     double t_cut = 0.0;
-    do {
-      double t = ts[i];
-      double dt = (t - t_cut) * 0.5;
-      P cp{(qa.x * (t * 2.0) + qb.x) * dt, (qa.y * (t * 2.0) + qb.y) * dt};
-      P tp{(qa.x * t + qb.x) * t + qc.x, (qa.y * t + qb.y) * t + qc.y};
-      if (++i == n) tp = last;
-      out[1] = P{tp.x - cp.x, tp.y - cp.y};
-      out[2] = tp;
-      out += 2;
-      pieces++;
-      t_cut = t;
-    } while (i != n);
-    return pieces;
+    for (int i = 0; i < n; i++, out += 2) {
+      piece_quad(cv, t_cut, ts[i], i + 1 == n, at, out);
+      at = out[2];
+      t_cut = ts[i];
+    }
+    return n;
   }
 
-  __device__ int split_cubic(const P* cv, P* out) {
-    double ts[8];
+  // The same for a cubic (`ts` holds 8); a parameter may repeat, and the
+  // piece that would be empty is skipped.
+  __device__ static int cuts_cubic(const P* cv, double* ts) {
     int n = 0;
     P v1 = psub(cv[1], cv[0]);
     P v2 = psub(cv[2], cv[1]);
@@ -593,7 +617,6 @@ RTL_AddLine:
     P ca{v3.x - v2.x - v2.x + v1.x, v3.y - v2.y - v2.y + v1.y};
     P cb{3.0 * (v2.x - v1.x), 3.0 * (v2.y - v1.y)};
     P cc{3.0 * v1.x, 3.0 * v1.y};
-    P cd = cv[0];
     double q0 = cross(cb, ca);
     double q1 = cross(cc, ca);
     double q2 = cross(cc, cb);
@@ -607,68 +630,58 @@ RTL_AddLine:
     P dc{3.0 * v1.x, 3.0 * v1.y};
     n += quad_roots(ts + n, da.x, db.x, dc.x, kAfter0, kBefore1);
     n += quad_roots(ts + n, da.y, db.y, dc.y, kAfter0, kBefore1);
-    if (n == 0) { out[0] = cv[0]; out[1] = cv[1]; out[2] = cv[2]; out[3] = cv[3]; return 1; }
+    if (n == 0) return 0;
     for (int m = 1; m < n; m++)
       for (int l = m; l > 0 && ts[l - 1] > ts[l]; l--) { double t = ts[l - 1]; ts[l - 1] = ts[l]; ts[l] = t; }
     ts[n++] = 1.0;
-    out[0] = cv[0];
-    P last = cv[3];
-    int i = 0, pieces = 0;
+    return n;
+  }
+  __device__ __forceinline__ static void piece_cubic(const P* cv, double t_cut, double tv, bool final, P at, P* out) {
+    P v1 = psub(cv[1], cv[0]);
+    P v2 = psub(cv[2], cv[1]);
+    P v3 = psub(cv[3], cv[2]);
+    P ca{v3.x - v2.x - v2.x + v1.x, v3.y - v2.y - v2.y + v1.y};
+    P cb{3.0 * (v2.x - v1.x), 3.0 * (v2.y - v1.y)};
+    P cc{3.0 * v1.x, 3.0 * v1.y};
+    P cd = cv[0];
+    const double k1Div3 = 1.0 / 3.0;
+    double dt = (tv - t_cut) * k1Div3;
+    P tp{((ca.x * tv + cb.x) * tv + cc.x) * tv + cd.x, ((ca.y * tv + cb.y) * tv + cc.y) * tv + cd.y};
+    if (final) tp = cv[3];
+    P cp1{((ca.x * (t_cut * 3.0) + cb.x * 2.0) * t_cut + cc.x) * dt, ((ca.y * (t_cut * 3.0) + cb.y * 2.0) * t_cut + cc.y) * dt};
+    P cp2{((ca.x * (tv * 3.0) + cb.x * 2.0) * tv + cc.x) * dt, ((ca.y * (tv * 3.0) + cb.y * 2.0) * tv + cc.y) * dt};
+    out[0] = at;
+    out[1] = P{at.x + cp1.x, at.y + cp1.y};
+    out[2] = P{tp.x - cp2.x, tp.y - cp2.y};
+    out[3] = tp;
+  }
+  __device__ int split_cubic(const P* cv, P* out) {
+    double ts[8];
+    const int n = cuts_cubic(cv, ts);
+    if (n == 0) { out[0] = cv[0]; out[1] = cv[1]; out[2] = cv[2]; out[3] = cv[3]; return 1; }
+    P at = cv[0];
     double t_cut = 0.0;
-    do {
-      double tv = ts[i++];
-      if (tv == t_cut) continue;
-      const double k1Div3 = 1.0 / 3.0;
-      double dt = (tv - t_cut) * k1Div3;
-      P tp{((ca.x * tv + cb.x) * tv + cc.x) * tv + cd.x, ((ca.y * tv + cb.y) * tv + cc.y) * tv + cd.y};
-      if (i == n) tp = last;
-      P cp1{((ca.x * (t_cut * 3.0) + cb.x * 2.0) * t_cut + cc.x) * dt, ((ca.y * (t_cut * 3.0) + cb.y * 2.0) * t_cut + cc.y) * dt};
-      P cp2{((ca.x * (tv * 3.0) + cb.x * 2.0) * tv + cc.x) * dt, ((ca.y * (tv * 3.0) + cb.y * 2.0) * tv + cc.y) * dt};
-      out[1] = P{out[0].x + cp1.x, out[0].y + cp1.y};
-      out[2] = P{tp.x - cp2.x, tp.y - cp2.y};
-      out[3] = tp;
+    int pieces = 0;
+    for (int i = 0; i < n; i++) {
+      if (ts[i] == t_cut) continue;
+      piece_cubic(cv, t_cut, ts[i], i + 1 == n, at, out);
+      at = out[3];
       out += 3;
       pieces++;
-      t_cut = tv;
-    } while (i != n);
+      t_cut = ts[i];
+    }
     return pieces;
   }
 
-  // quad_to / cubic_to for one source curve (edgebuilder_p.h:1618-1890),
-  // in two parts.  curve_split: a curve wholly on one side of the clip box
-  // emits its border line here and gives 0; otherwise the monotonic pieces
-  // are written to `spline` (npts - 1 points apart, end point shared) and
-  // their number returned, with `any` set when a control point lies outside
-  // the clip box.  curve_piece flattens one piece; pieces are independent.
-  __device__ int curve_split(const P* cv, int npts, P* spline, uint32_t* any_out) {
-    uint32_t common = 0xFu, any = 0u;
-    for (int i = 0; i < npts; i++) { uint32_t f = fxy(c, cv[i]); common &= f; any |= f; }
-    *any_out = any;
-    if (common) {
-      if (common & CY0) return 0;
-      if (common & CY1) return 0;
-      double y0 = dclamp(cv[0].y, c.y0, c.y1);
-      double y1 = dclamp(cv[npts - 1].y, c.y0, c.y1);
-      if (common & CX0) acc_left(y0, y1); else acc_right(y0, y1);
-      return 0;
-    }
-    return npts == 3 ? split_quad(cv, spline) : split_cubic(cv, spline);
-  }
-
+  // quad_to / cubic_to of one source curve (edgebuilder_p.h:1618-1890): its
+  // monotonic pieces are flattened independently; `any`: a control point lies
+  // outside the clip box.
   __device__ void curve_piece(const P* sp, int npts, uint32_t any, P* stack) {
     Mono m;
     m.n = npts;
     const uint32_t sign = sp[0].y > sp[npts - 1].y;
     if (any) flatten_unsafe(m, sp, sign, stack);
     else flatten_safe(m, sp, sign, stack);
-  }
-
-  __device__ void curve(const P* cv, int npts, P* stack) {
-    P spline[8 * 3 + 1];
-    uint32_t any;
-    const int pieces = curve_split(cv, npts, spline, &any);
-    const P* sp = spline;
-    for (int k = 0; k < pieces; k++, sp += npts - 1) curve_piece(sp, npts, any, stack);
   }
 };
 
