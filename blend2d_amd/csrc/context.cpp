@@ -337,8 +337,8 @@ struct Runner {
   uint32_t strips_for(uint32_t n_a) const;
   // Launches the render stage: the analytic tiles in the schedule in force
   // (`allow_queue` false: GRID), the box tile groups one workgroup each.
-  uint32_t render_stage(FrameScratch& s, uint32_t n_a, uint32_t n_f, uint32_t n_s, uint32_t n_g, bool allow_queue,
-                        Stats& stats);
+  uint32_t render_stage(FrameScratch& s, uint32_t n_a, uint32_t n_f, uint32_t n_s, uint32_t n_g, uint32_t n_binned,
+                        bool allow_queue, Stats& stats);
 
   uint32_t upload(const std::vector<FrameHost*>& parts);
   uint32_t execute(Stats& stats);
@@ -353,7 +353,7 @@ struct Runner {
   // captured before is launched when nothing changed).
   uint32_t execute_exact(Stats& stats, ScratchArena* arena = nullptr, const ExactPlan* known = nullptr);
   // The schedule the analytic tiles of this frame run with.
-  void resolve_schedule(uint32_t n_a, bool allow_queue, uint32_t& sched, uint32_t& wgs) const;
+  void resolve_schedule(uint32_t n_a, uint32_t n_binned, bool allow_queue, uint32_t& sched, uint32_t& wgs) const;
   // The buffers whose sizes the resident frame alone fixes, each from
   // take(own buffer, bytes); false when one could not be had.
   template<typename Take> bool frame_scratch(FrameScratch& s, Take&& take);
@@ -874,7 +874,7 @@ uint32_t Runner::execute_pool(Stats& stats, uint32_t mode) {
   if (n_atiles > f.n_tiles || (uint64_t)n_fgroups + n_sgroups + n_ggroups > f.n_groups) return kErrDevice;
 
   HIP_OK(hipEventRecord(ev0, stream));
-  if (uint32_t r = render_stage(s, n_atiles, n_fgroups, n_sgroups, n_ggroups, true, stats)) return r;
+  if (uint32_t r = render_stage(s, n_atiles, n_fgroups, n_sgroups, n_ggroups, host_readback[kCounterBinned], true, stats)) return r;
   stats.render_kernels = (n_atiles ? 1u : 0u) | (n_sgroups ? 2u : 0u) | (n_ggroups ? 4u : 0u) | (n_fgroups ? 8u : 0u);
   HIP_OK(hipEventRecord(ev1, stream));
   launch_report(s, host_readback, stream);
@@ -905,7 +905,7 @@ uint32_t Runner::execute_pool(Stats& stats, uint32_t mode) {
   return BL_AMD_SUCCESS;
 }
 
-void Runner::resolve_schedule(uint32_t n_a, bool allow_queue, uint32_t& sched, uint32_t& wgs) const {
+void Runner::resolve_schedule(uint32_t n_a, uint32_t n_binned, bool allow_queue, uint32_t& sched, uint32_t& wgs) const {
   sched = BL_AMD_SCHEDULE_GRID;
   wgs = 0;
   if (allow_queue && n_a) {
@@ -913,8 +913,19 @@ void Runner::resolve_schedule(uint32_t n_a, bool allow_queue, uint32_t& sched, u
     else if (force_schedule != BL_AMD_SCHEDULE_AUTO) { sched = force_schedule; wgs = force_wgs; }
     else if (g_schedule != BL_AMD_SCHEDULE_AUTO) { sched = g_schedule; wgs = g_queue_wgs; }
     else {
+      // A shape never tuned: longest tiles first when the tiles are a few
+      // rounds of workgroups, where a long one left for the end holds up the
+      // frame; one workgroup per tile for a frame smaller than one round
+      // (strips share out its tiles) or so large that the tail is nothing and
+      // sorting scatters the tiles of a band over the chip.  Render stage ms,
+      // grid against sorted queue: 256 tiles 0.76 / 1.02, 1024 tiles (1000
+      // polygons) 1.01 / 0.90, 2040 (cubics 1080p) 1.98 / 1.84, 8100 (pattern
+      // shapes) 1.22 / 1.21, 15 600 (glyph canvases) 1.77 / 1.51, 170 000
+      // (uneven canvases) 1.94 / 2.43.  Tiles of few segments (40 gradient
+      // panels: 25 a tile) are over before their sorting pays.
       auto it = g_tuned.find(shape_key());
       if (it != g_tuned.end()) { sched = it->second.schedule; wgs = it->second.wgs; }
+      else if (strips_for(n_a) == 1 && n_a <= 32768 && n_binned / 64 >= n_a) { sched = BL_AMD_SCHEDULE_QUEUE_HEURISTIC; wgs = 4; }
     }
   }
   if (sched == BL_AMD_SCHEDULE_QUEUE_LEARNED && g_tile_model.empty()) sched = BL_AMD_SCHEDULE_QUEUE_HEURISTIC;
@@ -928,15 +939,15 @@ void Runner::resolve_schedule(uint32_t n_a, bool allow_queue, uint32_t& sched, u
 // it hides once the tiles fill the chip.  Measured on 1000 polygons (render
 // stage ms for 1 / 2 / 4 strips): 64 tiles 1.17 / 0.82 / 0.73, 256 tiles
 // 1.01 / 0.82 / 0.89, 512 tiles 1.12 / 1.02 / 1.22, 1024 tiles
-// 1.33 / 1.47 / 1.94.
+// 1.33 / 1.47 / 1.94 (before the XCDs shared out the tiles evenly).
 uint32_t Runner::strips_for(uint32_t n_a) const {
   return n_a * 2ull <= cus ? 4u : n_a <= cus * 2ull ? 2u : 1u;
 }
 
-uint32_t Runner::render_stage(FrameScratch& s, uint32_t n_a, uint32_t n_f, uint32_t n_s, uint32_t n_g, bool allow_queue,
-                              Stats& stats) {
+uint32_t Runner::render_stage(FrameScratch& s, uint32_t n_a, uint32_t n_f, uint32_t n_s, uint32_t n_g, uint32_t n_binned,
+                              bool allow_queue, Stats& stats) {
   uint32_t sched, wgs;
-  resolve_schedule(n_a, allow_queue, sched, wgs);
+  resolve_schedule(n_a, n_binned, allow_queue, sched, wgs);
   stats.schedule = sched;
   stats.queue_wgs = sched == BL_AMD_SCHEDULE_GRID ? 0u : wgs;
   if (sched == BL_AMD_SCHEDULE_GRID) {
@@ -1060,7 +1071,7 @@ uint32_t Runner::execute_exact(Stats& stats, ScratchArena* arena, const ExactPla
     s.list_cols = (uint32_t*)take(list_style, (size_t)std::max<uint32_t>(known->n_list, 1) * 8);
     if (!s.binned || !s.list_ent || !s.list_cols) return kErrOOM;
     s.list_style = s.list_cols + std::max<uint32_t>(known->n_list, 1);
-    resolve_schedule(known->n_atiles, true, g_sched, g_wgs);
+    resolve_schedule(known->n_atiles, known->n_binned, true, g_sched, g_wgs);
     if (g_sched != BL_AMD_SCHEDULE_GRID) {
       const size_t n_a = known->n_atiles;
       if (!q_misc.reserve(1024 + 64) || !q_queue.reserve(n_a * 4) || !q_key.reserve(n_a * 4) || !q_feat.reserve(n_a * 64) ||
@@ -1187,7 +1198,7 @@ uint32_t Runner::execute_exact(Stats& stats, ScratchArena* arena, const ExactPla
 
   // Stage 3: render.
   if (!graph) HIP_OK(hipEventRecord(ev0, stream));
-  if (uint32_t r = render_stage(s, n_atiles, n_fgroups, n_sgroups, n_ggroups, !arena, stats)) return r;
+  if (uint32_t r = render_stage(s, n_atiles, n_fgroups, n_sgroups, n_ggroups, n_binned, !arena, stats)) return r;
   stats.render_kernels = (n_atiles ? 1u : 0u) | (n_sgroups ? 2u : 0u) | (n_ggroups ? 4u : 0u) | (n_fgroups ? 8u : 0u);
   if (!graph) HIP_OK(hipEventRecord(ev1, stream));
   launch_report(s, host_readback, stream);

@@ -410,8 +410,8 @@ BLAmdResult bl_amd_cost_model_train(const float* features, const float* targets,
  * The tiles of bands with path fills (the heavy part of the render stage)
  * run in one of these schedules; none changes pixels (tiles own disjoint
  * pixels):
- *   GRID             one workgroup per tile, tiles dealt to the XCDs in
- *                    contiguous ranges;
+ *   GRID             one workgroup per tile (or strip of it, in frames of
+ *                    few tiles), runs of tiles dealt to the XCDs in turn;
  *   QUEUE            a persistent grid (wgs_per_cu workgroups per CU)
  *                    draining a device work queue of the tiles in band order;
  *   QUEUE_HEURISTIC  the queue sorted longest first by each tile's binned
@@ -424,7 +424,8 @@ BLAmdResult bl_amd_cost_model_train(const float* features, const float* targets,
  *                    runs as QUEUE_HEURISTIC);
  *   AUTO (default)   the schedule the autotuner picked for frames of this
  *                    shape (tile, command and canvas counts, each by its
- *                    power of two), else GRID.
+ *                    power of two), else by a rule on the tile and segment
+ *                    counts QUEUE_HEURISTIC or GRID.
  * bl_amd_context_replay_noalloc always runs GRID. */
 enum { BL_AMD_SCHEDULE_GRID = 0, BL_AMD_SCHEDULE_QUEUE = 1, BL_AMD_SCHEDULE_QUEUE_HEURISTIC = 2,
        BL_AMD_SCHEDULE_QUEUE_LEARNED = 3, BL_AMD_SCHEDULE_AUTO = 4 };
