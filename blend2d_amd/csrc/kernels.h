@@ -79,7 +79,8 @@ struct FrameScratch {
   uint32_t* list_off;      // n_mat + 1
   // Per listed (band, command) cell:
   uint32_t* list_cols;     // n_list: tile-column range, first | last << 16
-  uint4* list_ent;         // n_list: {command, binned offset, binned count, kMeta* bits}
+  uint4* list_ent;         // n_list: {command, binned offset, binned count, kMeta* bits}; boxes:
+                           // {command, x0 | x1 << 16, 0, kMeta* bits}
   uint32_t* list_style;    // n_list: solid colour, or the style index of another kind of style
   DevSeg* binned;          // n_binned
   uint32_t* scan_tmp;      // scan_tmp_words()
@@ -116,7 +117,8 @@ struct FrameScratch {
 // What the compositor branches on, one word per list entry: CmdKind in bits
 // 0-1, then at these bits ExecOp (3), alpha (8), even-odd (1), FetchKind (3)
 // and the source format (2).
-constexpr uint32_t kMetaOp = 2, kMetaAlpha = 5, kMetaEvenOdd = 13, kMetaFetch = 14, kMetaFmt = 17;
+constexpr uint32_t kMetaOp = 2, kMetaAlpha = 5, kMetaEvenOdd = 13, kMetaFetch = 14, kMetaFmt = 17,
+                   kMetaRow0 = 20, kMetaRow1 = 25;   // boxes: rows of the band [row 0, row 1), 5 bits each
 
 size_t scan_tmp_words(void);
 

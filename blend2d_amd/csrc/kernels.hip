@@ -1097,7 +1097,14 @@ __device__ __forceinline__ void list_build(const FrameDev& f, const FrameScratch
   const DevCmd& c = f.cmds[cmd];
   const DevStyle& st = f.styles[c.style];
   s.list_cols[li] = cmd_columns(s, c, cmd, cv);
-  s.list_ent[li] = make_uint4(cmd, off, s.mat_off[i + 1] - off, cmd_meta(c, st.kind));
+  uint4 ent = make_uint4(cmd, off, s.mat_off[i + 1] - off, cmd_meta(c, st.kind));
+  if (c.kind != kCmdAnalytic) {
+    const int y0 = (int)((uint32_t)(i - cv.mat_base) / cv.n_cmds) * kTileH;
+    ent.y = (uint32_t)c.box[0] | ((uint32_t)c.box[2] << 16);
+    ent.z = 0u;
+    ent.w |= ((uint32_t)max(c.box[1] - y0, 0) << kMetaRow0) | ((uint32_t)min(c.box[3] - y0, kTileH) << kMetaRow1);
+  }
+  s.list_ent[li] = ent;
   s.list_style[li] = st.kind == kFetchSolid ? st.solid : c.style;
 }
 
@@ -1122,8 +1129,9 @@ __device__ __forceinline__ void tile_setup(const FrameDev& f, const FrameScratch
 // Per box tile group two header words: {canvas, the band's command
 // list range, group column | band << 16} and the destination address of the
 // group's first pixel {address low, address high, stride, width left of the
-// group's first pixel | valid rows << 16 | A8 << 21 | tiles << 24}, so the
-// compositor needs no canvas record.
+// group's first pixel | valid rows << 16 | A8 << 21 | fresh << 22 | tiles << 24},
+// so the compositor needs no canvas record.  fresh: the canvas's first command
+// copies an opaque colour over the whole group.
 __device__ __forceinline__ void group_setup(const FrameDev& f, const FrameScratch& s, uint32_t i) {
   uint32_t lo = 0, hi = f.n_canvases;
   while (hi - lo > 1) {
@@ -1146,10 +1154,15 @@ __device__ __forceinline__ void group_setup(const FrameDev& f, const FrameScratc
   const uint32_t rows = cv.h - y0 < (uint32_t)kTileH ? cv.h - y0 : (uint32_t)kTileH;
   const uint32_t a8 = cv.format == kFmtA8 ? 1u : 0u;
   const uint64_t ptr = cv.ptr + (uint64_t)((int64_t)y0 * cv.stride) + (uint64_t)x0 * (a8 ? 1u : 4u);
+  const DevCmd& first = f.cmds[cv.cmd_base];
+  const DevStyle& fs = f.styles[first.style];
+  const uint32_t fresh = first.kind == kCmdBoxA && first.alpha == 255u && fs.kind == kFetchSolid &&
+                         (first.op == kOpSrcCopy || (first.op == kOpSrcOver && (fs.solid >> 24) == 255u)) && first.box[0] <= (int)x0 && first.box[1] <= (int)y0 &&
+                         first.box[2] >= (int)min(cv.w, x0 + kGroupTiles * kTileW) && first.box[3] >= (int)(y0 + rows);
   uint4* h = s.group_hdr + 2 * (size_t)slot;
   h[0] = make_uint4(lo, s.list_off[row_base], s.list_off[row_base + cv.n_cmds], col | (band << 16));
   h[1] = make_uint4((uint32_t)ptr, (uint32_t)(ptr >> 32), (uint32_t)cv.stride,
-                    (cv.w - x0) | (rows << 16) | (a8 << 21) | (ntiles << 24));
+                    min(cv.w - x0, 0xFFFFu) | (rows << 16) | (a8 << 21) | (fresh << 22) | (ntiles << 24));
 }
 
 // Lists, scatter cursors and headers in one launch.
@@ -1178,40 +1191,6 @@ void launch_setup(const FrameDev& f, const FrameScratch& s, hipStream_t st) {
 // reads a thread's four cells with one 128-bit load.
 __device__ __forceinline__ int cell_index(int row, int x) {
   return row * kTileW + ((((x >> 2) ^ row) & 15) << 2) + (x & 3);
-}
-
-// Per-command record staged in LDS for the render loop.
-struct RenderRecData {
-  DevCmd cmd;
-  DevStyle style;
-  int32_t min_y;       // fill-row origin of analytic fills (24.8)
-  int32_t pad;
-};
-union RenderRec {
-  RenderRecData r;
-  uint32_t w[sizeof(RenderRecData) / 4];
-};
-constexpr int kRecWords = (int)(sizeof(RenderRecData) / 4);
-static_assert(sizeof(DevCmd) % 8 == 0, "DevStyle must stay 8-byte aligned in the record");
-
-// Records staged together by the box compositor (double buffered).
-constexpr int kBatch = 7;
-static_assert(kBatch * kRecWords <= 2 * kTileThreads, "two record words per thread");
-
-// Word `w` of the record of command `cmd_i` (style index `style_i`).
-__device__ __forceinline__ uint32_t rec_word(const FrameDev& f, const FrameScratch& s, uint32_t cmd_i, uint32_t style_i, int w) {
-  constexpr int kCmdW = (int)(sizeof(DevCmd) / 4), kStyleW = (int)(sizeof(DevStyle) / 4);
-  if (w < kCmdW) return ((const uint32_t*)(f.cmds + cmd_i))[w];
-  if (w < kCmdW + kStyleW) return ((const uint32_t*)(f.styles + style_i))[w - kCmdW];
-  if (w == kCmdW + kStyleW) return (uint32_t)s.bounds[cmd_i].min_y;
-  return 0u;
-}
-
-// Word `gw` of the records of the batch that starts at selected command `kb`.
-__device__ __forceinline__ uint32_t batch_rec_word(const FrameDev& f, const FrameScratch& s, const uint32_t* sel_cmd,
-                                                   const uint32_t* sel_style, uint32_t kb, int gw) {
-  const int b = gw / kRecWords, w = gw - b * kRecWords;
-  return rec_word(f, s, sel_cmd[kb + b], sel_style[kb + b], w);
 }
 
 // First pass over one binned segment of an analytic fill, for the rows
@@ -1252,111 +1231,6 @@ __device__ __forceinline__ void raster_row(const DevSeg& g, uint32_t* cells, uin
     if (v) atomicAdd(&cells[cell_index(lr, k)], v);
   });
   if (bd) atomicAdd(&backdrop[lr], bd);
-}
-
-// Destination pixels px .. px + 3 of a row (zero where outside the canvas).
-__device__ __forceinline__ void load4(const uint8_t* rowp, int px, int w, bool a8, uint32_t d[4]) {
-  const bool full4 = px + 3 < w;
-  if (a8) {
-    if (full4 && (((uintptr_t)(rowp + px)) & 3) == 0) {
-      const uint32_t v = *(const uint32_t*)(rowp + px);
-#pragma unroll
-      for (int k = 0; k < 4; k++) d[k] = (v >> (8 * k)) & 0xFFu;
-    }
-    else {
-#pragma unroll
-      for (int k = 0; k < 4; k++) d[k] = px + k < w ? rowp[px + k] : 0u;
-    }
-  }
-  else {
-    const uint32_t* r32 = (const uint32_t*)rowp;
-    if (full4 && (((uintptr_t)(r32 + px)) & 15) == 0) {
-      const uint4 v = *(const uint4*)(r32 + px);
-      d[0] = v.x; d[1] = v.y; d[2] = v.z; d[3] = v.w;
-    }
-    else {
-#pragma unroll
-      for (int k = 0; k < 4; k++) d[k] = px + k < w ? r32[px + k] : 0u;
-    }
-  }
-}
-
-__device__ __forceinline__ void store4(uint8_t* rowp, int px, int w, bool a8, const uint32_t d[4]) {
-  const bool full4 = px + 3 < w;
-  if (a8) {
-    if (full4 && (((uintptr_t)(rowp + px)) & 3) == 0) {
-      *(uint32_t*)(rowp + px) = d[0] | (d[1] << 8) | (d[2] << 16) | (d[3] << 24);
-    }
-    else {
-#pragma unroll
-      for (int k = 0; k < 4; k++) if (px + k < w) rowp[px + k] = (uint8_t)d[k];
-    }
-  }
-  else {
-    uint32_t* r32 = (uint32_t*)rowp;
-    if (full4 && (((uintptr_t)(r32 + px)) & 15) == 0) {
-      *(uint4*)(r32 + px) = make_uint4(d[0], d[1], d[2], d[3]);
-    }
-    else {
-#pragma unroll
-      for (int k = 0; k < 4; k++) if (px + k < w) r32[px + k] = d[k];
-    }
-  }
-}
-
-// Masks of pixels px .. px + 3 of row y for a box fill.
-__device__ __forceinline__ void box_masks4(const FrameDev& f, const DevCmd& c, int y, int px, uint32_t m[4]) {
-#pragma unroll
-  for (int k = 0; k < 4; k++) m[k] = 0u;
-  if (y < c.box[1] || y >= c.box[3]) return;
-  if (c.kind == kCmdBoxA) {
-#pragma unroll
-    for (int k = 0; k < 4; k++) m[k] = (px + k >= c.box[0] && px + k < c.box[2]) ? c.alpha : 0u;
-  }
-  else if (c.kind == kCmdBoxM) {
-    // FillMask with a VMaskA8 command (rendercommandprocsync_p.h:65-84,
-    // compopgeneric_p.h:165-183): byte x - x0 of the mask row, times the
-    // alpha below full alpha.  The view is exactly the box (host-checked), so
-    // every byte read lies in row y - y0 of the view.
-    const DevImage& mi = f.images[c.box_mask[0]];
-    const uint8_t* row = (const uint8_t*)mi.ptr + (int64_t)(y - c.box[1]) * mi.stride;
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-      const int x = px + k;
-      if (x >= c.box[0] && x < c.box[2]) {
-        const uint32_t v = row[x - c.box[0]];
-        m[k] = c.alpha >= 255u ? v : pipe::div255(v * c.alpha);
-      }
-    }
-  }
-  else {
-    const int kind = (y == c.box_row_first) ? 0 : (y == c.box_row_last) ? 2 : 1;
-    const uint32_t rm = c.box_mask[kind];
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-      const int x = px + k;
-      if (x >= c.box[0] && x < c.box[2]) {
-        const int col = (x == c.box[0]) ? 0 : (x == c.box[2] - 1) ? 2 : 1;
-        m[k] = (rm >> (8 * col)) & 0xFFu;
-      }
-    }
-  }
-}
-
-// Fetch and composite of pixels px .. px + 3 under masks m; returns how many
-// were composited.
-template<bool kSolid = false, bool kDither = false>
-__device__ __forceinline__ uint32_t composite4(const FrameDev& f, const DevCmd& c, const DevStyle& st, const pipe::Row& rs,
-                                               int px, int w, bool a8, const uint32_t m[4], uint32_t d[4]) {
-  uint32_t n = 0;
-#pragma unroll
-  for (int k = 0; k < 4; k++) {
-    if (!m[k] || px + k >= w) continue;
-    const uint32_t src = kSolid ? st.solid : pipe::fetch<kDither>(st, rs, px + k, f.luts, f.images, c.src_fmt);
-    d[k] = a8 ? pipe::composite8(c.op, d[k], src >> 24, m[k]) : pipe::composite32(c.op, d[k], src, m[k]);
-    n++;
-  }
-  return n;
 }
 
 // Composited pixels of one wave or workgroup, into one of 64 counters (the
@@ -1422,25 +1296,36 @@ constexpr uint32_t kTileGroup = 64u / kTileBatch * kTileBatch;   // selected ent
 
 // Masks of pixels px .. px + N - 1 of row y for a box fill (uniform command).
 template<int N>
-__device__ __forceinline__ void box_masks_n(const FrameDev& f, pipe::CPtr<DevCmd> c, uint32_t kind, uint32_t alpha, int y, int px,
-                                            uint32_t m[N]) {
-  const int bx0 = c->box[0], by0 = c->box[1], bx1 = c->box[2], by1 = c->box[3];
-  const bool row_in = y >= by0 && y < by1;
+__device__ __forceinline__ void box_masks_n(const FrameDev& f, uint4 ent, int y, int px, uint32_t m[N]) {
+  const uint32_t kind = ent.w & 3u, alpha = (ent.w >> kMetaAlpha) & 0xFFu;
+  const int bx0 = (int)(ent.y & 0xFFFFu), bx1 = (int)(ent.y >> 16);
+  const uint32_t row = (uint32_t)y % kTileH;
+  const bool row_in = row >= ((ent.w >> kMetaRow0) & 31u) && row < ((ent.w >> kMetaRow1) & 31u);
   if (kind == kCmdBoxA) {
 #pragma unroll
     for (int k = 0; k < N; k++) m[k] = (row_in && px + k >= bx0 && px + k < bx1) ? alpha : 0u;
+    return;
   }
-  else if (kind == kCmdBoxM) {
+  const pipe::CPtr<DevCmd> c = pipe::cptr(f.cmds + ent.x);
+  if (kind == kCmdBoxM) {
     // FillMask with a VMaskA8 command (rendercommandprocsync_p.h:65-84,
     // compopgeneric_p.h:165-183): byte x - x0 of the mask row, times the
     // alpha below full alpha.  The view is exactly the box (host-checked), so
     // every byte read lies in row y - y0 of the view.
     const pipe::CPtr<DevImage> mi = pipe::cptr(f.images + c->box_mask[0]);
-    const pipe::GBytes row = pipe::global_bytes(mi->ptr) + (int64_t)(y - by0) * mi->stride - bx0;
+    const pipe::GBytes bytes = pipe::global_bytes(mi->ptr) + (int64_t)(y - c->box[1]) * mi->stride - bx0;
+    if (N == 4 && row_in && px >= bx0 && px + 3 < bx1) {
+      typedef uint32_t bytes4 __attribute__((aligned(1)));
+      const uint32_t v = *(const B2AMD_GLOBAL bytes4*)(bytes + px);
 #pragma unroll
-    for (int k = 0; k < N; k++) {
-      m[k] = 0u;
-      if (row_in && px + k >= bx0 && px + k < bx1) m[k] = row[px + k];
+      for (int k = 0; k < N; k++) m[k] = (v >> (8 * k)) & 0xFFu;
+    }
+    else {
+#pragma unroll
+      for (int k = 0; k < N; k++) {
+        m[k] = 0u;
+        if (row_in && px + k >= bx0 && px + k < bx1) m[k] = bytes[px + k];
+      }
     }
     if (alpha < 255u) {
 #pragma unroll
@@ -1459,6 +1344,81 @@ __device__ __forceinline__ void box_masks_n(const FrameDev& f, pipe::CPtr<DevCmd
   }
 }
 
+// Masks of four pixels from px on in each of R rows from y on (uniform), one
+// byte each, for a box that isn't kCmdBoxA.  All rows' bytes are loaded before
+// any is used.
+template<int R>
+__device__ __forceinline__ void box_mask_rows(const FrameDev& f, uint4 ent, int y, int px, uint32_t pm[R]) {
+  const uint32_t alpha = (ent.w >> kMetaAlpha) & 0xFFu;
+  const int bx0 = (int)(ent.y & 0xFFFFu), bx1 = (int)(ent.y >> 16);
+  const pipe::CPtr<DevCmd> c = pipe::cptr(f.cmds + ent.x);
+  const int by0 = c->box[1], by1 = c->box[3];
+#pragma unroll
+  for (int r = 0; r < R; r++) pm[r] = 0u;
+  if ((ent.w & 3u) == kCmdBoxM) {
+    // see box_masks_n; rows outside the box read its nearest one and drop it
+    const pipe::CPtr<DevImage> mi = pipe::cptr(f.images + c->box_mask[0]);
+    const pipe::GBytes at = pipe::global_bytes(mi->ptr) - bx0;
+    const int64_t stride = mi->stride;
+    auto row = [&](int r) { return at + (int64_t)(min(max(y + r, by0), by1 - 1) - by0) * stride; };
+    if (px >= bx0 && px + 3 < bx1) {
+      typedef uint32_t bytes4 __attribute__((aligned(1)));
+#pragma unroll
+      for (int r = 0; r < R; r++) pm[r] = *(const B2AMD_GLOBAL bytes4*)(row(r) + px);
+    }
+    else if (px < bx1 && px + 3 >= bx0) {
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        if (px + k < bx0 || px + k >= bx1) continue;
+#pragma unroll
+        for (int r = 0; r < R; r++) pm[r] |= (uint32_t)row(r)[px + k] << (8 * k);
+      }
+    }
+    if (alpha < 255u) {
+#pragma unroll
+      for (int r = 0; r < R; r++) {
+        const pipe::Px p = pipe::px_of(pm[r]);
+        pm[r] = pipe::px_bits(pipe::Px{pipe::div255p(p.rb * (uint16_t)alpha), pipe::div255p(p.ag * (uint16_t)alpha)});
+      }
+    }
+  }
+  else {
+    const uint32_t top = c->box_mask[0], mid = c->box_mask[1], bot = c->box_mask[2];
+    const int first = c->box_row_first, last = c->box_row_last;
+    uint32_t sh[4];
+    bool in[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const int x = px + k;
+      sh[k] = x == bx0 ? 0u : x == bx1 - 1 ? 16u : 8u;
+      in[k] = x >= bx0 && x < bx1;
+    }
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      const uint32_t rm = y + r == first ? top : y + r == last ? bot : mid;
+#pragma unroll
+      for (int k = 0; k < 4; k++) pm[r] |= in[k] ? ((rm >> sh[k]) & 0xFFu) << (8 * k) : 0u;
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < R; r++)
+    if (y + r < by0 || y + r >= by1) pm[r] = 0u;
+}
+
+// A solid colour over the whole wave under one mask (32-bit SRC_OVER and
+// SRC_COPY): composited with the source terms formed once; false otherwise.
+template<int N>
+__device__ __forceinline__ bool solid_flat(uint32_t op, uint32_t color, const uint32_t m[N], pipe::Px d[N]) {
+  if (op > kOpSrcOver) return false;
+  const uint32_t m0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)m[0]);
+  uint32_t diff = m[0] ^ m0;
+#pragma unroll
+  for (int k = 1; k < N; k++) diff |= m[k] ^ m0;
+  if (__ballot(diff != 0u)) return false;
+  pipe::composite32_flat<N>(op, d, color, m0);
+  return true;
+}
+
 // One command's pixels: fetch and composite under masks m.
 template<int N, bool kDither>
 __device__ __forceinline__ void apply_n(const FrameDev& f, const FrameScratch& s, uint32_t meta, uint32_t cmd, uint32_t style,
@@ -1467,16 +1427,7 @@ __device__ __forceinline__ void apply_n(const FrameDev& f, const FrameScratch& s
   constexpr int kPairs = (N + 1) / 2;
   uint32_t src[N];
   if (fetch == kFetchSolid) {
-    if (!a8 && op <= kOpSrcOver) {
-      const uint32_t m0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)m[0]);
-      uint32_t diff = m[0] ^ m0;
-#pragma unroll
-      for (int k = 1; k < N; k++) diff |= m[k] ^ m0;
-      if (__ballot(diff != 0u) == 0ull) {
-        pipe::composite32_flat<N>(op, d, style, m0);
-        return;
-      }
-    }
+    if (!a8 && solid_flat<N>(op, style, m, d)) return;
 #pragma unroll
     for (int k = 0; k < N; k++) src[k] = style;
   }
@@ -1509,9 +1460,13 @@ __device__ __forceinline__ void apply_n(const FrameDev& f, const FrameScratch& s
     return;
   }
   pipe::Px sp[N];
+  pipe::u16x2 mm[N];
 #pragma unroll
-  for (int k = 0; k < N; k++) sp[k] = pipe::px_of(src[k]);
-  pipe::composite32_n<N>(op, d, sp, m, fetch >= kFetchPatternNN);
+  for (int k = 0; k < N; k++) {
+    sp[k] = pipe::px_of(src[k]);
+    mm[k] = pipe::both(m[k]);
+  }
+  pipe::composite32_n<N>(op, d, sp, mm, fetch >= kFetchPatternNN);
 }
 
 // Destination pixels px .. px + N - 1 of a row, as pairs (A8: neighbouring
@@ -1550,7 +1505,7 @@ __device__ __forceinline__ void load_px(const uint8_t* rowp, int px, int w, bool
   for (int k = 0; k < N; k++) d[k] = pipe::px_of(v[k]);
 }
 
-template<int N>
+template<int N, bool kStream = false>
 __device__ __forceinline__ void store_px(uint8_t* rowp, int px, int w, bool a8, const pipe::Px d[N]) {
   if (a8) {
     uint32_t v[N];
@@ -1573,7 +1528,10 @@ __device__ __forceinline__ void store_px(uint8_t* rowp, int px, int w, bool a8, 
 #pragma unroll
   for (int k = 0; k < N; k++) v[k] = pipe::px_bits(d[k]);
   if (N == 4 && px + 3 < w && (((uintptr_t)(r32 + px)) & 15) == 0) {
-    *(uint4*)(r32 + px) = make_uint4(v[0], v[1 % N], v[2 % N], v[3 % N]);
+    typedef uint32_t words4 __attribute__((ext_vector_type(4)));
+    const words4 q = {v[0], v[1 % N], v[2 % N], v[3 % N]};
+    if (kStream) __builtin_nontemporal_store(q, (words4*)(r32 + px));
+    else *(words4*)(r32 + px) = q;
   }
   else {
 #pragma unroll
@@ -1810,7 +1768,7 @@ __device__ __forceinline__ uint32_t render_tile(const FrameDev& f, const FrameSc
             }
           }
           else {
-            box_masks_n<N>(f, pipe::cptr(f.cmds + lane_value(ent.x, p)), meta & 3u, alpha, y, px, m);
+            box_masks_n<N>(f, make_uint4(lane_value(ent.x, p), lane_value(ent.y, p), 0u, meta), y, px, m);
           }
           uint32_t n = 0;
 #pragma unroll
@@ -2017,306 +1975,235 @@ __global__ __launch_bounds__(kQueueBuckets) void k_tile_scatter(FrameDev f, Fram
 }
 
 // Bands with box fills only: one workgroup per group of up to 4 tiles of a
-// band (256 x 16 pixels, 16 pixels per thread).  No coverage cells are
-// needed, so the workgroup is light, and one walk of the band's command list
-// and records serves four tiles.
+// band (256 x 16 pixels).  What bounds them is memory: every destination pixel
+// read and written once, a blit's or mask's pixels read once.  So wave w takes
+// rows 4w .. 4w + 3 and lane l the pixels 4l .. 4l + 3 of each: every load and
+// store of a wave moves one contiguous 1 KB row segment, those of four rows are
+// in flight together, and no LDS or barrier keeps waves from filling the CU.
+// The band's commands (kind, colour and box of 64 at a time) sit in the lanes
+// of the wave and are read into scalar registers, so that all branches are
+// scalar; a command's own fields are read once for the four rows.  Where the
+// canvas's first command is an opaque colour over the whole group the
+// destination isn't read at all.
 //
-// A thread's 16 pixels are four quads.  Solid styles (the pure compositing
-// load): wave w takes rows 4w .. 4w + 3 of the group and lane l the pixels
-// 4l .. 4l + 3 of each, so every load and store instruction of a wave moves
-// one contiguous 1 KB row segment (lane-contiguous accesses measured 25 %
-// faster than 64 contiguous bytes per thread).  Other styles keep one row
-// per thread, four consecutive quads along it, so their per-row fetch setup
-// is done once per command.
-template<bool kSolid, bool kDither = false>
+// Instances: solid SRC_OVER / SRC_COPY aligned boxes on 32-bit canvases
+// (fast), other solid styles, and every style.  Measured against one thread
+// per 16 pixels of a row with records in LDS, 4K canvases: four with three
+// translucent layers each 72 -> 40 us (fresh; 54 with the layers composited per
+// pixel), four with an image, a half-size one at a fraction or scaled and 24
+// sprites 422 -> 119, two with a colour through a mask 70 -> 43 and two with a
+// gradient through another above it 117 -> 48.  What is left there: the vector
+// instructions of the composite, and at 4 waves per SIMD the latency of the
+// header, list and source loads.  Streaming stores took 3 to 6 % off.
+enum BoxClass { kBoxFast, kBoxSolid, kBoxGeneral };
+
+template<int kClass, bool kDither>
 __device__ __forceinline__ void render_box(const FrameDev& f, const FrameScratch& s, uint32_t n) {
+  constexpr int kRows = 4;
   const uint32_t slot = xcd_tile(blockIdx.x);
   if (slot >= n) return;
-  // Headers: the fast bands' groups first, then the solid ones, then the
-  // general ones.  The check is uniform, as in k_render.
-  const uint32_t n_groups = (kSolid ? s.sgroup_off : s.ggroup_off)[f.n_bands];
-  if (slot >= n_groups) return;
-  const size_t hi = 2 * ((size_t)slot + s.fgroup_off[f.n_bands] + (kSolid ? 0u : s.sgroup_off[f.n_bands]));
-  const uint4 gh = s.group_hdr[hi];
-  const uint4 gd = s.group_hdr[hi + 1];
-  const uint32_t pool_flags = s.flags ? *s.flags : 0u;
-  const int t = threadIdx.x;
-  const uint32_t lb = gh.y, le = gh.z;
-  const uint32_t band = gh.w >> 16;
-  const uint32_t tc0 = (gh.w & 0xFFFFu) * kGroupTiles;
-  const uint32_t ntiles = gd.w >> 24;
-  const uint32_t tc1 = tc0 + ntiles - 1;
-  if (pool_flags) return;
-
-  const int lane = t & 63, wave = t >> 6;
-  const int X0 = (int)tc0 * kTileW;
-  const int w = X0 + (int)(gd.w & 0xFFFFu);        // canvas width
-  const int rows = (int)((gd.w >> 16) & 0x1Fu);    // rows of the band inside the canvas
-  const bool a8 = (gd.w >> 21) & 1u;
-  // quad g: group row qrow(g), first pixel qx(g)
-  const int row0 = kSolid ? wave * 4 : t >> 4;
-  auto qrow = [&](int g) { return kSolid ? row0 + g : row0; };
-  auto qx = [&](int g) { return kSolid ? X0 + lane * 4 : X0 + (t & 15) * 16 + 4 * g; };
-  // the thread's pixel span, for skipping commands that miss it
-  const int span_x0 = qx(0), span_x1 = kSolid ? qx(0) + 4 : qx(0) + 16;
-  const int span_y0 = (int)band * kTileH + row0, span_y1 = span_y0 + (kSolid ? 4 : 1);
-  const bool any_row = row0 < rows;
-
-  // destination pointer of the group's row 0, offset so that pixel x is at
-  // base + x * bpp
-  uint8_t* const base = (uint8_t*)(((uint64_t)gd.y << 32) | gd.x) - (int64_t)X0 * (a8 ? 1 : 4);
-  const int64_t stride = (int32_t)gd.z;
-  uint32_t d[4][4];
+  // headers: the fast bands' groups first, then the solid ones, then the
+  // general ones.  n is at most the number of all groups: a fast group's header
+  // is loaded together with the counts.
+  const uint32_t n_fast = s.fgroup_off[f.n_bands], n_solid = s.sgroup_off[f.n_bands];
+  const uint32_t count_of = kClass == kBoxFast ? n_fast : kClass == kBoxSolid ? n_solid : s.ggroup_off[f.n_bands];
+  const uint32_t failed = s.flags ? *s.flags : 0u;   // pool overflow: nothing is composited
+  const uint32_t before = kClass == kBoxFast ? 0u : kClass == kBoxSolid ? n_fast : n_fast + n_solid;
+  if (kClass != kBoxFast && (slot >= count_of || failed)) return;
+  const pipe::CPtr<uint32_t> h = pipe::cptr((const uint32_t*)(s.group_hdr + 2 * ((size_t)before + slot)));
+  const uint32_t lb = h[1], le = h[2], where = h[3], shape = h[7];
+  const uint64_t ptr = ((uint64_t)h[5] << 32) | h[4];
+  const int64_t stride = (int32_t)h[6];
+  if (slot >= count_of || failed) return;
+  const int lane = threadIdx.x & 63;
+  const int row0 = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) * kRows;
+  const int rows = min((int)((shape >> 16) & 0x1Fu) - row0, kRows);   // the wave's rows inside the canvas
+  if (rows <= 0) return;
+  const uint32_t tc0 = (where & 0xFFFFu) * kGroupTiles;
+  const int X0 = (int)tc0 * kTileW, w = X0 + (int)(shape & 0xFFFFu);
+  const int Y = (int)(where >> 16) * kTileH + row0;
+  const bool a8 = kClass != kBoxFast && ((shape >> 21) & 1u);
+  const bool fresh = (shape >> 22) & 1u;
+  const int px = X0 + lane * 4;
+  const int xr = min(X0 + (int)kGroupTiles * kTileW, w);   // right end of the group's pixels
+  // the wave's first row, so that pixel x is at base + x * bytes per pixel
+  uint8_t* const base = (uint8_t*)ptr + row0 * stride - (int64_t)X0 * (a8 ? 1 : 4);
+  // masks of four pixels in a word
+  const int n_in = min(max(w - px, 0), 4);
+  const uint32_t in_mask = n_in == 4 ? 0xFFFFFFFFu : (1u << (8 * n_in)) - 1u;
+  auto count = [&](uint32_t pm) {
+    uint32_t c = 0;
 #pragma unroll
-  for (int g = 0; g < 4; g++) {
+    for (int k = 0; k < 4; k++) c += (uint32_t)__popcll(__ballot((pm & in_mask & (0xFFu << (8 * k))) != 0u));
+    return c;
+  };
+
+  pipe::Px d[kRows][4];
 #pragma unroll
-    for (int k = 0; k < 4; k++) d[g][k] = 0u;
-    if (qrow(g) < rows && qx(g) < w) load4(base + qrow(g) * stride, qx(g), w, a8, d[g]);
+  for (int r = 0; r < kRows; r++) {
+#pragma unroll
+    for (int k = 0; k < 4; k++) d[r][k] = pipe::px_of(0u);
+    if (!fresh && r < rows) load_px<4>(base + r * stride, px, w, a8, d[r]);
   }
+  // While the pixels of a fresh group are one value, that value alone is
+  // composited.
+  bool one = kClass == kBoxFast ? fresh : fresh && !a8;
+  pipe::Px value[1] = {pipe::px_of(0u)};
+  auto spread = [&]() {
+    if (!one) return;
+    one = false;
+#pragma unroll
+    for (int r = 0; r < kRows; r++)
+#pragma unroll
+      for (int k = 0; k < 4; k++) d[r][k] = value[0];
+  };
 
-  bool touched = false;
-  uint32_t npix = 0;
-  __shared__ uint32_t sel_cmd[kTileThreads], sel_style[kTileThreads];
-  __shared__ uint32_t sel_wave[kTileThreads / 64];
-  __shared__ RenderRec rec[2][kBatch];
-
-  for (uint32_t chunk = lb; chunk < le; chunk += kTileThreads) {
-    const uint32_t li = chunk + (uint32_t)t;
-    uint32_t cmd_i = 0, style_i = 0;
-    bool keep = false;
+  uint32_t npix = 0, touched = 0;   // touched: bit r, row r
+  for (uint32_t chunk = lb; chunk < le; chunk += 64u) {
+    // up to 64 commands in the lanes
+    const uint32_t li = chunk + (uint32_t)lane;
+    uint4 ent = make_uint4(0u, 0u, 0u, 0u);
+    uint32_t style = 0;
+    bool on = false;
     if (li < le) {
-      const uint32_t cols = s.list_cols[li];
-      cmd_i = s.list_ent[li].x;
-      style_i = f.cmds[cmd_i].style;
-      keep = (cols & 0xFFFFu) <= tc1 && (cols >> 16) >= tc0;
+      ent = s.list_ent[li];
+      style = s.list_style[li];
+      on = (int)(ent.y & 0xFFFFu) < xr && (int)(ent.y >> 16) > X0 && (int)((ent.w >> kMetaRow0) & 31u) < row0 + rows &&
+           (int)((ent.w >> kMetaRow1) & 31u) > row0;
     }
-    const uint64_t bal = __ballot(keep);
-    if (lane == 0) sel_wave[wave] = (uint32_t)__popcll(bal);
-    __syncthreads();
-    uint32_t off = 0, n_sel = 0;
-#pragma unroll
-    for (int wv = 0; wv < kTileThreads / 64; wv++) {
-      const uint32_t cw = sel_wave[wv];
-      off += wv < wave ? cw : 0u;
-      n_sel += cw;
-    }
-    if (keep) {
-      const uint32_t slot = off + (uint32_t)__popcll(bal & ((1ull << lane) - 1ull));
-      sel_cmd[slot] = cmd_i;
-      sel_style[slot] = style_i;
-    }
-    __syncthreads();
-    if (n_sel == 0) continue;
+    for (uint64_t bits = __ballot(on); bits; bits &= bits - 1ull) {
+      const uint32_t p = (uint32_t)__builtin_ctzll(bits);
+      const uint32_t cmd = lane_value(ent.x, p), xs = lane_value(ent.y, p), meta = lane_value(ent.w, p), st = lane_value(style, p);
+      const uint32_t alpha = (meta >> kMetaAlpha) & 0xFFu, op = (meta >> kMetaOp) & 7u, fetch = (meta >> kMetaFetch) & 7u;
+      const int x0 = (int)(xs & 0xFFFFu), x1 = (int)(xs >> 16);
+      const int ra = max((int)((meta >> kMetaRow0) & 31u) - row0, 0);
+      const int rb = min((int)((meta >> kMetaRow1) & 31u) - row0, rows);   // rows ra .. rb - 1 (not empty)
+      const uint32_t row_bits = (1u << rb) - (1u << ra);
 
-    {
-      const uint32_t nb = n_sel < (uint32_t)kBatch ? n_sel : (uint32_t)kBatch;
-      if (t < (int)nb * kRecWords) rec[0][t / kRecWords].w[t % kRecWords] = batch_rec_word(f, s, sel_cmd, sel_style, 0, t);
-      if (t + kTileThreads < (int)nb * kRecWords) {
-        const int gw = t + kTileThreads;
-        rec[0][gw / kRecWords].w[gw % kRecWords] = batch_rec_word(f, s, sel_cmd, sel_style, 0, gw);
-      }
-    }
-    __syncthreads();
-
-    for (uint32_t kb = 0, bi = 0; kb < n_sel; kb += kBatch, bi++) {
-      const int cur = (int)(bi & 1u);
-      const uint32_t nb = n_sel - kb < (uint32_t)kBatch ? n_sel - kb : (uint32_t)kBatch;
-      const uint32_t kn = kb + kBatch;
-      const bool has_next = kn < n_sel;
-      uint32_t pw0 = 0, pw1 = 0;
-      int nwn = 0;
-      if (has_next) {
-        const uint32_t nbn = n_sel - kn < (uint32_t)kBatch ? n_sel - kn : (uint32_t)kBatch;
-        nwn = (int)nbn * kRecWords;
-        if (t < nwn) pw0 = batch_rec_word(f, s, sel_cmd, sel_style, kn, t);
-        if (t + kTileThreads < nwn) pw1 = batch_rec_word(f, s, sel_cmd, sel_style, kn, t + kTileThreads);
-      }
-      for (uint32_t b = 0; b < nb; b++) {
-        const DevCmd& c = rec[cur][b].r.cmd;
-        if (c.kind == kCmdAnalytic || !any_row) continue;
-        if (span_y1 <= c.box[1] || span_y0 >= c.box[3] || span_x1 <= c.box[0] || span_x0 >= c.box[2]) continue;
-        touched = true;
-        const DevStyle& st = rec[cur][b].r.style;
-        const pipe::Row rs = kSolid ? pipe::Row{} : pipe::row_setup(st, span_y0, (int)c.fetch_row0, 0u);
-        if (kSolid && !a8 && c.kind == kCmdBoxA && (c.op == kOpSrcOver || c.op == kOpSrcCopy) && c.alpha) {
-          // The pure compositing load: a solid colour under one constant
-          // mask (an aligned box's alpha) over PRGB32.  Everything that
-          // depends on the source alone is formed once per command; per
-          // pixel only the destination terms of composite32 remain (same
-          // arithmetic, so the same bits), selected where the box and the
-          // canvas cover the pixel.
-          const uint32_t m = c.alpha, src = st.solid;
-          const bool over = c.op == kOpSrcOver;
-          const uint32_t s_rb = (src & 0x00FF00FFu) * m, s_ag = ((src >> 8) & 0x00FF00FFu) * m;
-          const uint32_t s1 = pipe::div255x2(s_rb) | (pipe::div255x2(s_ag) << 8);
-          const uint32_t k = over ? (s1 >> 24) ^ 0xFFu : m ^ 0xFFu;   // destination factor
-          const uint32_t add_rb = over ? 0u : s_rb, add_ag = over ? 0u : s_ag;
-          const uint32_t add_px = over ? s1 : 0u;
-          const int bx0 = c.box[0], bx1 = c.box[2] < w ? c.box[2] : w;
-#pragma unroll
-          for (int g = 0; g < 4; g++) {
-            const int yg = (int)band * kTileH + qrow(g);
-            const bool row_in = qrow(g) < rows && yg >= c.box[1] && yg < c.box[3];
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-              const bool in = row_in && span_x0 + j >= bx0 && span_x0 + j < bx1;
-              const uint32_t dv = d[g][j];
-              const uint32_t rb = pipe::div255x2((dv & 0x00FF00FFu) * k + add_rb);
-              const uint32_t ag = pipe::div255x2(((dv >> 8) & 0x00FF00FFu) * k + add_ag);
-              d[g][j] = in ? (rb | (ag << 8)) + add_px : dv;
-              npix += in ? 1u : 0u;
-            }
+      uint32_t pm[kRows];
+      bool full = false;   // one mask, alpha, for every pixel of the group
+      if (kClass == kBoxFast || (meta & 3u) == kCmdBoxA) {
+        // a box that goes past the canvas's right edge of the group takes
+        // every lane: those pixels are neither counted nor stored, and a whole
+        // wave under one mask is cheaper
+        full = x0 <= X0 && x1 >= xr;
+        uint32_t on4 = 0xFFFFFFFFu;
+        if (!full) {
+          const int n0 = min(max(x0 - px, 0), 4), n1 = min(max(x1 - px, 0), 4);
+          on4 = (uint32_t)((1ull << (8 * n1)) - 1u) & ~(uint32_t)((1ull << (8 * n0)) - 1u);
+        }
+        pm[0] = on4 & (alpha * 0x01010101u);
+        const uint32_t c = count(pm[0]);
+        if (!c) continue;
+        npix += c * (uint32_t)(rb - ra);
+        touched |= row_bits;
+        if ((kClass == kBoxFast || (fetch == kFetchSolid && !a8)) && op <= kOpSrcOver && full) {
+          if (one && row_bits == (1u << rows) - 1u) {
+            pipe::composite32_flat<1>(op, value, st, alpha);
+            continue;
           }
+          spread();
+#pragma unroll
+          for (int r = 0; r < kRows; r++)
+            if ((row_bits >> r) & 1u) pipe::composite32_flat<4>(op, d[r], st, alpha);
           continue;
         }
-        // One composite body for the four pixel quads: quad g is always in
-        // d[0], the quads rotate through it.
-#pragma unroll 1
-        for (int g = 0; g < 4; g++) {
-          uint32_t m[4];
-          const int px = qx(g);
-          box_masks4(f, c, (int)band * kTileH + qrow(g), px, m);
-          if (qrow(g) < rows) npix += composite4<kSolid, kDither>(f, c, st, rs, px, w, a8, m, d[0]);
 #pragma unroll
-          for (int k = 0; k < 4; k++) {
-            const uint32_t r0 = d[0][k];
-            d[0][k] = d[1][k];
-            d[1][k] = d[2][k];
-            d[2][k] = d[3][k];
-            d[3][k] = r0;
+        for (int r = 1; r < kRows; r++) pm[r] = pm[0];
+      }
+      else {
+        box_mask_rows<kRows>(f, make_uint4(cmd, xs, 0u, meta), Y, px, pm);
+        uint32_t any = 0;
+#pragma unroll
+        for (int r = 0; r < kRows; r++) {
+          if (r >= rows) continue;
+          const uint32_t c = count(pm[r]);
+          npix += c;
+          any |= (c ? 1u : 0u) << r;
+        }
+        if (!any) continue;
+        touched |= any;
+      }
+
+      spread();
+      // Sources that are colours or texels as they lie in memory: the four
+      // rows together.
+      const uint32_t fmt = (meta >> kMetaFmt) & 3u;
+      if (kClass == kBoxFast ||
+          (!a8 && (fetch == kFetchSolid || (kClass == kBoxGeneral && pipe::fetches_rows(fetch, fmt))))) {
+        uint32_t src[kRows][4];
+#pragma unroll
+        for (int r = 0; r < kRows; r++)
+#pragma unroll
+          for (int k = 0; k < 4; k++) src[r][k] = st;
+        if (kClass == kBoxGeneral && fetch != kFetchSolid) {
+          uint32_t any = pm[0];
+#pragma unroll
+          for (int r = 1; r < kRows; r++) any |= pm[r];
+          if (any) pipe::fetch_rows<kRows>(pipe::cptr(f.styles + st), fetch, Y, px, f.images, fmt, src);
+        }
+#pragma unroll
+        for (int r = 0; r < kRows; r++) {
+          if (!((row_bits >> r) & 1u)) continue;
+          pipe::Px sp[4];
+#pragma unroll
+          for (int k = 0; k < 4; k++) sp[k] = pipe::px_of(src[r][k]);
+          if (kClass == kBoxGeneral && full && alpha == 255u && op == kOpSrcOver) {
+            pipe::src_over_full<4>(d[r], sp, fetch != kFetchSolid);
+            continue;
+          }
+          pipe::u16x2 mm[4];
+#pragma unroll
+          for (int k = 0; k < 4; k++) mm[k] = pipe::byte_pair(pm[r], k);
+          pipe::composite32_n<4>(op, d[r], sp, mm, fetch != kFetchSolid);
+        }
+        continue;
+      }
+      if constexpr (kClass != kBoxFast) {
+        // the rest a row at a time: the fetchers are long
+#pragma unroll 1
+        for (int r = ra; r < rb; r++) {
+          pipe::Px t[4];
+          uint32_t tp = 0;
+#pragma unroll
+          for (int q = 0; q < kRows; q++) {
+            if (r != q) continue;
+            tp = pm[q];
+#pragma unroll
+            for (int k = 0; k < 4; k++) t[k] = d[q][k];
+          }
+          uint32_t m[4];
+#pragma unroll
+          for (int k = 0; k < 4; k++) m[k] = (tp >> (8 * k)) & 0xFFu;
+          apply_n<4, kDither>(f, s, meta, cmd, st, a8, 0u, Y + r, px, m, t);
+#pragma unroll
+          for (int q = 0; q < kRows; q++) {
+            if (r != q) continue;
+#pragma unroll
+            for (int k = 0; k < 4; k++) d[q][k] = t[k];
           }
         }
       }
-      if (has_next) {
-        if (t < nwn) rec[cur ^ 1][t / kRecWords].w[t % kRecWords] = pw0;
-        if (t + kTileThreads < nwn) {
-          const int gw = t + kTileThreads;
-          rec[cur ^ 1][gw / kRecWords].w[gw % kRecWords] = pw1;
-        }
-      }
-      __syncthreads();
     }
   }
-
-  npix = lane_scan_add<64>(npix);
-  if (lane == 63) count_pixels(s, npix);
-
-  if (!touched) return;
+  spread();
 #pragma unroll
-  for (int g = 0; g < 4; g++)
-    if (qrow(g) < rows && qx(g) < w) store4(base + qrow(g) * stride, qx(g), w, a8, d[g]);
+  for (int r = 0; r < kRows; r++)
+    if ((touched >> r) & 1u) store_px<4, true>(base + r * stride, px, w, a8, d[r]);
+  if (lane == 0) count_pixels(s, npix);
 }
 
-// Bands whose box fills are all aligned boxes of a solid colour with
-// SRC_OVER or SRC_COPY on a 32-bit canvas -- the pure compositing load.  One
-// workgroup per group of up to 4 tiles (256 x 16 pixels); wave w takes rows
-// 4w .. 4w + 3 and lane l the pixels 4l .. 4l + 3 of each, so every load and
-// store instruction of a wave moves one contiguous 1 KB row segment.  The
-// band's commands are read 256 at a time into a compact record each (box,
-// alpha, op, colour), with no compaction or selection pass; a thread skips
-// the commands whose box misses its pixels.  Per command everything that
-// depends on the source alone is formed once, per pixel only the
-// destination terms of pipe::composite32 remain (same arithmetic, so the
-// same bits).  Few registers and records of 24 bytes let eight workgroups
-// share a CU, which is what keeps enough loads in flight.
-struct FastBoxRec {
-  int32_t x0, y0, x1, y1;   // the box (pixels, x1 / y1 exclusive)
-  uint32_t alpha_op;        // alpha | op << 8
-  uint32_t solid;           // premultiplied colour
-};
-
-__global__ __launch_bounds__(kTileThreads, 8) void k_render_box_fast(FrameDev f, FrameScratch s, uint32_t n) {
-  __shared__ FastBoxRec rec[kTileThreads];
-  const uint32_t slot = xcd_tile(blockIdx.x);
-  if (slot >= n) return;
-  // the fast groups' headers come first: 2 * slot lies inside the header
-  // buffer (two words per group of the frame) for every slot below the
-  // launch count, so the count, the header and the pool flag load together
-  const uint32_t n_groups = s.fgroup_off[f.n_bands];
-  const uint4 gh = s.group_hdr[2 * (size_t)slot];
-  const uint4 gd = s.group_hdr[2 * (size_t)slot + 1];
-  const uint32_t pool_flags = s.flags ? *s.flags : 0u;
-  if (slot >= n_groups) return;   // uniform
-  const int t = threadIdx.x;
-  const uint32_t lb = gh.y, le = gh.z;
-  const uint32_t band = gh.w >> 16;
-  const uint32_t tc0 = (gh.w & 0xFFFFu) * kGroupTiles;
-  const uint32_t ntiles = gd.w >> 24;
-  if (pool_flags) return;
-  const int lane = t & 63, row0 = (t >> 6) * 4;
-  const int X0 = (int)tc0 * kTileW;
-  const int w = X0 + (int)(gd.w & 0xFFFFu);        // canvas width
-  const int rows = (int)((gd.w >> 16) & 0x1Fu);    // rows of the band inside the canvas
-  const int px = X0 + lane * 4;
-  const int y0 = (int)band * kTileH + row0;
-  uint8_t* const base = (uint8_t*)(((uint64_t)gd.y << 32) | gd.x) - (int64_t)X0 * 4;
-  const int64_t stride = (int32_t)gd.z;
-  uint32_t d[4][4];
-#pragma unroll
-  for (int g = 0; g < 4; g++) {
-#pragma unroll
-    for (int k = 0; k < 4; k++) d[g][k] = 0u;
-    if (row0 + g < rows && px < w) load4(base + (row0 + g) * stride, px, w, false, d[g]);
-  }
-
-  uint32_t npix = 0;
-  bool touched = false;
-  for (uint32_t chunk = lb; chunk < le; chunk += kTileThreads) {
-    const uint32_t nc = le - chunk < (uint32_t)kTileThreads ? le - chunk : (uint32_t)kTileThreads;
-    __syncthreads();   // the previous chunk's records are consumed
-    if ((uint32_t)t < nc) {
-      const DevCmd& c = f.cmds[s.list_ent[chunk + t].x];
-      rec[t] = FastBoxRec{c.box[0], c.box[1], c.box[2], c.box[3], c.alpha | (c.op << 8),
-                          s.list_style[chunk + t]};
-    }
-    __syncthreads();
-    for (uint32_t k = 0; k < nc; k++) {
-      const FastBoxRec r = rec[k];
-      if (y0 + 4 <= r.y0 || y0 >= r.y1 || px + 4 <= r.x0 || px >= r.x1 || row0 >= rows) continue;
-      touched = true;
-      const uint32_t m = r.alpha_op & 0xFFu;
-      const bool over = (r.alpha_op >> 8) == kOpSrcOver;
-      const uint32_t s_rb = (r.solid & 0x00FF00FFu) * m, s_ag = ((r.solid >> 8) & 0x00FF00FFu) * m;
-      const uint32_t s1 = pipe::div255x2(s_rb) | (pipe::div255x2(s_ag) << 8);
-      const uint32_t kd = over ? (s1 >> 24) ^ 0xFFu : m ^ 0xFFu;   // destination factor
-      const uint32_t add_rb = over ? 0u : s_rb, add_ag = over ? 0u : s_ag;
-      const uint32_t add_px = over ? s1 : 0u;
-      const int bx1 = r.x1 < w ? r.x1 : w;
-#pragma unroll
-      for (int g = 0; g < 4; g++) {
-        const bool row_in = row0 + g < rows && y0 + g >= r.y0 && y0 + g < r.y1;
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-          const bool in = row_in && px + j >= r.x0 && px + j < bx1;
-          const uint32_t dv = d[g][j];
-          const uint32_t rb = pipe::div255x2((dv & 0x00FF00FFu) * kd + add_rb);
-          const uint32_t ag = pipe::div255x2(((dv >> 8) & 0x00FF00FFu) * kd + add_ag);
-          d[g][j] = in ? (rb | (ag << 8)) + add_px : dv;
-          npix += in ? 1u : 0u;
-        }
-      }
-    }
-  }
-
-  npix = lane_scan_add<64>(npix);
-  if (lane == 63) count_pixels(s, npix);
-
-  if (!touched) return;
-#pragma unroll
-  for (int g = 0; g < 4; g++)
-    if (row0 + g < rows && px < w) store4(base + (row0 + g) * stride, px, w, false, d[g]);
+__global__ __launch_bounds__(kTileThreads) void k_render_box_fast(FrameDev f, FrameScratch s, uint32_t n) {
+  render_box<kBoxFast, false>(f, s, n);
 }
 
-// Solid styles need few registers: seven workgroups per CU (72 VGPRs, no
-// spills), where the general instance fits four.  Capping it at 64 for eight
-// spills and runs slower.
-__global__ __launch_bounds__(kTileThreads, 6) void k_render_box_solid(FrameDev f, FrameScratch s, uint32_t n) {
-  render_box<true>(f, s, n);
+__global__ __launch_bounds__(kTileThreads, 3) void k_render_box_solid(FrameDev f, FrameScratch s, uint32_t n) {
+  render_box<kBoxSolid, false>(f, s, n);
 }
 
 template<bool kDither>
-__global__ __launch_bounds__(kTileThreads) void k_render_box(FrameDev f, FrameScratch s, uint32_t n) {
-  render_box<false, kDither>(f, s, n);
+__global__ __launch_bounds__(kTileThreads, 4) void k_render_box(FrameDev f, FrameScratch s, uint32_t n) {
+  render_box<kBoxGeneral, kDither>(f, s, n);
 }
 
 void launch_render(const FrameDev& f, const FrameScratch& s, uint32_t n_a, uint32_t strips, uint32_t n_f, uint32_t n_s, uint32_t n_g,

@@ -26,19 +26,11 @@ __device__ __forceinline__ uint32_t div255(uint32_t x) {
   return ((u + ((u >> 8) & 0xFFu)) >> 8) & 0xFFu;
 }
 
-__device__ __forceinline__ uint32_t ch(uint32_t p, int i) { return (p >> (i * 8)) & 0xFFu; }
-
 // div255 of two 16-bit lanes at once (bits 0-15 and 16-31, each <= 255 * 255):
 // every intermediate of a lane stays below 65536, so no carry crosses lanes.
 __device__ __forceinline__ uint32_t div255x2(uint32_t x) {
   const uint32_t u = x + 0x00800080u;
   return ((u + ((u >> 8) & 0x00FF00FFu)) >> 8) & 0x00FF00FFu;
-}
-
-// Per-lane min(v, 255) of two lanes holding values <= 510.
-__device__ __forceinline__ uint32_t sat255x2(uint32_t v) {
-  const uint32_t o = v & 0x01000100u;
-  return (v | (o - (o >> 8))) & 0x00FF00FFu;
 }
 
 // x86 cvttss2si / cvtss2si: out-of-range and NaN produce INT32_MIN.
@@ -49,90 +41,6 @@ __device__ __forceinline__ int32_t trunc_f32_to_i32(float v) {
 __device__ __forceinline__ int32_t rint_f32_to_i32(float v) {
   if (!(v >= -2147483648.0f && v < 2147483648.0f)) return INT32_MIN;
   return (int32_t)__builtin_rintf(v);
-}
-
-// Translated pattern, texel row of pattern row v (fetchgeneric_p.h:80-165):
-// pad clamps to [0, h-1]; repeat wraps by h; reflect wraps by 2h and mirrors
-// the second half.
-__device__ __forceinline__ uint32_t sp_row(const DevStyle& s, int64_t v) {
-  const int64_t h = (int64_t)s.sp_h;
-  if (s.sp_ry == 0) return (uint32_t)(v < 0 ? 0 : v > h - 1 ? h - 1 : v);
-  int64_t r = v % s.sp_ry;
-  if (r < 0) r += s.sp_ry;
-  if (r >= h) r = s.sp_ry - 1 - r;
-  return (uint32_t)r;
-}
-
-// Translated pattern, texel column of pattern column u
-// (fetchgeneric_p.h:187-352): pad clamps; a period rx (repeat: w, reflect:
-// 2w) wraps, and a wrapped position v >= w maps to rx - 1 - v.  For repeat
-// and reflect the offset is kept in [0, rx), so u >= 0 there.
-__device__ __forceinline__ uint32_t sp_col(const DevStyle& s, int64_t u) {
-  const int64_t w = (int64_t)s.sp_w;
-  if (s.sp_rx == 0) return (uint32_t)(u < 0 ? 0 : u > w - 1 ? w - 1 : u);
-  uint32_t v = (uint32_t)u % (uint32_t)s.sp_rx;
-  if (v >= (uint32_t)w) v = (uint32_t)s.sp_rx - 1u - v;
-  return v;
-}
-
-// Per (command, row) fetch state.
-struct Row {
-  uint64_t a, b;       // linear: pt at x = 0; pattern: tx, ty of the row;
-                       // gradients: the row in b (dither thresholds)
-  float f0, f1, f2;    // radial: b, d, dd;  conic: tx, ay, by
-};
-
-__device__ __forceinline__ Row row_setup(const DevStyle& s, int y, int fill_row0, uint32_t ref_band_h) {
-  Row r;
-  r.a = 0; r.b = (uint32_t)y; r.f0 = 0.f; r.f1 = 0.f; r.f2 = 0.f;
-  switch (s.kind) {
-    case kFetchLinear:
-      r.a = s.lin_pt0 + (uint64_t)(uint32_t)y * s.lin_dy;
-      break;
-    case kFetchRadial: {
-      double yd = (double)y;
-      double ptx = s.rad_yx * yd + s.rad_tx;
-      double pty = s.rad_yy * yd + s.rad_ty;
-      double b = yd * s.rad_by + s.rad_b0;
-      double sq_dist = ptx * ptx + pty * pty;
-      r.f0 = (float)(b * s.rad_inv2a);
-      r.f1 = (float)((s.rad_amul4 * (sq_dist - s.rad_sq_fr) + b * b) * s.rad_sq_inv2a);
-      r.f2 = (float)((yd * s.rad_ddy + s.rad_dd0) * s.rad_sq_inv2a);
-      break;
-    }
-    case kFetchConic: {
-      // First row of the reference fill call that covers `y`: analytic fills
-      // run per band (first band starts at the path's first row), box fills
-      // start at the box's first row.
-      int ys = fill_row0;
-      if (ref_band_h) {
-        int band_start = (y / (int)ref_band_h) * (int)ref_band_h;
-        if (band_start > ys) ys = band_start;
-      }
-      double tpx = s.con_tx + s.con_yx * (double)ys;
-      double tpy = s.con_ty + s.con_yy * (double)ys;
-      for (int k = ys; k < y; k++) { tpx += s.con_yx; tpy += s.con_yy; }
-      float ay = (float)tpy;
-      r.f0 = (float)tpx;
-      r.f2 = __builtin_signbit(ay) ? s.con_n1 : 0.0f;
-      r.f1 = __builtin_fabsf(ay);
-      break;
-    }
-    case kFetchPatternNN:
-    case kFetchPatternBI:
-      r.a = s.pa_tx + s.pa_yx * (uint64_t)(uint32_t)y;
-      r.b = s.pa_ty + s.pa_yy * (uint64_t)(uint32_t)y;
-      break;
-    case kFetchPatternAligned:
-    case kFetchPatternFxFy:
-      // texel rows of this row and of the next one (FxFy)
-      r.a = sp_row(s, (int64_t)y + s.sp_ty);
-      r.b = sp_row(s, (int64_t)y + 1 + s.sp_ty);
-      break;
-    default:
-      break;
-  }
-  return r;
 }
 
 // bayer_matrix_16x16 (tables/tables_p.h:448-469): dither thresholds of
@@ -155,39 +63,6 @@ __constant__ uint8_t kBayer16[256] = {
    42, 233,  26, 217,  38, 229,  22, 213,  41, 232,  25, 216,  37, 228,  21, 212,
   169, 106, 153,  90, 165, 102, 149,  86, 168, 105, 152,  89, 164, 101, 148,  85};
 
-// Gradient table entry `i` at pixel (x, row y): the 32-bit entry, or for a
-// dithered gradient the 64-bit one with the pixel's Bayer threshold added to
-// each colour channel before it is cut to 8 bits, limited by alpha
-// (FetchGradientBase<DITHER>::fetch_pixel, fetchgeneric_p.h:899-934).
-// kDither = false (frames without dithered gradients) leaves the dither path
-// out of the code, and its registers out of the render kernels.
-template<bool kDither>
-__device__ __forceinline__ uint32_t lut_px(const DevStyle& s, const uint32_t* __restrict__ luts, uint32_t i, int x,
-                                           uint32_t y) {
-  if (!kDither || !s.dither) return luts[s.lut + i];
-  const uint32_t lo = luts[s.lut + 2u * i], hi = luts[s.lut + 2u * i + 1u];
-  const uint32_t dd = kBayer16[((y & 15u) << 4) | ((uint32_t)x & 15u)];
-  const uint32_t a = hi >> 24;
-  uint32_t r = ((hi & 0xFFFFu) + dd) >> 8;
-  uint32_t g = ((lo >> 16) + dd) >> 8;
-  uint32_t b = ((lo & 0xFFFFu) + dd) >> 8;
-  r = r < a ? r : a;
-  g = g < a ? g : a;
-  b = b < a ? b : a;
-  return (a << 24) | (r << 16) | (g << 8) | b;
-}
-
-__device__ __forceinline__ uint32_t grad_index(uint32_t idx, const DevStyle& s) {
-  if (s.extend == 0) {
-    int32_t i = (int32_t)idx;
-    if (i < 0) i = 0;
-    if (i > (int32_t)s.maxi) i = (int32_t)s.maxi;
-    return (uint32_t)i;
-  }
-  uint32_t a = idx & s.maxi, b = a ^ s.rori;
-  return b < a ? b : a;
-}
-
 __device__ __forceinline__ uint64_t pa_norm(int32_t tw, int32_t rx, int32_t ox, uint64_t v) {
   uint32_t x = (uint32_t)((int32_t)(v >> 32) % tw);
   if ((int32_t)x < 0) x += (uint32_t)rx;
@@ -201,172 +76,11 @@ __device__ __forceinline__ int32_t pa_index(int32_t v, int32_t mn, int32_t mx, i
   return v ^ (v >> 31);
 }
 
-__device__ __forceinline__ uint32_t texel(const DevImage& im, uint32_t fmt, int32_t x, int32_t y) {
-  const uint8_t* row = (const uint8_t*)im.ptr + (int64_t)y * im.stride;
-  if (fmt == kFmtA8) return (uint32_t)row[x] * 0x01010101u;
-  uint32_t v = ((const uint32_t*)row)[x];
-  if (fmt == kFmtXRGB32) v |= 0xFF000000u;
-  return v;
-}
-
-template<bool kDither = false>
-__device__ __forceinline__ uint32_t fetch(const DevStyle& s, const Row& r, int x, const uint32_t* __restrict__ luts,
-                                          const DevImage* __restrict__ images, uint32_t src_fmt) {
-  switch (s.kind) {
-    case kFetchSolid:
-      return s.solid;
-    case kFetchLinear: {
-      uint64_t pt = r.a + (uint64_t)(uint32_t)x * s.lin_dt;
-      return lut_px<kDither>(s, luts, grad_index((uint32_t)(pt >> 32), s), x, (uint32_t)r.b);
-    }
-    case kFetchRadial: {
-      float fx = (float)x;
-      float sq_x = fx * fx;
-      float a = __builtin_sqrtf(__builtin_fabsf(sq_x * s.rad_ddd + (fx * r.f2 + r.f1)));
-      float v = (fx * s.rad_bd + r.f0) + a;
-      return lut_px<kDither>(s, luts, grad_index((uint32_t)trunc_f32_to_i32(v), s), x, (uint32_t)r.b);
-    }
-    case kFetchConic: {
-      float fx = (float)x;
-      float xv = fx * s.con_xx + r.f0;
-      float ax = __builtin_fabsf(xv);
-      float ay = r.f1;
-      float xy_min = ay < ax ? ay : ax;
-      float xy_max = ax < ay ? ay : ax;
-      float sv = (ax == xy_min) ? s.con_n4 : 0.0f;
-      float p = xy_min / xy_max;
-      float p_sq = p * p;
-      float v = p_sq * s.con_q[3] + s.con_q[2];
-      v = v * p_sq + s.con_q[1];
-      v = v * p_sq + s.con_q[0];
-      v = __builtin_fabsf(v * p - sv);
-      v = __builtin_fabsf(v - (__builtin_signbit(xv) ? s.con_n2 : 0.0f));
-      v = __builtin_fabsf(v - r.f2) + s.con_offset;
-      int32_t i = rint_f32_to_i32(v);
-      if (i > s.con_maxi) i = s.con_maxi;
-      return lut_px<kDither>(s, luts, (uint32_t)i & (uint32_t)s.con_rori, x, (uint32_t)r.b);
-    }
-    case kFetchPatternNN:
-    case kFetchPatternBI: {
-      const DevImage& im = images[s.img];
-      uint64_t px = pa_norm(s.pa_tw, s.pa_rx, s.pa_ox, r.a + s.pa_xx * (uint64_t)(uint32_t)x);
-      uint64_t py = pa_norm(s.pa_th, s.pa_ry, s.pa_oy, r.b + s.pa_xy * (uint64_t)(uint32_t)x);
-      int32_t ix = (int32_t)(px >> 32), iy = (int32_t)(py >> 32);
-      if (s.kind == kFetchPatternNN)
-        return texel(im, src_fmt, pa_index(ix, s.pa_minx, s.pa_maxx, s.pa_corx), pa_index(iy, s.pa_miny, s.pa_maxy, s.pa_cory));
-      int32_t x0 = pa_index(ix, s.pa_minx, s.pa_maxx, s.pa_corx);
-      int32_t y0 = pa_index(iy, s.pa_miny, s.pa_maxy, s.pa_cory);
-      int32_t x1 = pa_index(ix + 1, s.pa_minx, s.pa_maxx, s.pa_corx);
-      int32_t y1 = pa_index(iy + 1, s.pa_miny, s.pa_maxy, s.pa_cory);
-      uint32_t wx = (uint32_t)(px & 0xFFFFFFFFull) >> 24;
-      uint32_t wy = (uint32_t)(py & 0xFFFFFFFFull) >> 24;
-      uint32_t iw = 256 - wx, ih = 256 - wy;
-      uint32_t t00 = texel(im, src_fmt, x0, y0), t01 = texel(im, src_fmt, x0, y1);
-      uint32_t t10 = texel(im, src_fmt, x1, y0), t11 = texel(im, src_fmt, x1, y1);
-      uint32_t out = 0;
-#pragma unroll
-      for (int c = 0; c < 4; c++) {
-        uint32_t p0 = ((ch(t00, c) * ih + ch(t01, c) * wy) >> 8) & 0xFFu;
-        uint32_t p1 = ((ch(t10, c) * ih + ch(t11, c) * wy) >> 8) & 0xFFu;
-        out |= (((p0 * iw + p1 * wx) >> 8) & 0xFFu) << (c * 8);
-      }
-      return out;
-    }
-    case kFetchPatternAligned:
-      return texel(images[s.img], src_fmt, (int32_t)sp_col(s, (int64_t)x + s.sp_tx), (int32_t)r.a);
-    case kFetchPatternFxFy: {
-      // fetchgeneric_p.h:601-687: columns x0 = x + tx and x1 = x0 + 1 of rows
-      // y0, y1, weighted wa (x0 y0), wb (x1 y0), wc (x0 y1), wd (x1 y1).  The
-      // weights sum to at most 256, so each 16-bit lane of the R/B and A/G
-      // pairs stays below 65536.
-      const DevImage& im = images[s.img];
-      const int32_t x0 = (int32_t)sp_col(s, (int64_t)x + s.sp_tx), x1 = (int32_t)sp_col(s, (int64_t)x + 1 + s.sp_tx);
-      const uint32_t t00 = texel(im, src_fmt, x0, (int32_t)r.a), t01 = texel(im, src_fmt, x0, (int32_t)r.b);
-      const uint32_t t10 = texel(im, src_fmt, x1, (int32_t)r.a), t11 = texel(im, src_fmt, x1, (int32_t)r.b);
-      const uint32_t m = 0x00FF00FFu;
-      const uint32_t rb = (t00 & m) * s.sp_wa + (t01 & m) * s.sp_wc + (t10 & m) * s.sp_wb + (t11 & m) * s.sp_wd;
-      const uint32_t ag = ((t00 >> 8) & m) * s.sp_wa + ((t01 >> 8) & m) * s.sp_wc +
-                          ((t10 >> 8) & m) * s.sp_wb + ((t11 >> 8) & m) * s.sp_wd;
-      return ((rb >> 8) & m) | (ag & ~m);
-    }
-    default:
-      return 0;
-  }
-}
-
-// One PRGB32 destination pixel.
-__device__ __forceinline__ uint32_t composite32(uint32_t op, uint32_t d, uint32_t s, uint32_t m) {
-  uint32_t r = 0;
-  switch (op) {
-    // SRC_COPY, SRC_OVER and PLUS work on the R/B and A/G channel pairs
-    // (two 16-bit lanes per register); per channel the arithmetic is the
-    // scalar div255 form.
-    case kOpSrcCopy: {
-      const uint32_t im = m ^ 0xFFu;
-      const uint32_t rb = div255x2((d & 0x00FF00FFu) * im + (s & 0x00FF00FFu) * m);
-      const uint32_t ag = div255x2(((d >> 8) & 0x00FF00FFu) * im + ((s >> 8) & 0x00FF00FFu) * m);
-      return rb | (ag << 8);
-    }
-    case kOpSrcOver: {
-      const uint32_t s1 = div255x2((s & 0x00FF00FFu) * m) | (div255x2(((s >> 8) & 0x00FF00FFu) * m) << 8);
-      const uint32_t ia = (s1 >> 24) ^ 0xFFu;
-      const uint32_t t = div255x2((d & 0x00FF00FFu) * ia) | (div255x2(((d >> 8) & 0x00FF00FFu) * ia) << 8);
-      return s1 + t;
-    }
-    case kOpPlus: {
-      const uint32_t rb = sat255x2((d & 0x00FF00FFu) + div255x2((s & 0x00FF00FFu) * m));
-      const uint32_t ag = sat255x2(((d >> 8) & 0x00FF00FFu) + div255x2(((s >> 8) & 0x00FF00FFu) * m));
-      return rb | (ag << 8);
-    }
-    case kOpMultiply: {
-      uint32_t s1[4];
-#pragma unroll
-      for (int i = 0; i < 4; i++) s1[i] = div255(ch(s, i) * m);
-      uint32_t da = ch(d, 3);
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        uint32_t v = ch(d, i) * ((s1[i] + (s1[3] ^ 0xFFu)) & 0xFFFFu) + s1[i] * (da ^ 0xFFu);
-        r |= div255(v & 0xFFFFu) << (i * 8);
-      }
-      return r;
-    }
-    case kOpScreen: {
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        uint32_t s1 = div255(ch(s, i) * m);
-        r |= ((div255(ch(d, i) * (s1 ^ 0xFFu)) + s1) & 0xFFu) << (i * 8);
-      }
-      return r;
-    }
-    default:
-      return d;
-  }
-}
-
-// One A8 destination pixel; `sa` is the source alpha.
-__device__ __forceinline__ uint32_t composite8(uint32_t op, uint32_t d, uint32_t sa, uint32_t m) {
-  switch (op) {
-    case kOpSrcCopy: return div255(d * (m ^ 0xFFu) + sa * m);
-    case kOpSrcOver: {
-      uint32_t s1 = div255(sa * m);
-      return (s1 + div255(d * (s1 ^ 0xFFu))) & 0xFFu;
-    }
-    case kOpPlus: {
-      uint32_t v = d + div255(sa * m);
-      return v > 255u ? 255u : v;
-    }
-    default:
-      return d;
-  }
-}
-
-// ---------------------------------------------------------------------------
-// The render kernel's form of the same: N pixels per lane, one command for the
-// whole wave.  What a command and its style hold is uniform, so it is read
-// through the constant address space (scalar loads into SGPRs) and its
-// branches are scalar; pixels are kept as two pairs of 16-bit lanes (blue and
-// red, green and alpha) for the packed 16-bit instructions.
-// ---------------------------------------------------------------------------
+// N pixels per lane, one command for the whole wave.  What a command and its
+// style hold is uniform, so it is read through the constant address space
+// (scalar loads into SGPRs) and its branches are scalar; pixels are kept as two
+// pairs of 16-bit lanes (blue and red, green and alpha) for the packed 16-bit
+// instructions.
 
 #define B2AMD_CONST __attribute__((address_space(4)))
 template<typename T> using CPtr = const B2AMD_CONST T*;
@@ -383,6 +97,11 @@ __device__ __forceinline__ u16x2 as_pair(uint32_t v) { return __builtin_bit_cast
 __device__ __forceinline__ uint32_t as_u32(u16x2 v) { return __builtin_bit_cast(uint32_t, v); }
 __device__ __forceinline__ u16x2 both(uint32_t v) { const uint16_t h = (uint16_t)v; return u16x2{h, h}; }
 
+// Byte k of v in both lanes (k a constant).
+__device__ __forceinline__ u16x2 byte_pair(uint32_t v, int k) {
+  return as_pair(__builtin_amdgcn_perm(0u, v, 0x0C000C00u | (uint32_t)k * 0x00010001u));
+}
+
 struct Px { u16x2 rb, ag; };
 __device__ __forceinline__ Px px_of(uint32_t v) { return Px{as_pair(v & 0x00FF00FFu), as_pair((v >> 8) & 0x00FF00FFu)}; }
 __device__ __forceinline__ uint32_t px_bits(Px p) { return as_u32(p.rb) | (as_u32(p.ag) << 8); }
@@ -395,18 +114,19 @@ __device__ __forceinline__ u16x2 div255p(u16x2 x) {
   return (u + (u >> (uint16_t)8)) >> (uint16_t)8;
 }
 
-// Source pixels under masks m, onto destination pixels d: composite32 on
-// pairs.  m == 0 leaves a pixel as it is under every operator.  `carry`: the
-// source may hold a colour above its alpha (an image with any contents);
-// SRC_OVER's final sum then carries from one byte into the next as the 32-bit
-// addition of composite32 does.
+// Source pixels under masks m (the same in both lanes), onto destination
+// pixels d.  m == 0 leaves a
+// pixel as it is under every operator.  `carry`: the source may hold a colour
+// above its alpha (an image with any contents); SRC_OVER's final sum then
+// carries from one byte into the next, as the reference's addition of the
+// whole 32-bit pixel does.
 template<int N>
-__device__ __forceinline__ void composite32_n(uint32_t op, Px d[N], const Px s[N], const uint32_t m[N], bool carry) {
+__device__ __forceinline__ void composite32_n(uint32_t op, Px d[N], const Px s[N], const u16x2 m[N], bool carry) {
   switch (op) {
     case kOpSrcCopy:
 #pragma unroll
       for (int k = 0; k < N; k++) {
-        const u16x2 mm = both(m[k]), im = (uint16_t)0xFF - mm;
+        const u16x2 mm = m[k], im = (uint16_t)0xFF - mm;
         d[k].rb = div255p(d[k].rb * im + s[k].rb * mm);
         d[k].ag = div255p(d[k].ag * im + s[k].ag * mm);
       }
@@ -414,7 +134,7 @@ __device__ __forceinline__ void composite32_n(uint32_t op, Px d[N], const Px s[N
     case kOpSrcOver:
 #pragma unroll
       for (int k = 0; k < N; k++) {
-        const u16x2 mm = both(m[k]);
+        const u16x2 mm = m[k];
         const u16x2 srb = div255p(s[k].rb * mm), sag = div255p(s[k].ag * mm);
         const u16x2 ia = (uint16_t)0xFF - sag.yy;
         d[k].rb = srb + div255p(d[k].rb * ia);
@@ -428,7 +148,7 @@ __device__ __forceinline__ void composite32_n(uint32_t op, Px d[N], const Px s[N
     case kOpPlus:
 #pragma unroll
       for (int k = 0; k < N; k++) {
-        const u16x2 mm = both(m[k]), top = both(255u);
+        const u16x2 mm = m[k], top = both(255u);
         d[k].rb = __builtin_elementwise_min(d[k].rb + div255p(s[k].rb * mm), top);
         d[k].ag = __builtin_elementwise_min(d[k].ag + div255p(s[k].ag * mm), top);
       }
@@ -436,7 +156,7 @@ __device__ __forceinline__ void composite32_n(uint32_t op, Px d[N], const Px s[N
     case kOpMultiply:
 #pragma unroll
       for (int k = 0; k < N; k++) {
-        const u16x2 mm = both(m[k]);
+        const u16x2 mm = m[k];
         const u16x2 srb = div255p(s[k].rb * mm), sag = div255p(s[k].ag * mm);
         const u16x2 ia = (uint16_t)0xFF - sag.yy, ida = (uint16_t)0xFF - d[k].ag.yy;
         d[k].rb = div255p(d[k].rb * (srb + ia) + srb * ida);
@@ -446,7 +166,7 @@ __device__ __forceinline__ void composite32_n(uint32_t op, Px d[N], const Px s[N
     case kOpScreen:
 #pragma unroll
       for (int k = 0; k < N; k++) {
-        const u16x2 mm = both(m[k]);
+        const u16x2 mm = m[k];
         const u16x2 srb = div255p(s[k].rb * mm), sag = div255p(s[k].ag * mm);
         d[k].rb = div255p(d[k].rb * ((uint16_t)0xFF - srb)) + srb;
         d[k].ag = div255p(d[k].ag * ((uint16_t)0xFF - sag)) + sag;
@@ -457,11 +177,31 @@ __device__ __forceinline__ void composite32_n(uint32_t op, Px d[N], const Px s[N
   }
 }
 
+// SRC_OVER under full masks: the source needs no scaling.
+template<int N>
+__device__ __forceinline__ void src_over_full(Px d[N], const Px s[N], bool carry) {
+#pragma unroll
+  for (int k = 0; k < N; k++) {
+    const u16x2 ia = (uint16_t)0xFF - s[k].ag.yy;
+    d[k].rb = s[k].rb + div255p(d[k].rb * ia);
+    d[k].ag = s[k].ag + div255p(d[k].ag * ia);
+  }
+  if (carry) {
+#pragma unroll
+    for (int k = 0; k < N; k++) d[k] = px_of(as_u32(d[k].rb) + (as_u32(d[k].ag) << 8));
+  }
+}
+
 // A solid colour under one mask over the whole wave: everything that depends
 // on the source alone is formed once in scalar registers, per pixel only the
 // destination terms remain.  SRC_OVER and SRC_COPY.
 template<int N>
 __device__ __forceinline__ void composite32_flat(uint32_t op, Px d[N], uint32_t color, uint32_t m) {
+  if (m == 255u && (op == kOpSrcCopy || (color >> 24) == 255u)) {   // the colour itself
+#pragma unroll
+    for (int k = 0; k < N; k++) d[k] = px_of(color);
+    return;
+  }
   const uint32_t s_rb = (color & 0x00FF00FFu) * m, s_ag = ((color >> 8) & 0x00FF00FFu) * m;
   if (op == kOpSrcOver) {
     const uint32_t s1_rb = div255x2(s_rb), s1_ag = div255x2(s_ag);
@@ -482,7 +222,7 @@ __device__ __forceinline__ void composite32_flat(uint32_t op, Px d[N], uint32_t 
   }
 }
 
-// composite8 on pairs of neighbouring A8 pixels.
+// The same on pairs of neighbouring A8 pixels; sa: source alpha.
 template<int P>
 __device__ __forceinline__ void composite8_n(uint32_t op, u16x2 d[P], const u16x2 sa[P], const u16x2 m[P]) {
   switch (op) {
@@ -570,10 +310,15 @@ __device__ __forceinline__ void pa_walk(uint64_t v, uint64_t step, int32_t tw, i
 // N consecutive words at a 4-byte aligned address.
 template<int N>
 __device__ __forceinline__ void wide_load(const B2AMD_GLOBAL uint32_t* p, uint32_t out[N]) {
-  typedef uint32_t words __attribute__((ext_vector_type(N == 1 ? 2 : N), aligned(4)));
-  const words v = *(const B2AMD_GLOBAL words*)p;
+  if constexpr (N == 1) {
+    out[0] = *p;
+  }
+  else {
+    typedef uint32_t words __attribute__((ext_vector_type(N), aligned(4)));
+    const words v = *(const B2AMD_GLOBAL words*)p;
 #pragma unroll
-  for (int k = 0; k < N; k++) out[k] = v[k];
+    for (int k = 0; k < N; k++) out[k] = v[k];
+  }
 }
 
 __device__ __forceinline__ uint32_t texel_at(GBytes row, uint32_t fmt, uint32_t x) {
@@ -591,6 +336,126 @@ __device__ __forceinline__ uint32_t blend4(uint32_t t00, uint32_t t01, uint32_t 
   const u16x2 rb = (((a.rb * y0 + b.rb * y1) >> sh) * x0 + ((c.rb * y0 + e.rb * y1) >> sh) * x1) >> sh;
   const u16x2 ag = (((a.ag * y0 + b.ag * y1) >> sh) * x0 + ((c.ag * y0 + e.ag * y1) >> sh) * x1) >> sh;
   return px_bits(Px{rb, ag});
+}
+
+// Translated pattern: the texels of pixels px .. px + N - 1 from a row.
+// Neighbours by one wide load (4-byte aligned); lanes whose pixels meet an edge
+// of the image take them one by one.  Steps between texels are at most one up,
+// so the ends being N - 1 apart means that all lie in a line.
+template<int N>
+__device__ __forceinline__ void aligned_texels(GBytes row, uint32_t fmt, int px, int32_t tx, int32_t rx, int32_t w, float inv_x,
+                                               uint32_t out[N]) {
+  const uint32_t x0 = sp_wrap(px, tx, rx, w, inv_x), xl = sp_wrap(px + N - 1, tx, rx, w, inv_x);
+  if (N > 1 && fmt != kFmtA8 && xl == x0 + (uint32_t)(N - 1)) {
+    wide_load<N>((const B2AMD_GLOBAL uint32_t*)row + x0, out);
+    if (fmt == kFmtXRGB32) {
+#pragma unroll
+      for (int k = 0; k < N; k++) out[k] |= 0xFF000000u;
+    }
+    return;
+  }
+  out[0] = texel_at(row, fmt, x0);
+#pragma unroll
+  for (int k = 1; k < N; k++) out[k] = texel_at(row, fmt, k == N - 1 ? xl : sp_wrap(px + k, tx, rx, w, inv_x));
+}
+
+// The texels of pixels px .. px + N from two rows, the same way.
+template<int N>
+__device__ __forceinline__ void neighbour_texels(GBytes row0, GBytes row1, uint32_t fmt, int px, int32_t tx, int32_t rx,
+                                                 int32_t w, float inv_x, uint32_t a[N + 1], uint32_t b[N + 1]) {
+  const uint32_t x0 = sp_wrap(px, tx, rx, w, inv_x), xn = sp_wrap(px + N, tx, rx, w, inv_x);
+  if (fmt == kFmtPRGB32 && xn == x0 + (uint32_t)N) {
+    const B2AMD_GLOBAL uint32_t* const pa = (const B2AMD_GLOBAL uint32_t*)row0 + x0;
+    const B2AMD_GLOBAL uint32_t* const pb = (const B2AMD_GLOBAL uint32_t*)row1 + x0;
+    wide_load<N>(pa, a);
+    wide_load<N>(pb, b);
+    a[N] = pa[N];
+    b[N] = pb[N];
+    return;
+  }
+#pragma unroll
+  for (int k = 0; k <= N; k++) {
+    const uint32_t x = k == 0 ? x0 : k == N ? xn : sp_wrap(px + k, tx, rx, w, inv_x);
+    a[k] = texel_at(row0, fmt, x);
+    b[k] = texel_at(row1, fmt, x);
+  }
+}
+
+// fetchgeneric_p.h:601-687: four texels under weights that sum to at most 256.
+__device__ __forceinline__ uint32_t weigh4(uint32_t t00, uint32_t t10, uint32_t t01, uint32_t t11, u16x2 wa, u16x2 wb, u16x2 wc,
+                                           u16x2 wd) {
+  const Px a = px_of(t00), b = px_of(t10), c = px_of(t01), e = px_of(t11);
+  const u16x2 rb = a.rb * wa + c.rb * wc + b.rb * wb + e.rb * wd;
+  const u16x2 ag = a.ag * wa + c.ag * wc + b.ag * wb + e.ag * wd;
+  return px_bits(Px{rb >> (uint16_t)8, ag >> (uint16_t)8});
+}
+
+// Styles that fetch_rows takes: translated patterns of 32-bit pixels.
+__device__ __forceinline__ bool fetches_rows(uint32_t kind, uint32_t fmt) {
+  return kind == kFetchPatternAligned ? fmt != kFmtA8 : kind == kFetchPatternFxFy && fmt == kFmtPRGB32;
+}
+
+// fetch_n of four pixels in each of R rows from y on (uniform): all rows' loads
+// are in flight together, and with a fractional offset each texel row is read
+// once.
+template<int R>
+__device__ __forceinline__ void fetch_rows(CPtr<DevStyle> s, uint32_t kind, int y, int px, const DevImage* images, uint32_t fmt,
+                                           uint32_t out[R][4]) {
+  const CPtr<DevImage> im = cptr(images + s->img);
+  const GBytes base = global_bytes(im->ptr);
+  const int64_t stride = im->stride;
+  const int32_t w = s->sp_w, h = s->sp_h, rx = s->sp_rx, ry = s->sp_ry, tx = s->sp_tx, ty = s->sp_ty;
+  const float inv_y = ry ? __builtin_amdgcn_rcpf((float)ry) : 0.0f, inv_x = rx ? __builtin_amdgcn_rcpf((float)rx) : 0.0f;
+  const uint32_t x0 = sp_wrap(px, tx, rx, w, inv_x);
+  if (kind == kFetchPatternAligned) {
+    const bool line = sp_wrap(px + 3, tx, rx, w, inv_x) == x0 + 3u;
+    if (line) {
+#pragma unroll
+      for (int r = 0; r < R; r++)
+        wide_load<4>((const B2AMD_GLOBAL uint32_t*)(base + (int64_t)sp_wrap(y + r, ty, ry, h, inv_y) * stride) + x0, out[r]);
+    }
+    else {
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        const uint32_t x = sp_wrap(px + k, tx, rx, w, inv_x);
+#pragma unroll
+        for (int r = 0; r < R; r++)
+          out[r][k] = ((const B2AMD_GLOBAL uint32_t*)(base + (int64_t)sp_wrap(y + r, ty, ry, h, inv_y) * stride))[x];
+      }
+    }
+    if (fmt == kFmtXRGB32) {
+#pragma unroll
+      for (int r = 0; r < R; r++)
+#pragma unroll
+        for (int k = 0; k < 4; k++) out[r][k] |= 0xFF000000u;
+    }
+    return;
+  }
+  uint32_t t[R + 1][5];
+  const bool line = sp_wrap(px + 4, tx, rx, w, inv_x) == x0 + 4u;
+  if (line) {
+#pragma unroll
+    for (int r = 0; r <= R; r++) {
+      const B2AMD_GLOBAL uint32_t* const row =
+        (const B2AMD_GLOBAL uint32_t*)(base + (int64_t)sp_wrap(y + r, ty, ry, h, inv_y) * stride) + x0;
+      wide_load<4>(row, t[r]);
+      t[r][4] = row[4];
+    }
+  }
+  else {
+#pragma unroll
+    for (int k = 0; k <= 4; k++) {
+      const uint32_t x = sp_wrap(px + k, tx, rx, w, inv_x);
+#pragma unroll
+      for (int r = 0; r <= R; r++)
+        t[r][k] = ((const B2AMD_GLOBAL uint32_t*)(base + (int64_t)sp_wrap(y + r, ty, ry, h, inv_y) * stride))[x];
+    }
+  }
+  const u16x2 wa = both(s->sp_wa), wb = both(s->sp_wb), wc = both(s->sp_wc), wd = both(s->sp_wd);
+#pragma unroll
+  for (int r = 0; r < R; r++)
+#pragma unroll
+    for (int k = 0; k < 4; k++) out[r][k] = weigh4(t[r][k], t[r][k + 1], t[r + 1][k], t[r + 1][k + 1], wa, wb, wc, wd);
 }
 
 // The source pixels px .. px + N - 1 of row y (per lane) of a non-solid style
@@ -710,43 +575,17 @@ __device__ __forceinline__ void fetch_n(CPtr<DevStyle> s, uint32_t kind, int y, 
     const float inv_y = ry ? __builtin_amdgcn_rcpf((float)ry) : 0.0f, inv_x = rx ? __builtin_amdgcn_rcpf((float)rx) : 0.0f;
     const GBytes row0 = base + (int64_t)sp_wrap(y, ty, ry, h, inv_y) * stride;
     if (kind == kFetchPatternAligned) {
-      const uint32_t x0 = sp_wrap(px, tx, rx, w, inv_x), x3 = sp_wrap(px + N - 1, tx, rx, w, inv_x);
-      if (fmt != kFmtA8 && N > 1) {
-        // N neighbouring texels: one wide load (4-byte aligned)
-        const bool run = x3 == x0 + (uint32_t)(N - 1);
-        if (__ballot(!run) == 0ull) {
-          wide_load<N>((const B2AMD_GLOBAL uint32_t*)row0 + x0, out);
-          if (fmt == kFmtXRGB32) {
-#pragma unroll
-            for (int k = 0; k < N; k++) out[k] |= 0xFF000000u;
-          }
-          return;
-        }
-      }
-      out[0] = texel_at(row0, fmt, x0);
-#pragma unroll
-      for (int k = 1; k < N; k++) out[k] = texel_at(row0, fmt, k == N - 1 ? x3 : sp_wrap(px + k, tx, rx, w, inv_x));
+      aligned_texels<N>(row0, fmt, px, tx, rx, w, inv_x, out);
       return;
     }
-    // fetchgeneric_p.h:601-687: columns x0 = x + tx and x1 = x0 + 1 of rows
-    // y0, y1, weighted wa (x0 y0), wb (x1 y0), wc (x0 y1), wd (x1 y1), which
-    // sum to at most 256
+    // columns x + tx and the next of rows y + ty and the next, weighted wa
+    // (x0 y0), wb (x1 y0), wc (x0 y1), wd (x1 y1)
     const GBytes row1 = base + (int64_t)sp_wrap(y + 1, ty, ry, h, inv_y) * stride;
     uint32_t a[N + 1], b[N + 1];
-#pragma unroll
-    for (int k = 0; k <= N; k++) {
-      const uint32_t x = sp_wrap(px + k, tx, rx, w, inv_x);
-      a[k] = texel_at(row0, fmt, x);
-      b[k] = texel_at(row1, fmt, x);
-    }
+    neighbour_texels<N>(row0, row1, fmt, px, tx, rx, w, inv_x, a, b);
     const u16x2 wa = both(s->sp_wa), wb = both(s->sp_wb), wc = both(s->sp_wc), wd = both(s->sp_wd);
 #pragma unroll
-    for (int k = 0; k < N; k++) {
-      const Px t00 = px_of(a[k]), t01 = px_of(b[k]), t10 = px_of(a[k + 1]), t11 = px_of(b[k + 1]);
-      const u16x2 rb = t00.rb * wa + t01.rb * wc + t10.rb * wb + t11.rb * wd;
-      const u16x2 ag = t00.ag * wa + t01.ag * wc + t10.ag * wb + t11.ag * wd;
-      out[k] = px_bits(Px{rb >> (uint16_t)8, ag >> (uint16_t)8});
-    }
+    for (int k = 0; k < N; k++) out[k] = weigh4(a[k], a[k + 1], b[k], b[k + 1], wa, wb, wc, wd);
     return;
   }
 
@@ -766,16 +605,53 @@ __device__ __forceinline__ void fetch_n(CPtr<DevStyle> s, uint32_t kind, int y, 
     return;
   }
   uint32_t t00[N], t01[N], t10[N], t11[N];
+  uint32_t x0[N], x1[N];
+  bool apart = fmt == kFmtA8 || im->w < 2u;
 #pragma unroll
   for (int k = 0; k < N; k++) {
-    const int32_t ix = (int32_t)(ux[k] >> 32), iy = (int32_t)(uy[k] >> 32);
-    const uint32_t x0 = (uint32_t)pa_index(ix, minx, maxx, corx), x1 = (uint32_t)pa_index(ix + 1, minx, maxx, corx);
-    const GBytes r0 = base + (int64_t)pa_index(iy, miny, maxy, cory) * stride;
-    const GBytes r1 = base + (int64_t)pa_index(iy + 1, miny, maxy, cory) * stride;
-    t00[k] = texel_at(r0, fmt, x0);
-    t01[k] = texel_at(r1, fmt, x0);
-    t10[k] = texel_at(r0, fmt, x1);
-    t11[k] = texel_at(r1, fmt, x1);
+    const int32_t ix = (int32_t)(ux[k] >> 32);
+    x0[k] = (uint32_t)pa_index(ix, minx, maxx, corx);
+    x1[k] = (uint32_t)pa_index(ix + 1, minx, maxx, corx);
+    apart |= x0[k] - x1[k] + 1u > 2u;
+  }
+  if (__ballot(apart) == 0ull) {
+    // the two texels of a row are neighbours or the same one: an 8-byte load
+    // holds both (half the loads; the pair at the row's end starts a texel
+    // before it)
+    const uint32_t last = im->w - 2u;
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+      const int32_t iy = (int32_t)(uy[k] >> 32);
+      const uint32_t xl = min(min(x0[k], x1[k]), last);
+      uint32_t a[2], b[2];
+      wide_load<2>((const B2AMD_GLOBAL uint32_t*)(base + (int64_t)pa_index(iy, miny, maxy, cory) * stride) + xl, a);
+      wide_load<2>((const B2AMD_GLOBAL uint32_t*)(base + (int64_t)pa_index(iy + 1, miny, maxy, cory) * stride) + xl, b);
+      t00[k] = x0[k] == xl ? a[0] : a[1];
+      t10[k] = x1[k] == xl ? a[0] : a[1];
+      t01[k] = x0[k] == xl ? b[0] : b[1];
+      t11[k] = x1[k] == xl ? b[0] : b[1];
+    }
+    if (fmt == kFmtXRGB32) {
+#pragma unroll
+      for (int k = 0; k < N; k++) {
+        t00[k] |= 0xFF000000u;
+        t01[k] |= 0xFF000000u;
+        t10[k] |= 0xFF000000u;
+        t11[k] |= 0xFF000000u;
+      }
+    }
+  }
+  else {
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+      const int32_t iy = (int32_t)(uy[k] >> 32);
+      const GBytes r0 = base + (int64_t)pa_index(iy, miny, maxy, cory) * stride;
+      const GBytes r1 = base + (int64_t)pa_index(iy + 1, miny, maxy, cory) * stride;
+      t00[k] = texel_at(r0, fmt, x0[k]);
+      t01[k] = texel_at(r1, fmt, x0[k]);
+      t10[k] = texel_at(r0, fmt, x1[k]);
+      t11[k] = texel_at(r1, fmt, x1[k]);
+    }
   }
 #pragma unroll
   for (int k = 0; k < N; k++) out[k] = blend4(t00[k], t01[k], t10[k], t11[k], (uint32_t)ux[k] >> 24, (uint32_t)uy[k] >> 24);
