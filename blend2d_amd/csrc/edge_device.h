@@ -255,6 +255,12 @@ struct Builder {
   }
   __device__ __forceinline__ static bool flat_enough(const Mono& m, double tol_sq) {
     double value, limit;
+    flatness(m, tol_sq, value, limit);
+    return value <= limit;
+  }
+  // Squared distance of the control points from the chord, and the most that
+  // counts as flat (both times the chord's squared length).
+  __device__ __forceinline__ static void flatness(const Mono& m, double tol_sq, double& value, double& limit) {
     if (m.n == 3) {
       P v1 = psub(m.p[1], m.p[0]);
       P v2 = psub(m.p[2], m.p[0]);
@@ -269,7 +275,6 @@ struct Builder {
       value = dmax(c1 * c1, c2 * c2);
       limit = tol_sq * mag_sq(v);
     }
-    return value <= limit;
   }
   __device__ __forceinline__ static void msplit(const Mono& m, Step& s) {
     if (m.n == 3) {

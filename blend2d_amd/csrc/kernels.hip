@@ -355,14 +355,31 @@ __device__ __forceinline__ void fold_bounds(CmdBounds* __restrict__ bounds, uint
 // Measured against splitting, counting and writing in passes of their own
 // (clip list included): 1024 glyph canvases, 5.1 million quads into 18.3
 // million segments, 3.12 -> 1.18 ms; 10 000 cubic paths, 2.8 million segments,
-// 0.82 -> 0.58.  Few long curves are a serial chain either way (32 uneven
-// canvases 0.58 -> 0.65).
+// 0.82 -> 0.58.
+//
+// Few long curves would leave most of a wave's lanes without work and be one
+// serial chain each.  Once a wave has no sources left, a lane that halves its
+// root (the piece, or what is left of it when nothing waits above the node in
+// hand) keeps the first half and hands the other to a waiting lane: the nodes
+// and their points are the same whichever lane gets to them, and the order of
+// segments doesn't matter.  With it, clip list not included: 32 uneven canvases
+// 380 -> 100 us, 10 000 cubic paths 418 -> 213, 2000 pattern shapes 65 -> 29,
+// a frame of panels 64 -> 27.
 constexpr uint32_t kLaneStage = 4;
 constexpr uint32_t kMaxLevel = 31;
+// A root is shared from this bend on (squared distance of its control points
+// from the chord over the squared tolerance; a split divides it by 16): each
+// half then needs a split of its own.  k_edges in us at 1 (any split one) / 16 /
+// 64 / 256 / 4096 / never: 10 000 cubic paths 312 / 213 / 233 / 239 / 310 / 418,
+// uneven canvases 117 / 100 / 117 / 121 / 168 / 380, panels 27 / 27 / 31 / 31 /
+// 40 / 64, glyph canvases (three segments a quad) 1258 / 881 / 875 / 872 / 875 /
+// 874.
+constexpr double kShareBend = 16.0;
 struct EdgeWave {
   DevSeg seg[kLaneStage][64];
   double cv[8][64];    // each lane's source curve, transformed (x, y)
   double cut[8][64];   // parameters it is cut at, then 1
+  uint32_t giver[64];  // lanes that hand half of their node over
 };
 
 __global__ __launch_bounds__(256) void k_edges(FrameDev f, FrameScratch s, uint32_t batch) {
@@ -610,9 +627,13 @@ __global__ __launch_bounds__(256) void k_edges(FrameDev f, FrameScratch s, uint3
         if (!busy) break;
         if (__popcll(busy) < 40 && (next < end || __ballot(mode == kPiece) != 0ull)) break;
         if (__ballot(staged == kLaneStage)) flush();
+        bool halved = false;   // the lane's root: `m` and `top` are all there is of it
         if (mode == kFlat) {
-          if (level != kMaxLevel && !B::flat_enough(m, f.tol_sq)) {
+          double bend, limit;
+          B::flatness(m, f.tol_sq, bend, limit);
+          if (level != kMaxLevel && !(bend <= limit)) {
             B::halves(m, top);
+            halved = level == 0 && bend > kShareBend * limit;
             level++;
             path <<= 1;
           }
@@ -643,6 +664,51 @@ __global__ __launch_bounds__(256) void k_edges(FrameDev f, FrameScratch s, uint3
                   }
                 }
               }
+              if (path == (1u << level) - 1u) {   // nothing waits above it: a root of its own
+#pragma unroll
+                for (int i = 0; i < 4; i++) root.p[i] = m.p[i];
+                level = path = 0;
+              }
+            }
+          }
+        }
+        // No sources left: lanes that have just halved their root keep the
+        // first half as theirs and hand the other to lanes that wait.
+        if (next >= end) {
+          const uint64_t give = __ballot(halved), idle = __ballot(mode == kIdle);
+          if (give && idle) {
+            const uint32_t n = min((uint32_t)__popcll(give), (uint32_t)__popcll(idle));
+            const bool gives = halved && (uint32_t)__popcll(give & below) < n;
+            const uint32_t rank = (uint32_t)__popcll(idle & below);
+            const bool takes = mode == kIdle && rank < n;
+            if (gives) ws.giver[__popcll(give & below)] = lane;
+            wave_sync();
+            const int from = takes ? (int)ws.giver[rank] : (int)lane;
+            wave_sync();
+            const uint32_t cmd = (uint32_t)__shfl((int)bd.cmd, from, 64);
+            const uint32_t how = (uint32_t)__shfl((int)(sign | (uint32_t)root.n << 1), from, 64);
+            const bool other = takes && cmd != bd.cmd;
+            if (__ballot(other && staged)) flush();
+            const uint64_t fold = __ballot(other && bd.cmd != 0xFFFFFFFFu);
+            if (fold) fold_bounds(s.bounds, fold, bd);
+            if (other) bd.reset(cmd);
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+              const double x = __shfl(top[i].x, from, 64), y = __shfl(top[i].y, from, 64);
+              if (takes) m.p[i] = edge::P{x, y};
+            }
+            if (takes) {
+              sign = how & 1u;
+              root.n = m.n = (int)(how >> 1);
+              ax = edge::trunc_i(m.p[0].x);
+              ay = edge::trunc_i(m.p[0].y);
+              cut_i = n_cuts = 0;
+              mode = kFlat;
+            }
+            if (takes || gives) {
+#pragma unroll
+              for (int i = 0; i < 4; i++) root.p[i] = m.p[i];
+              level = path = 0;
             }
           }
         }

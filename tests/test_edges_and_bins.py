@@ -93,3 +93,25 @@ def test_many_segments_in_one_frame(amd):
     for k in (7, 100):
         want, _ = checkers.render_oracle(scenes[k])
         assert np.array_equal(outs[k], want)
+
+
+# fewer curves than lanes, each a command of its own, from a few pixels to the
+# whole canvas: halves of long ones go to lanes that held another command; and
+# more curves than lanes, the last ones long
+@pytest.mark.parametrize("count", [1, 2, 7, 8, 9, 33, 150])
+@pytest.mark.parametrize("kind", ["quad", "cubic", "mixed"])
+def test_few_curves(amd, count, kind):
+    rng = np.random.default_rng(count)
+    sc = S.Scene(1300, 900, S.FMT_A8, 0)
+    for k in range(count):
+        size = np.array([1300.0, 900.0]) * (0.01 if k % 3 == 1 else 0.12 if k % 3 == 2 else 1.0) * 0.98
+        base = (np.array([1300.0, 900.0]) - size) * (0.02 + 0.96 * rng.random(2))
+        pts = base + rng.random((6, 2)) * size
+        quad = kind == "quad" or (kind == "mixed" and k & 1)
+        sc.set_fill_rule(k & 1)
+        sc.set_fill_style_rgba32(0x60FFFFFF)
+        if quad:
+            sc.fill_path([S.CMD_MOVE, S.CMD_QUAD, S.CMD_ON, S.CMD_QUAD, S.CMD_ON, S.CMD_CLOSE], np.vstack([pts[:5], pts[:1]]))
+        else:
+            sc.fill_path([S.CMD_MOVE, S.CMD_CUBIC, S.CMD_CUBIC, S.CMD_ON, S.CMD_CLOSE], np.vstack([pts[:4], pts[:1]]))
+    _cmp(amd, sc)
