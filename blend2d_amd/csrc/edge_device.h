@@ -294,14 +294,17 @@ struct Builder {
   // Splits `m`: it becomes its left half, `right` receives the other (a quad's
   // end point in both of the last two places).
   __device__ __forceinline__ static void halves(Mono& m, P right[4]) {
-    const P p01 = pmid(m.p[0], m.p[1]), p12 = pmid(m.p[1], m.p[2]), p012 = pmid(p01, p12);
+    // (points are read first and unconditionally: a choice between two places
+    // of `m` would keep it in memory)
+    const P p2{m.p[2].x, m.p[2].y}, p3{m.p[3].x, m.p[3].y};
+    const P p01 = pmid(m.p[0], m.p[1]), p12 = pmid(m.p[1], p2), p012 = pmid(p01, p12);
     if (m.n == 3) {
-      right[0] = p012; right[1] = p12; right[2] = m.p[2]; right[3] = m.p[2];
+      right[0] = p012; right[1] = p12; right[2] = p2; right[3] = p2;
       m.p[1] = p01; m.p[2] = p012; m.p[3] = p012;
     }
     else {
-      const P p23 = pmid(m.p[2], m.p[3]), p123 = pmid(p12, p23), p0123 = pmid(p012, p123);
-      right[0] = p0123; right[1] = p123; right[2] = p23; right[3] = m.p[3];
+      const P p23 = pmid(p2, p3), p123 = pmid(p12, p23), p0123 = pmid(p012, p123);
+      right[0] = p0123; right[1] = p123; right[2] = p23; right[3] = p3;
       m.p[1] = p01; m.p[2] = p012; m.p[3] = p0123;
     }
   }
@@ -326,6 +329,26 @@ struct Builder {
     m.sp--;
     const P* st = stack + m.sp * 4;
     for (int i = 0; i < m.n; i++) m.p[i] = st[i];
+  }
+
+  // A node strictly inside the clip box that takes several splits: nothing
+  // below it meets the clipper, so another lane may flatten it.  (Deep in the
+  // stack the subdivision limit could come into it.)
+  __device__ __forceinline__ bool give(const Mono& m, uint32_t sign) {
+    double bend, limit;
+    flatness(m, tol_sq, bend, limit);
+    if (m.sp > 16 || !(bend > 16.0 * limit)) return false;
+    uint32_t any = 0;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const P q = i == 3 ? mlast(m) : m.p[i];
+      any |= (uint32_t)!(q.x > c.x0) | (uint32_t)!(q.x < c.x1) | (uint32_t)!(q.y > c.y0) | (uint32_t)!(q.y < c.y1);
+    }
+    if (any || !out.give(m.p, m.n, sign)) return false;
+    const P l = mlast(m);
+    ax = trunc_i(l.x);
+    ay = trunc_i(l.y);
+    return true;
   }
 
   __device__ void flatten_safe(Mono& m, const P* src, uint32_t sign, P* stack) {
@@ -424,6 +447,11 @@ LTR_BeforeX0_Pop:
           open_at(mfirst(m).x, mfirst(m).y);
           for (;;) {
             if (!is_flat(m)) {
+              if (give(m, sign)) {
+                if (m.sp == 0) break;
+                mpop(m, stack);
+                continue;
+              }
               msplit(m, s);
               if (m.sp != kLimit) { mpush(m, s, stack); continue; }
             }
@@ -515,6 +543,11 @@ RTL_AfterX1_Pop:
           open_at(mfirst(m).x, mfirst(m).y);
           for (;;) {
             if (!is_flat(m)) {
+              if (give(m, sign)) {
+                if (m.sp == 0) break;
+                mpop(m, stack);
+                continue;
+              }
               msplit(m, s);
               if (m.sp != kLimit) { mpush(m, s, stack); continue; }
             }

@@ -226,10 +226,16 @@ struct LaneBounds {
 // Segments of one wave of k_edges_clip on their way out: staged in LDS and
 // written to the wave's region of the segment buffer with coalesced stores,
 // one atomic on the region's cursor per flush.
-constexpr uint32_t kEdgeStage = 1024;
+constexpr uint32_t kEdgeStage = 512;
+// Parts of curves that lie inside the clip box, found by lanes in their walk
+// across it: the whole wave flattens them afterwards.
+constexpr uint32_t kInnerList = 64;
 struct EdgeStage {
   DevSeg seg[kEdgeStage];
   uint32_t cmd[kEdgeStage];
+  double inner[8][kInnerList];         // the four points (x, y)
+  uint32_t inner_cmd[kInnerList];
+  uint32_t inner_how[kInnerList];      // sign | points << 1
 };
 struct EdgeOut {
   EdgeStage& stage;
@@ -266,8 +272,22 @@ struct EdgeOut {
 // once the stage is full.
 struct ClipEmit {
   EdgeOut& out;
-  uint32_t* count;
+  uint32_t* count;   // of staged segments, then of inner parts
   LaneBounds& bd;
+  __device__ __forceinline__ bool give(const edge::P* p, int n, uint32_t sign) {
+    const uint32_t at = atomicAdd(count + 1, 1u);
+    if (at >= kInnerList) return false;
+    EdgeStage& st = out.stage;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const edge::P q = p[i == 3 ? n - 1 : i];
+      st.inner[2 * i][at] = q.x;
+      st.inner[2 * i + 1][at] = q.y;
+    }
+    st.inner_cmd[at] = bd.cmd;
+    st.inner_how[at] = sign | (uint32_t)n << 1;
+    return true;
+  }
   __device__ __forceinline__ void push(int32_t x0, int32_t y0, int32_t x1, int32_t y1, uint32_t sign) {
     const DevSeg g{x0, y0, (int32_t)((uint32_t)x1 | (sign << 31)), y1};
     bd.add(x0, y0, x1, y1);
@@ -319,6 +339,121 @@ __device__ __forceinline__ void fold_bounds(CmdBounds* __restrict__ bounds, uint
   }
 }
 
+constexpr uint32_t kMaxLevel = 31;
+// A root is shared from this bend on (squared distance of its control points
+// from the chord over the squared tolerance; a split divides it by 16): each
+// half then needs a split of its own.  k_edges in us at 1 (any split one) / 16 /
+// 64 / 256 / 4096 / never: 10 000 cubic paths 312 / 213 / 233 / 239 / 310 / 418,
+// uneven canvases 117 / 100 / 117 / 121 / 168 / 380, panels 27 / 27 / 31 / 31 /
+// 40 / 64, glyph canvases (three segments a quad) 1258 / 881 / 875 / 872 / 875 /
+// 874.
+constexpr double kShareBend = 16.0;
+
+// One lane's curve in the flattening: a monotonic piece inside the clip box
+// (the root), and the node of it in hand.
+template<typename B>
+struct CurveWalk {
+  typename B::Mono root, m;
+  edge::P top[4];              // right half of the last split
+  uint32_t level, path;        // of the node in hand
+  int32_t ax, ay;              // last point of the chain
+  uint32_t sign;
+
+  __device__ __forceinline__ void start(const edge::P p[4], int n, uint32_t sg) {
+    root.n = m.n = n;
+#pragma unroll
+    for (int i = 0; i < 4; i++) root.p[i] = m.p[i] = p[i];
+    level = path = 0;
+    sign = sg;
+    ax = edge::trunc_i(p[0].x);
+    ay = edge::trunc_i(p[0].y);
+  }
+  // Splits the node in hand, or emits it and goes on to the next.  False when
+  // that was the last; `halved`: the root was split and is worth sharing (`m`
+  // and `top` are all there is of it).
+  template<typename Put>
+  __device__ __forceinline__ bool step(double tol_sq, bool& halved, Put&& put) {
+    double bend, limit;
+    B::flatness(m, tol_sq, bend, limit);
+    if (level != kMaxLevel && !(bend <= limit)) {
+      B::halves(m, top);
+      halved = level == 0 && bend > kShareBend * limit;
+      level++;
+      path <<= 1;
+      return true;
+    }
+    const edge::P l = m.p[3];   // (a quad's last point too)
+    const int32_t nx = edge::trunc_i(l.x), ny = edge::trunc_i(l.y);
+    if (ay != ny) put(ax, ay, nx, ny, sign);
+    ax = nx;
+    ay = ny;
+    // the next node: up while it was a right half, then the right half beside
+    // it
+    const uint32_t ups = (uint32_t)__builtin_ctz(~path);
+    if (ups >= level) return false;
+    level -= ups;
+    path = (path >> ups) + 1u;
+#pragma unroll
+    for (int i = 0; i < 4; i++) m.p[i] = top[i];
+    if (ups) {
+#pragma unroll
+      for (int i = 0; i < 4; i++) m.p[i] = root.p[i];
+      for (uint32_t k = level; k-- > 0;) {
+        edge::P r[4];
+        B::halves(m, r);
+        if ((path >> k) & 1u) {
+#pragma unroll
+          for (int i = 0; i < 4; i++) m.p[i] = r[i];
+        }
+      }
+    }
+    if (path == (1u << level) - 1u) {   // nothing waits above it: a root of its own
+#pragma unroll
+      for (int i = 0; i < 4; i++) root.p[i] = m.p[i];
+      level = path = 0;
+    }
+    return true;
+  }
+};
+
+// Lanes that have just halved their root keep the first half as theirs and
+// hand the other to lanes that wait (all lanes call it).  True for a lane that
+// got one, its bounds being those of the curve's command then; before(other)
+// is called by all lanes, `other` where a lane changes its command.
+template<typename B, typename Before>
+__device__ __forceinline__ bool share_halves(CurveWalk<B>& w, uint32_t* giver, bool halved, bool waits, LaneBounds& bd,
+                                             CmdBounds* bounds, Before&& before) {
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint64_t below = (1ull << lane) - 1ull;
+  const uint64_t give = __ballot(halved), idle = __ballot(waits);
+  if (!give || !idle) return false;
+  const uint32_t n = min((uint32_t)__popcll(give), (uint32_t)__popcll(idle));
+  const bool gives = halved && (uint32_t)__popcll(give & below) < n;
+  const uint32_t rank = (uint32_t)__popcll(idle & below);
+  const bool takes = waits && rank < n;
+  if (gives) giver[__popcll(give & below)] = lane;
+  wave_sync();
+  const int from = takes ? (int)giver[rank] : (int)lane;
+  wave_sync();
+  const uint32_t cmd = (uint32_t)__shfl((int)bd.cmd, from, 64);
+  const uint32_t how = (uint32_t)__shfl((int)(w.sign | (uint32_t)w.root.n << 1), from, 64);
+  const bool other = takes && cmd != bd.cmd;
+  before(other);
+  const uint64_t fold = __ballot(other && bd.cmd != 0xFFFFFFFFu);
+  if (fold) fold_bounds(bounds, fold, bd);
+  if (other) bd.reset(cmd);
+  edge::P half[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) half[i] = edge::P{__shfl(w.top[i].x, from, 64), __shfl(w.top[i].y, from, 64)};
+  if (takes) w.start(half, (int)(how >> 1), how & 1u);
+  if (gives) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) w.root.p[i] = w.m.p[i];
+    w.level = w.path = 0;
+  }
+  return takes;
+}
+
 // Source segments -> 24.8 edge segments, in one pass.
 //
 // A curve of ten segments next to one of a single segment leaves most lanes
@@ -366,15 +501,6 @@ __device__ __forceinline__ void fold_bounds(CmdBounds* __restrict__ bounds, uint
 // 380 -> 100 us, 10 000 cubic paths 418 -> 213, 2000 pattern shapes 65 -> 29,
 // a frame of panels 64 -> 27.
 constexpr uint32_t kLaneStage = 4;
-constexpr uint32_t kMaxLevel = 31;
-// A root is shared from this bend on (squared distance of its control points
-// from the chord over the squared tolerance; a split divides it by 16): each
-// half then needs a split of its own.  k_edges in us at 1 (any split one) / 16 /
-// 64 / 256 / 4096 / never: 10 000 cubic paths 312 / 213 / 233 / 239 / 310 / 418,
-// uneven canvases 117 / 100 / 117 / 121 / 168 / 380, panels 27 / 27 / 31 / 31 /
-// 40 / 64, glyph canvases (three segments a quad) 1258 / 881 / 875 / 872 / 875 /
-// 874.
-constexpr double kShareBend = 16.0;
 struct EdgeWave {
   DevSeg seg[kLaneStage][64];
   double cv[8][64];    // each lane's source curve, transformed (x, y)
@@ -403,13 +529,10 @@ __global__ __launch_bounds__(256) void k_edges(FrameDev f, FrameScratch s, uint3
   edge::P at{0.0, 0.0};          // end point of the last piece
   double t_cut = 0.0;
   int n_cuts = 0, cut_i = 0;
-  typename B::Mono root, m;      // the piece, and the node of it in hand
-  root.n = 3; root.sp = 0;
-  m.n = 3; m.sp = 0;
-  edge::P top[4];                // right half of the last split
-  uint32_t level = 0, path = 0;  // of the node in hand
-  int32_t ax = 0, ay = 0;        // last point of the chain
-  uint32_t sign = 0;
+  int points = 3;
+  CurveWalk<B> walk;
+  walk.root.n = walk.m.n = 3;
+  walk.sign = 0;
   bool crossing = false;         // the curve leaves the clip box of `size`
   uint32_t size = 0;
 
@@ -495,7 +618,7 @@ __global__ __launch_bounds__(256) void k_edges(FrameDev f, FrameScratch s, uint3
             any |= fl;
           }
           int32_t lx0 = 0, ly0 = 0, lx1 = 0, ly1 = 0;   // a line's or border line's segment
-          root.n = m.n = npts;
+          points = npts;
           if (npts == 2) {
             if (any) to_clip = true;
             else {
@@ -547,7 +670,7 @@ __global__ __launch_bounds__(256) void k_edges(FrameDev f, FrameScratch s, uint3
         bool to_clip = false;
         edge::P p[4];
         if (mode == kPiece) {
-          const bool quad = root.n == 3;
+          const bool quad = points == 3;
           edge::P cv[4];
 #pragma unroll
           for (int i = 0; i < 4; i++) cv[i] = edge::P{ws.cv[2 * i][lane], ws.cv[2 * i + 1][lane]};
@@ -568,7 +691,7 @@ __global__ __launch_bounds__(256) void k_edges(FrameDev f, FrameScratch s, uint3
             t_cut = t;
           }
           at = p[3];
-          sign = p[0].y > at.y ? 1u : 0u;
+          const uint32_t sign = p[0].y > at.y ? 1u : 0u;
           // from the top down: first and last point, and the control points
           // kept between them
           const edge::P a = sign ? p[3] : p[0], z = sign ? p[0] : p[3];
@@ -608,17 +731,13 @@ __global__ __launch_bounds__(256) void k_edges(FrameDev f, FrameScratch s, uint3
           }
           if (mode == kFlat) {
             const double xl = edge::dmin(a.x, z.x), xr = edge::dmax(a.x, z.x);
-            root.p[0] = a;
-            root.p[1] = edge::P{edge::dclamp(c1.x, xl, xr), edge::dclamp(c1.y, a.y, z.y)};
-            root.p[2] = quad ? z : edge::P{edge::dclamp(c2.x, xl, xr), edge::dclamp(c2.y, a.y, z.y)};
-            root.p[3] = z;
-            m = root;
-            level = path = 0;
-            ax = edge::trunc_i(a.x);
-            ay = edge::trunc_i(a.y);
+            const edge::P from_top[4] = {
+              a, edge::P{edge::dclamp(c1.x, xl, xr), edge::dclamp(c1.y, a.y, z.y)},
+              quad ? z : edge::P{edge::dclamp(c2.x, xl, xr), edge::dclamp(c2.y, a.y, z.y)}, z};
+            walk.start(from_top, points, sign);
           }
         }
-        if (__ballot(to_clip)) clip_put(to_clip, p, (uint32_t)root.n);
+        if (__ballot(to_clip)) clip_put(to_clip, p, (uint32_t)points);
       }
 
       // flatten, a step for every lane at a time, until enough lanes wait
@@ -627,89 +746,14 @@ __global__ __launch_bounds__(256) void k_edges(FrameDev f, FrameScratch s, uint3
         if (!busy) break;
         if (__popcll(busy) < 40 && (next < end || __ballot(mode == kPiece) != 0ull)) break;
         if (__ballot(staged == kLaneStage)) flush();
-        bool halved = false;   // the lane's root: `m` and `top` are all there is of it
-        if (mode == kFlat) {
-          double bend, limit;
-          B::flatness(m, f.tol_sq, bend, limit);
-          if (level != kMaxLevel && !(bend <= limit)) {
-            B::halves(m, top);
-            halved = level == 0 && bend > kShareBend * limit;
-            level++;
-            path <<= 1;
-          }
-          else {
-            const edge::P l = m.p[3];   // (a quad's last point too)
-            const int32_t nx = edge::trunc_i(l.x), ny = edge::trunc_i(l.y);
-            if (ay != ny) put(ax, ay, nx, ny, sign);
-            ax = nx;
-            ay = ny;
-            // the next node: up while it was a right half, then the right
-            // half beside it
-            const uint32_t ups = (uint32_t)__builtin_ctz(~path);
-            if (ups >= level) mode = cut_i == n_cuts ? kIdle : kPiece;
-            else {
-              level -= ups;
-              path = (path >> ups) + 1u;
-#pragma unroll
-              for (int i = 0; i < 4; i++) m.p[i] = top[i];
-              if (ups) {
-#pragma unroll
-                for (int i = 0; i < 4; i++) m.p[i] = root.p[i];
-                for (uint32_t k = level; k-- > 0;) {
-                  edge::P r[4];
-                  B::halves(m, r);
-                  if ((path >> k) & 1u) {
-#pragma unroll
-                    for (int i = 0; i < 4; i++) m.p[i] = r[i];
-                  }
-                }
-              }
-              if (path == (1u << level) - 1u) {   // nothing waits above it: a root of its own
-#pragma unroll
-                for (int i = 0; i < 4; i++) root.p[i] = m.p[i];
-                level = path = 0;
-              }
-            }
-          }
-        }
-        // No sources left: lanes that have just halved their root keep the
-        // first half as theirs and hand the other to lanes that wait.
+        bool halved = false;
+        if (mode == kFlat && !walk.step(f.tol_sq, halved, put)) mode = cut_i == n_cuts ? kIdle : kPiece;
         if (next >= end) {
-          const uint64_t give = __ballot(halved), idle = __ballot(mode == kIdle);
-          if (give && idle) {
-            const uint32_t n = min((uint32_t)__popcll(give), (uint32_t)__popcll(idle));
-            const bool gives = halved && (uint32_t)__popcll(give & below) < n;
-            const uint32_t rank = (uint32_t)__popcll(idle & below);
-            const bool takes = mode == kIdle && rank < n;
-            if (gives) ws.giver[__popcll(give & below)] = lane;
-            wave_sync();
-            const int from = takes ? (int)ws.giver[rank] : (int)lane;
-            wave_sync();
-            const uint32_t cmd = (uint32_t)__shfl((int)bd.cmd, from, 64);
-            const uint32_t how = (uint32_t)__shfl((int)(sign | (uint32_t)root.n << 1), from, 64);
-            const bool other = takes && cmd != bd.cmd;
-            if (__ballot(other && staged)) flush();
-            const uint64_t fold = __ballot(other && bd.cmd != 0xFFFFFFFFu);
-            if (fold) fold_bounds(s.bounds, fold, bd);
-            if (other) bd.reset(cmd);
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-              const double x = __shfl(top[i].x, from, 64), y = __shfl(top[i].y, from, 64);
-              if (takes) m.p[i] = edge::P{x, y};
-            }
-            if (takes) {
-              sign = how & 1u;
-              root.n = m.n = (int)(how >> 1);
-              ax = edge::trunc_i(m.p[0].x);
-              ay = edge::trunc_i(m.p[0].y);
-              cut_i = n_cuts = 0;
-              mode = kFlat;
-            }
-            if (takes || gives) {
-#pragma unroll
-              for (int i = 0; i < 4; i++) root.p[i] = m.p[i];
-              level = path = 0;
-            }
+          if (share_halves(walk, ws.giver, halved, mode == kIdle, bd, s.bounds, [&](bool other) {
+                if (__ballot(other && staged)) flush();
+              })) {
+            cut_i = n_cuts = 0;
+            mode = kFlat;
           }
         }
       }
@@ -722,10 +766,18 @@ __global__ __launch_bounds__(256) void k_edges(FrameDev f, FrameScratch s, uint3
 }
 
 // The clip list: lines and monotonic pieces that leave the canvas, one a lane,
-// through the general builder.
+// through the general builder.  What bounds it is the serial chain of the
+// longest curve, so the builder only follows a curve to where it crosses the
+// clip box: parts inside it are left to the wave, whose lanes share them as
+// k_edges does.  Few items go one to a wave (at least 1 / 4 / 16 a wave: uneven
+// canvases 64 / 75 / 129 us, 2000 pattern shapes 31 / 43 / 63, panels 26 / 30 /
+// 40).  Before, a lane walked its whole curve: uneven canvases 275 -> 64 us,
+// 10 000 cubic paths 163 -> 83, pattern shapes 67 -> 31, panels 38 -> 26, 1024
+// glyph canvases (short curves) 311 -> 289.
 __global__ __launch_bounds__(64) void k_edges_clip(FrameDev f, FrameScratch s) {
   __shared__ EdgeStage stage;
-  __shared__ uint32_t count;
+  __shared__ uint32_t count[2];
+  __shared__ uint32_t giver[64];
   const uint32_t lane = threadIdx.x;
   const uint32_t r = blockIdx.x % s.seg_regions;
   const uint32_t n = min(s.seg_cursor[(kSegRegions + r) * kCursorStep], s.clip_stride);
@@ -735,7 +787,7 @@ __global__ __launch_bounds__(64) void k_edges_clip(FrameDev f, FrameScratch s) {
   bd.reset(0xFFFFFFFFu);
   // few items are spread over many waves: each is a serial chain
   const uint32_t blocks = gridDim.x / s.seg_regions;
-  const uint32_t per = min(64u, max(4u, (n + blocks - 1u) / blocks));
+  const uint32_t per = min(64u, max(1u, (n + blocks - 1u) / blocks));
   for (uint32_t i0 = blockIdx.x / s.seg_regions * per; i0 < n; i0 += blocks * per) {
     const uint32_t i = i0 + lane;
     const bool on = lane < per && i < n;
@@ -745,12 +797,12 @@ __global__ __launch_bounds__(64) void k_edges_clip(FrameDev f, FrameScratch s) {
     if (fold) fold_bounds(s.bounds, fold, bd);
     if (other) bd.reset(cmd);
     out.flush();
-    if (lane == 0) count = 0u;
+    if (lane < 2u) count[lane] = 0u;
     wave_sync();
     if (on) {
       const ClipItem it = items[i];
       const edge::Clip clip = canvas_clip(f.xforms[cmd].canvas_size);
-      ClipEmit emit{out, &count, bd};
+      ClipEmit emit{out, count, bd};
       edge::Builder<ClipEmit> b(emit, clip, f.tol_sq);
       const edge::P* ip = (const edge::P*)it.p;
       if (it.n == 2) b.line(ip[0], ip[1]);
@@ -761,7 +813,44 @@ __global__ __launch_bounds__(64) void k_edges_clip(FrameDev f, FrameScratch s) {
       if (b.invalid) fail_cmd(s, cmd, b.invalid);
     }
     wave_sync();
-    out.staged = min((uint32_t)__builtin_amdgcn_readfirstlane((int)count), kEdgeStage);
+    const uint32_t n_inner = min((uint32_t)__builtin_amdgcn_readfirstlane((int)count[1]), kInnerList);
+    if (n_inner) {
+      CurveWalk<edge::Builder<ClipEmit>> walk;
+      walk.root.n = walk.m.n = 3;
+      walk.sign = 0;
+      bool busy = false;
+      uint32_t next = 0;
+      for (;;) {
+        const uint64_t idle = __ballot(!busy);
+        if (idle && next < n_inner) {
+          const uint32_t at = next + (uint32_t)__popcll(idle & ((1ull << lane) - 1ull));
+          const bool takes = !busy && at < n_inner;
+          next += min((uint32_t)__popcll(idle), n_inner - next);
+          const uint32_t c = takes ? stage.inner_cmd[at] : 0u;
+          const bool changes = takes && c != bd.cmd;
+          const uint64_t old = __ballot(changes && bd.cmd != 0xFFFFFFFFu);
+          if (old) fold_bounds(s.bounds, old, bd);
+          if (changes) bd.reset(c);
+          if (takes) {
+            edge::P p[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) p[i] = edge::P{stage.inner[2 * i][at], stage.inner[2 * i + 1][at]};
+            const uint32_t how = stage.inner_how[at];
+            walk.start(p, (int)(how >> 1), how & 1u);
+            busy = true;
+          }
+        }
+        if (!__ballot(busy)) break;
+        bool halved = false;
+        if (busy)
+          busy = walk.step(f.tol_sq, halved, [&](int32_t ax, int32_t ay, int32_t bx, int32_t by, uint32_t sg) {
+            ClipEmit{out, count, bd}.push(ax, ay, bx, by, sg);
+          });
+        if (next >= n_inner && share_halves(walk, giver, halved, !busy, bd, s.bounds, [](bool) {})) busy = true;
+      }
+      wave_sync();
+    }
+    out.staged = min((uint32_t)__builtin_amdgcn_readfirstlane((int)count[0]), kEdgeStage);
   }
   out.flush();
   const uint64_t have = __ballot(bd.cmd != 0xFFFFFFFFu);

@@ -115,3 +115,23 @@ def test_few_curves(amd, count, kind):
         else:
             sc.fill_path([S.CMD_MOVE, S.CMD_CUBIC, S.CMD_CUBIC, S.CMD_ON, S.CMD_CLOSE], np.vstack([pts[:4], pts[:1]]))
     _cmp(amd, sc)
+
+
+# curves of all lengths that leave the canvas, from one to many a wave: parts
+# inside it go to the wave's list until that is full, further segments past the
+# staging buffer
+@pytest.mark.parametrize("count", [1, 5, 70, 600])
+@pytest.mark.parametrize("kind", ["quad", "cubic"])
+def test_curves_leaving_the_canvas(amd, count, kind):
+    rng = np.random.default_rng(count)
+    size = np.array([900.0, 700.0])
+    sc = S.Scene(900, 700, S.FMT_A8, 0)
+    for k in range(count):
+        pts = (rng.random((5, 2)) * (3.0 if k % 3 else 1.1) - (1.0 if k % 3 else 0.05)) * size
+        sc.set_fill_rule(k & 1)
+        sc.set_fill_style_rgba32(0x30FFFFFF)
+        if kind == "quad":
+            sc.fill_path([S.CMD_MOVE, S.CMD_QUAD, S.CMD_ON, S.CMD_QUAD, S.CMD_ON, S.CMD_CLOSE], pts[[0, 1, 2, 3, 4, 0]])
+        else:
+            sc.fill_path([S.CMD_MOVE, S.CMD_CUBIC, S.CMD_CUBIC, S.CMD_ON, S.CMD_CLOSE], pts[[0, 1, 2, 3, 0]])
+    _cmp(amd, sc)
