@@ -117,7 +117,7 @@ struct Stats {
 
 // How a frame sizes its segment and bin buffers.
 enum Sizing : uint32_t {
-  kSizeExact = 0,     // counting pass of the edge builder + host read-back
+  kSizeExact = 0,     // the edge builder's counts, read back; larger buffers and a second run if need be
   kSizeLearned = 1,   // the cost model's predictions (pool mode)
   kSizeHistory = 2,   // the previous frame's exact totals (pool mode)
 };

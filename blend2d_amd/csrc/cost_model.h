@@ -1,7 +1,7 @@
 // Learned sizing: a small MLP that predicts, per fill command, how many 24.8
 // edge segments the edge builder will emit and how many (segment, band)
 // copies binning will make.  The predictions size the segment and bin pools
-// so a frame can skip the counting pass of the edge builder; an overflow of
+// so a frame can run the edge builder once whatever buffers it has; an overflow of
 // either pool makes the frame fall back to exact counting, so pixels never
 // depend on the model.
 //

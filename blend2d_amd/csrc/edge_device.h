@@ -63,8 +63,7 @@ struct Builder {
       : out(e), c(clip), tol_sq(t), ax(0), ay(0), asign(0), invalid(0), n_out(0) {}
 
   // Past the segment budget nothing more is emitted and is_flat() holds for
-  // every piece, so the flattening loops only unwind their stacks.  Both the
-  // counting and the writing pass stop at the same segment.
+  // every piece, so the flattening loops only unwind their stacks.
   __device__ __forceinline__ void emit(int32_t x0, int32_t y0, int32_t x1, int32_t y1, uint32_t sign) {
     if (n_out >= kMaxItemSegments) { invalid |= kFailTooManySegments; return; }
     n_out++;
