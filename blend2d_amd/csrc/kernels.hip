@@ -17,6 +17,7 @@
 
 #include "device_types.h"
 #include "edge_device.h"
+#include "group_device.h"
 #include "kernels.h"
 #include "pipe_device.h"
 #include "raster_device.h"
@@ -1309,11 +1310,7 @@ __device__ __forceinline__ void group_setup(const FrameDev& f, const FrameScratc
   const uint32_t rows = cv.h - y0 < (uint32_t)kTileH ? cv.h - y0 : (uint32_t)kTileH;
   const uint32_t a8 = cv.format == kFmtA8 ? 1u : 0u;
   const uint64_t ptr = cv.ptr + (uint64_t)((int64_t)y0 * cv.stride) + (uint64_t)x0 * (a8 ? 1u : 4u);
-  const DevCmd& first = f.cmds[cv.cmd_base];
-  const DevStyle& fs = f.styles[first.style];
-  const uint32_t fresh = first.kind == kCmdBoxA && first.alpha == 255u && fs.kind == kFetchSolid &&
-                         (first.op == kOpSrcCopy || (first.op == kOpSrcOver && (fs.solid >> 24) == 255u)) && first.box[0] <= (int)x0 && first.box[1] <= (int)y0 &&
-                         first.box[2] >= (int)min(cv.w, x0 + kGroupTiles * kTileW) && first.box[3] >= (int)(y0 + rows);
+  const uint32_t fresh = starts_opaque(cv, f.cmds, f.styles, x0, y0, min(cv.w, x0 + kGroupTiles * kTileW), y0 + rows) ? 1u : 0u;
   uint4* h = s.group_hdr + 2 * (size_t)slot;
   h[0] = make_uint4(lo, s.list_off[row_base], s.list_off[row_base + cv.n_cmds], col | (band << 16));
   h[1] = make_uint4((uint32_t)ptr, (uint32_t)(ptr >> 32), (uint32_t)cv.stride,
