@@ -63,13 +63,17 @@ enum CmdFail : uint32_t {
   // (raster/edgebuilder_p.h:1494-1496, 1584-1586,
   // raster/rastercontextops.cpp:38-45).
   kFailInvalidGeometry = 1,
-  // One edge work item flattened to more than kMaxItemSegments segments
-  // (control points astronomically far apart): the fill is dropped and
-  // reported as BL_ERROR_OUT_OF_MEMORY instead of being flattened on to the
-  // subdivision limit.
+  // One monotonic piece of a curve flattened to more than kMaxItemSegments
+  // segments or took more than kMaxItemSplits splits (control points
+  // astronomically far apart): the fill is dropped and reported as
+  // BL_ERROR_OUT_OF_MEMORY instead of being flattened on to the subdivision
+  // limit, or for ever.
   kFailTooManySegments = 2,
 };
 constexpr uint32_t kMaxItemSegments = 1u << 22;
+// (pieces that end at all took up to about 1000, over millions of curves with
+// control points of up to 1e308 on canvases up to 65535 pixels a side)
+constexpr uint32_t kMaxItemSplits = 1u << 16;
 
 // Source geometry unit processed by one edge-builder thread.
 enum SrcKind : uint32_t {

@@ -13,8 +13,15 @@
 // reference's merged accumulation.
 #pragma once
 
-#include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#if defined(__HIPCC__)
+#include <hip/hip_runtime.h>
+#else   // the host, for its checks
+#include <math.h>
+#define __device__
+#define __forceinline__ inline
+#endif
 
 #include "device_types.h"
 
@@ -26,7 +33,14 @@ struct P { double x, y; };
 __device__ __forceinline__ double dmin(double a, double b) { return b < a ? b : a; }
 __device__ __forceinline__ double dmax(double a, double b) { return a < b ? b : a; }
 __device__ __forceinline__ double dclamp(double v, double lo, double hi) { return dmin(hi, dmax(lo, v)); }
-__device__ __forceinline__ int trunc_i(double x) { return (int)x; }
+// (the device's conversion: out of range saturates, NaN gives 0)
+__device__ __forceinline__ int trunc_i(double x) {
+#if defined(__HIPCC__)
+  return (int)x;
+#else
+  return x != x ? 0 : x >= 2147483647.0 ? INT32_MAX : x <= -2147483648.0 ? INT32_MIN : (int)x;
+#endif
+}
 __device__ __forceinline__ P psub(P a, P b) { return P{a.x - b.x, a.y - b.y}; }
 __device__ __forceinline__ P pmid(P a, P b) { return P{(a.x + b.x) * 0.5, (a.y + b.y) * 0.5}; }
 __device__ __forceinline__ double cross(P a, P b) { return a.x * b.y - a.y * b.x; }
@@ -58,9 +72,10 @@ struct Builder {
   uint32_t asign;
   uint32_t invalid;     // CmdFail bits
   uint32_t n_out;       // segments emitted so far
+  uint32_t n_split;     // nodes that weren't flat so far
 
   __device__ Builder(Emit& e, const Clip& clip, double t)
-      : out(e), c(clip), tol_sq(t), ax(0), ay(0), asign(0), invalid(0), n_out(0) {}
+      : out(e), c(clip), tol_sq(t), ax(0), ay(0), asign(0), invalid(0), n_out(0), n_split(0) {}
 
   // Past the segment budget nothing more is emitted and is_flat() holds for
   // every piece, so the flattening loops only unwind their stacks.
@@ -249,13 +264,16 @@ struct Builder {
     P f = mfirst(m), l = mlast(m);
     for (int i = 1; i < m.n - 1; i++) { m.p[i].x = dclamp(m.p[i].x, l.x, f.x); m.p[i].y = dclamp(m.p[i].y, f.y, l.y); }
   }
-  __device__ __forceinline__ bool is_flat(const Mono& m) const {
-    return (invalid & kFailTooManySegments) || flat_enough(m, tol_sq);
-  }
-  __device__ __forceinline__ static bool flat_enough(const Mono& m, double tol_sq) {
+  // Points that overflow while they are halved, or that a cut made infinite or
+  // NaN, can give nodes that no number of splits makes flat: past the budget
+  // of splits every node counts as flat and the fill fails.
+  __device__ __forceinline__ bool is_flat(const Mono& m) {
     double value, limit;
     flatness(m, tol_sq, value, limit);
-    return value <= limit;
+    if (value <= limit || (invalid & kFailTooManySegments)) return true;
+    if (n_split++ < kMaxItemSplits) return false;
+    invalid |= kFailTooManySegments;
+    return true;
   }
   // Squared distance of the control points from the chord, and the most that
   // counts as flat (both times the chord's squared length).
@@ -719,6 +737,116 @@ RTL_AddLine:
     const uint32_t sign = sp[0].y > sp[npts - 1].y;
     if (any) flatten_unsafe(m, sp, sign, stack);
     else flatten_safe(m, sp, sign, stack);
+  }
+};
+
+// Where a monotonic piece of a curve that leaves the clip box goes.
+enum PieceWay : uint32_t {
+  kPieceInside,    // strictly inside the box: flattened as a curve inside it is
+  kPieceLine,      // one segment: a piece no wider than a 256th, or the border line of one left or right of the box
+  kPieceNothing,
+  kPieceClip,      // the clip list
+};
+
+// The piece `p` (a quad's end point twice) with the end points `a`, `z` from
+// the top down; `line`: its segment, y0 < y1, without a sign.  Control points
+// that overflow while the curve is cut are left to the clip list, whose
+// splits are bounded: no comparison below holds for a NaN.
+__device__ __forceinline__ PieceWay place_piece(const Clip& clip, const P p[4], P a, P z, DevSeg& line) {
+  const double sum = ((p[0].x + p[1].x) + (p[2].x + p[3].x)) + ((p[0].y + p[1].y) + (p[2].y + p[3].y));
+  if (!isfinite(sum)) return kPieceClip;
+  const double x_lo = dmin(dmin(p[0].x, p[1].x), dmin(p[2].x, p[3].x)), x_hi = dmax(dmax(p[0].x, p[1].x), dmax(p[2].x, p[3].x));
+  const double y_lo = dmin(dmin(p[0].y, p[1].y), dmin(p[2].y, p[3].y)), y_hi = dmax(dmax(p[0].y, p[1].y), dmax(p[2].y, p[3].y));
+  if (y_lo >= clip.y0 && y_hi < clip.y1 && x_lo > clip.x0 && x_hi < clip.x1) {
+    if (!(__builtin_fabs(a.x - z.x) <= 0.00390625)) return kPieceInside;
+    line = DevSeg{trunc_i(a.x), trunc_i(a.y), trunc_i(z.x), trunc_i(z.y)};
+    return line.y0 != line.y1 ? kPieceLine : kPieceNothing;
+  }
+  if (y_hi < clip.y0 || y_lo > clip.y1) return kPieceNothing;
+  if (x_hi < clip.x0 || x_lo > clip.x1) {
+    const int32_t x = x_hi < clip.x0 ? clip.ix0 : clip.ix1;
+    const double ys = dmax(a.y, clip.y0), ye = dmin(z.y, clip.y1);
+    line = DevSeg{x, trunc_i(ys), x, trunc_i(ye)};
+    return ys < ye && line.y0 != line.y1 ? kPieceLine : kPieceNothing;
+  }
+  return kPieceClip;
+}
+
+constexpr uint32_t kMaxLevel = 31;
+// A root is shared from this bend on (squared distance of its control points
+// from the chord over the squared tolerance; a split divides it by 16): each
+// half then needs a split of its own.  k_edges in us at 1 (any split one) / 16 /
+// 64 / 256 / 4096 / never: 10 000 cubic paths 312 / 213 / 233 / 239 / 310 / 418,
+// uneven canvases 117 / 100 / 117 / 121 / 168 / 380, panels 27 / 27 / 31 / 31 /
+// 40 / 64, glyph canvases (three segments a quad) 1258 / 881 / 875 / 872 / 875 /
+// 874.
+constexpr double kShareBend = 16.0;
+
+// One lane's curve in the flattening: a monotonic piece inside the clip box
+// (the root), and the node of it in hand.
+template<typename B>
+struct CurveWalk {
+  typename B::Mono root, m;
+  P top[4];              // right half of the last split
+  uint32_t level, path;        // of the node in hand
+  int32_t ax, ay;              // last point of the chain
+  uint32_t sign;
+
+  __device__ __forceinline__ void start(const P p[4], int n, uint32_t sg) {
+    root.n = m.n = n;
+#pragma unroll
+    for (int i = 0; i < 4; i++) root.p[i] = m.p[i] = p[i];
+    level = path = 0;
+    sign = sg;
+    ax = trunc_i(p[0].x);
+    ay = trunc_i(p[0].y);
+  }
+  // Splits the node in hand, or emits it and goes on to the next.  (Flatness
+  // that is NaN must not split: starting again from a root of its own, no
+  // level would ever be the last.)  False when that was the last; `halved`: the root was split and is worth sharing (`m`
+  // and `top` are all there is of it).
+  template<typename Put>
+  __device__ __forceinline__ bool step(double tol_sq, bool& halved, Put&& put) {
+    double bend, limit;
+    B::flatness(m, tol_sq, bend, limit);
+    if (level != kMaxLevel && bend > limit) {
+      B::halves(m, top);
+      halved = level == 0 && bend > kShareBend * limit;
+      level++;
+      path <<= 1;
+      return true;
+    }
+    const P l = m.p[3];   // (a quad's last point too)
+    const int32_t nx = trunc_i(l.x), ny = trunc_i(l.y);
+    if (ay != ny) put(ax, ay, nx, ny, sign);
+    ax = nx;
+    ay = ny;
+    // the next node: up while it was a right half, then the right half beside
+    // it
+    const uint32_t ups = (uint32_t)__builtin_ctz(~path);
+    if (ups >= level) return false;
+    level -= ups;
+    path = (path >> ups) + 1u;
+#pragma unroll
+    for (int i = 0; i < 4; i++) m.p[i] = top[i];
+    if (ups) {
+#pragma unroll
+      for (int i = 0; i < 4; i++) m.p[i] = root.p[i];
+      for (uint32_t k = level; k-- > 0;) {
+        P r[4];
+        B::halves(m, r);
+        if ((path >> k) & 1u) {
+#pragma unroll
+          for (int i = 0; i < 4; i++) m.p[i] = r[i];
+        }
+      }
+    }
+    if (path == (1u << level) - 1u) {   // nothing waits above it: a root of its own
+#pragma unroll
+      for (int i = 0; i < 4; i++) root.p[i] = m.p[i];
+      level = path = 0;
+    }
+    return true;
   }
 };
 

@@ -340,89 +340,12 @@ __device__ __forceinline__ void fold_bounds(CmdBounds* __restrict__ bounds, uint
   }
 }
 
-constexpr uint32_t kMaxLevel = 31;
-// A root is shared from this bend on (squared distance of its control points
-// from the chord over the squared tolerance; a split divides it by 16): each
-// half then needs a split of its own.  k_edges in us at 1 (any split one) / 16 /
-// 64 / 256 / 4096 / never: 10 000 cubic paths 312 / 213 / 233 / 239 / 310 / 418,
-// uneven canvases 117 / 100 / 117 / 121 / 168 / 380, panels 27 / 27 / 31 / 31 /
-// 40 / 64, glyph canvases (three segments a quad) 1258 / 881 / 875 / 872 / 875 /
-// 874.
-constexpr double kShareBend = 16.0;
-
-// One lane's curve in the flattening: a monotonic piece inside the clip box
-// (the root), and the node of it in hand.
-template<typename B>
-struct CurveWalk {
-  typename B::Mono root, m;
-  edge::P top[4];              // right half of the last split
-  uint32_t level, path;        // of the node in hand
-  int32_t ax, ay;              // last point of the chain
-  uint32_t sign;
-
-  __device__ __forceinline__ void start(const edge::P p[4], int n, uint32_t sg) {
-    root.n = m.n = n;
-#pragma unroll
-    for (int i = 0; i < 4; i++) root.p[i] = m.p[i] = p[i];
-    level = path = 0;
-    sign = sg;
-    ax = edge::trunc_i(p[0].x);
-    ay = edge::trunc_i(p[0].y);
-  }
-  // Splits the node in hand, or emits it and goes on to the next.  False when
-  // that was the last; `halved`: the root was split and is worth sharing (`m`
-  // and `top` are all there is of it).
-  template<typename Put>
-  __device__ __forceinline__ bool step(double tol_sq, bool& halved, Put&& put) {
-    double bend, limit;
-    B::flatness(m, tol_sq, bend, limit);
-    if (level != kMaxLevel && !(bend <= limit)) {
-      B::halves(m, top);
-      halved = level == 0 && bend > kShareBend * limit;
-      level++;
-      path <<= 1;
-      return true;
-    }
-    const edge::P l = m.p[3];   // (a quad's last point too)
-    const int32_t nx = edge::trunc_i(l.x), ny = edge::trunc_i(l.y);
-    if (ay != ny) put(ax, ay, nx, ny, sign);
-    ax = nx;
-    ay = ny;
-    // the next node: up while it was a right half, then the right half beside
-    // it
-    const uint32_t ups = (uint32_t)__builtin_ctz(~path);
-    if (ups >= level) return false;
-    level -= ups;
-    path = (path >> ups) + 1u;
-#pragma unroll
-    for (int i = 0; i < 4; i++) m.p[i] = top[i];
-    if (ups) {
-#pragma unroll
-      for (int i = 0; i < 4; i++) m.p[i] = root.p[i];
-      for (uint32_t k = level; k-- > 0;) {
-        edge::P r[4];
-        B::halves(m, r);
-        if ((path >> k) & 1u) {
-#pragma unroll
-          for (int i = 0; i < 4; i++) m.p[i] = r[i];
-        }
-      }
-    }
-    if (path == (1u << level) - 1u) {   // nothing waits above it: a root of its own
-#pragma unroll
-      for (int i = 0; i < 4; i++) root.p[i] = m.p[i];
-      level = path = 0;
-    }
-    return true;
-  }
-};
-
 // Lanes that have just halved their root keep the first half as theirs and
 // hand the other to lanes that wait (all lanes call it).  True for a lane that
 // got one, its bounds being those of the curve's command then; before(other)
 // is called by all lanes, `other` where a lane changes its command.
 template<typename B, typename Before>
-__device__ __forceinline__ bool share_halves(CurveWalk<B>& w, uint32_t* giver, bool halved, bool waits, LaneBounds& bd,
+__device__ __forceinline__ bool share_halves(edge::CurveWalk<B>& w, uint32_t* giver, bool halved, bool waits, LaneBounds& bd,
                                              CmdBounds* bounds, Before&& before) {
   const uint32_t lane = threadIdx.x & 63u;
   const uint64_t below = (1ull << lane) - 1ull;
@@ -475,10 +398,10 @@ __device__ __forceinline__ bool share_halves(CurveWalk<B>& w, uint32_t* giver, b
 //
 // A source that crosses the clip box goes to the clip list, whole lines or the
 // monotonic pieces of a curve: its walk is long and branchy, and k_edges_clip
-// gives every piece a lane.  A curve inside the box is at most 65535 pixels
-// across, and each split cuts its distance from its chord to a quarter, so it
-// is flat after about ten: the subdivision and segment limits of the general
-// builder cannot be reached here.
+// gives every piece a lane.  A piece inside the box is finite and at most 65535
+// pixels across, and each split cuts its distance from its chord to a quarter,
+// so it is flat after about ten: the subdivision, split and segment limits of
+// the general builder cannot be reached here.
 //
 // Each lane stages up to four segments in LDS; a flush writes them lane by
 // lane, so the segments of a contour stay together (binning gathers equal
@@ -531,7 +454,7 @@ __global__ __launch_bounds__(256) void k_edges(FrameDev f, FrameScratch s, uint3
   double t_cut = 0.0;
   int n_cuts = 0, cut_i = 0;
   int points = 3;
-  CurveWalk<B> walk;
+  edge::CurveWalk<B> walk;
   walk.root.n = walk.m.n = 3;
   walk.sign = 0;
   bool crossing = false;         // the curve leaves the clip box of `size`
@@ -699,36 +622,11 @@ __global__ __launch_bounds__(256) void k_edges(FrameDev f, FrameScratch s, uint3
           edge::P c1 = quad ? p[1] : sign ? p[2] : p[1], c2 = quad ? z : sign ? p[1] : p[2];
           mode = kFlat;
           if (crossing) {
-            // strictly inside the clip box: as a curve inside it, except that
-            // one no wider than a 256th is a single line; strictly left or
-            // right of it: its border line; strictly above or below:
-            // nothing; anything else goes to the clip list
-            const edge::Clip clip = canvas_clip(size);
-            const double x_lo = edge::dmin(edge::dmin(p[0].x, p[1].x), edge::dmin(p[2].x, p[3].x));
-            const double x_hi = edge::dmax(edge::dmax(p[0].x, p[1].x), edge::dmax(p[2].x, p[3].x));
-            const double y_lo = edge::dmin(edge::dmin(p[0].y, p[1].y), edge::dmin(p[2].y, p[3].y));
-            const double y_hi = edge::dmax(edge::dmax(p[0].y, p[1].y), edge::dmax(p[2].y, p[3].y));
-            const bool rows = y_lo >= clip.y0 && y_hi < clip.y1;
-            if (rows && x_lo > clip.x0 && x_hi < clip.x1) {
-              if (__builtin_fabs(a.x - z.x) <= 0.00390625) {
-                const int32_t y0 = edge::trunc_i(a.y), y1 = edge::trunc_i(z.y);
-                if (y0 != y1) put(edge::trunc_i(a.x), y0, edge::trunc_i(z.x), y1, sign);
-                mode = kPiece;
-              }
-            }
-            else if (y_hi < clip.y0 || y_lo > clip.y1) mode = kPiece;
-            else if (x_hi < clip.x0 || x_lo > clip.x1) {
-              const int32_t x = x_hi < clip.x0 ? clip.ix0 : clip.ix1;
-              const double ys = edge::dmax(a.y, clip.y0), ye = edge::dmin(z.y, clip.y1);
-              const int32_t y0 = edge::trunc_i(ys), y1 = edge::trunc_i(ye);
-              if (ys < ye && y0 != y1) put(x, y0, x, y1, sign);
-              mode = kPiece;
-            }
-            else {
-              to_clip = true;
-              mode = kPiece;
-            }
-            if (mode == kPiece && cut_i == n_cuts) mode = kIdle;
+            DevSeg line;
+            const edge::PieceWay way = edge::place_piece(canvas_clip(size), p, a, z, line);
+            if (way == edge::kPieceLine) put(line.x0, line.y0, line.x1, line.y1, sign);
+            to_clip = way == edge::kPieceClip;
+            if (way != edge::kPieceInside) mode = cut_i == n_cuts ? kIdle : kPiece;
           }
           if (mode == kFlat) {
             const double xl = edge::dmin(a.x, z.x), xr = edge::dmax(a.x, z.x);
@@ -816,7 +714,7 @@ __global__ __launch_bounds__(64) void k_edges_clip(FrameDev f, FrameScratch s) {
     wave_sync();
     const uint32_t n_inner = min((uint32_t)__builtin_amdgcn_readfirstlane((int)count[1]), kInnerList);
     if (n_inner) {
-      CurveWalk<edge::Builder<ClipEmit>> walk;
+      edge::CurveWalk<edge::Builder<ClipEmit>> walk;
       walk.root.n = walk.m.n = 3;
       walk.sign = 0;
       bool busy = false;
