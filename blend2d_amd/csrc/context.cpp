@@ -69,9 +69,18 @@ struct DevBuf {
     if (bytes <= cap) return true;
     if (ptr) { (void)hipFree(ptr); ptr = nullptr; cap = 0; }
     size_t n = std::max<size_t>(bytes + bytes / 4, 4096);
-    if (hipMalloc(&ptr, n) != hipSuccess) { ptr = nullptr; return false; }
+    if (hipMalloc(&ptr, n) != hipSuccess) {
+      ptr = nullptr;
+      (void)hipGetLastError();   // or a later launch check would find it
+      return false;
+    }
     cap = n;
     return true;
+  }
+  void release() {
+    if (ptr) (void)hipFree(ptr);
+    ptr = nullptr;
+    cap = 0;
   }
   template<typename T> T* as() const { return static_cast<T*>(ptr); }
 };
@@ -985,8 +994,9 @@ uint32_t Runner::render_stage(FrameScratch& s, uint32_t n_a, uint32_t n_f, uint3
 
 // Exact sizing: the edge builder writes into the segment buffer the runner has
 // and counts what it needs; after the read-back the buffer is grown and the
-// pass repeated if it did not fit (a first frame of curves).  The second
-// read-back sizes the binned segments and the command lists.
+// pass repeated if it did not fit (a first frame of curves).  A device with no
+// room for the first guess is counted for first.  The second read-back sizes
+// the binned segments and the command lists.
 uint32_t Runner::execute_exact(Stats& stats, ScratchArena* arena, const ExactPlan* known) {
   stats = Stats{};
   auto t0 = std::chrono::steady_clock::now();
@@ -1118,13 +1128,19 @@ uint32_t Runner::execute_exact(Stats& stats, ScratchArena* arena, const ExactPla
     if (arena) {
       if (n_src && !take_clip(item_cap)) return kErrFit;
     }
-    else {
-      if (!take_segs(stride) || (n_src && !reserve_clip(s))) return kErrOOM;
+    else if (take_segs(stride) && (!n_src || reserve_clip(s))) {
       if (n_src) {   // all that the buffers hold
         const size_t slots = std::min<size_t>({segs.cap / sizeof(DevSeg), seg_cmd.cap / 8, (size_t)0x7FFFF000u});
         s.seg_rank = s.seg_cmd + slots;
         s.seg_stride = (uint32_t)(slots / s.seg_regions);
       }
+    }
+    else {
+      // no room on the device for the guess: count first, as in an arena
+      segs.release();
+      seg_cmd.release();
+      clip.release();
+      s.seg_stride = s.clip_stride = 0;
     }
     launch_frame_init(f, s, true, stream);
     while (n_src) {   // a frame of box fills only has no edges: no round trip
