@@ -1198,6 +1198,10 @@ uint32_t Runner::execute_exact(Stats& stats, ScratchArena* arena, const ExactPla
     n_sgroups = host_readback[kCounterTiles + 2];
     n_ggroups = host_readback[kCounterTiles + 3];
     if (n_atiles > f.n_tiles || (uint64_t)n_fgroups + n_sgroups + n_ggroups > f.n_groups) return kErrDevice;
+    // a second edge pass needs what the first one counted; more would have been
+    // dropped without a word
+    for (uint32_t r = 0; n_src && r < s.seg_regions; r++)
+      if (host_readback[kReportCursors + r] > s.seg_stride || host_readback[kReportClip + r] > s.clip_stride) return kErrDevice;
     // every edge segment crosses at least one band and at most all of them;
     // the command lists hold at most one entry per (band, command) cell
     if ((n_binned < n_segs && !some_failed) || (uint64_t)n_binned > (uint64_t)n_segs * std::max<uint32_t>(max_bands(), 1) ||

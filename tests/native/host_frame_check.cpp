@@ -26,15 +26,16 @@ struct Handle { int device; };
 hipError_t fail(hipError_t e) { return g_last = e; }
 
 // What the frame's edges need: segments of k_edges and of its clip list, and
-// clip items, per region.
-uint32_t g_segs = 0, g_clip_segs = 0, g_clip = 0;
+// clip items, per region; from edge pass `later_from` on `later` more segments.
+uint32_t g_segs = 0, g_clip_segs = 0, g_clip = 0, g_later = 0;
+int g_later_from = 1 << 30;
 // Edge passes so far, with their strides.
 struct Pass { uint32_t seg_stride, clip_stride; };
 std::vector<Pass> g_passes;
 FrameScratch g_s{};
 
 uint32_t region_segs() {
-  return g_segs + (g_clip <= g_s.clip_stride ? g_clip_segs : 0u);
+  return g_segs + (g_clip <= g_s.clip_stride ? g_clip_segs : 0u) + ((int)g_passes.size() >= g_later_from ? g_later : 0u);
 }
 
 }  // namespace
@@ -232,12 +233,21 @@ void too_tight() {
   EXPECT(g_passes.size() == 1);
 }
 
+// A second pass that needs more than the first one counted is an error.
+void counts_differ() {
+  Frame fr;
+  set_needs(90000, 500, 400);
+  g_later = 1;
+  g_later_from = 2;
+  EXPECT(fr.flush() == BL_AMD_ERROR_DEVICE);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
   const std::map<std::string, void (*)()> cases = {
     {"enough", enough},           {"more_segments", more_segments}, {"more_clip_items", more_clip_items},
-    {"tight_device", tight_device}, {"too_tight", too_tight}};
+    {"tight_device", tight_device}, {"too_tight", too_tight},       {"counts_differ", counts_differ}};
   const auto it = argc > 1 ? cases.find(argv[1]) : cases.end();
   if (it == cases.end()) return 2;
   it->second();

@@ -33,7 +33,7 @@ def test_line_sources(amd, count):
     _cmp(amd, S.polygons_scene(count, 300, 200, count))
 
 
-# curves that flatten to far more segments than the buffer starts with
+# few long curves, and (40) more segments than the buffer starts with
 @pytest.mark.parametrize("count", [3, 40])
 def test_long_curves(amd, count):
     rng = np.random.default_rng(count)
