@@ -198,17 +198,26 @@ DeviceQueue& device_queue() {
 // the caller's rows while the next one is on its way.  hipMemcpy2D into
 // pageable memory takes 5-7 us a row instead: a 129 x 229 A8 image 1.57 ms
 // against 0.02, 1920 x 1080 PRGB32 7.7 ms against 0.4-0.9.  Shared by all threads,
-// two fixed chunks, kept until the process ends.
+// two fixed chunks, kept until the process ends; on the device that first read
+// back.
 struct Downloader {
   static constexpr size_t kChunk = (size_t)1 << 20;   // an image row is at most 256 KB
   std::mutex mu;
   uint8_t* pinned = nullptr;
   hipEvent_t done[2] = {nullptr, nullptr};
+  int device = -1;   // the events'
+  // False: not to be had, or the calling thread's device is another one, whose
+  // null stream takes no event of the first.
   bool init() {
-    if (!pinned && hipHostMalloc((void**)&pinned, 2 * kChunk, hipHostMallocDefault) != hipSuccess) { pinned = nullptr; return false; }
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || (device >= 0 && dev != device)) return false;
+    device = dev;
+    if (!pinned && hipHostMalloc((void**)&pinned, 2 * kChunk, hipHostMallocDefault) != hipSuccess) pinned = nullptr;
     for (hipEvent_t& e : done)
-      if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) { e = nullptr; return false; }
-    return true;
+      if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) e = nullptr;
+    if (pinned && done[0] && done[1]) return true;
+    (void)hipGetLastError();   // or a later launch check would find it
+    return false;
   }
   // Rows of `row` bytes from device memory (rows `src_stride` apart) to host
   // memory (rows `dst_stride` apart), behind the work of the null stream as

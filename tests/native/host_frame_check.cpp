@@ -242,12 +242,29 @@ void counts_differ() {
   EXPECT(fr.flush() == BL_AMD_ERROR_DEVICE);
 }
 
+// Images are read back whatever device is current.
+void other_device() {
+  for (int pass = 0; pass < 2; pass++)
+    for (int dev = 0; dev < 2; dev++) {
+      g_device = dev;
+      BLAmdImage* img = nullptr;
+      EXPECT(bl_amd_image_create(&img, 33, 21, BL_AMD_FORMAT_PRGB32) == 0);
+      std::vector<uint32_t> in(33 * 21), out(33 * 21);
+      for (size_t i = 0; i < in.size(); i++) in[i] = (uint32_t)(i * 2654435761u) + (uint32_t)dev;
+      EXPECT(bl_amd_image_upload(img, in.data(), 33 * 4) == 0);
+      EXPECT(bl_amd_image_download(img, out.data(), 33 * 4) == 0);
+      EXPECT(in == out);
+      bl_amd_image_destroy(img);
+    }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
   const std::map<std::string, void (*)()> cases = {
     {"enough", enough},           {"more_segments", more_segments}, {"more_clip_items", more_clip_items},
-    {"tight_device", tight_device}, {"too_tight", too_tight},       {"counts_differ", counts_differ}};
+    {"tight_device", tight_device}, {"too_tight", too_tight},       {"counts_differ", counts_differ},
+    {"other_device", other_device}};
   const auto it = argc > 1 ? cases.find(argv[1]) : cases.end();
   if (it == cases.end()) return 2;
   it->second();
