@@ -343,9 +343,9 @@ BLAmdResult bl_amd_set_graph_replay(uint32_t on);
 /* No counterpart in the reference.  For callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc): bl_amd_context_replay with exact sizing, whose
- * intermediate buffers (edge work items and segments, binned segments,
+ * intermediate buffers (edge segments and clip list, binned segments,
  * band matrices and lists, tile headers, counters) are slices of one
- * 64 MiB device region that the library holds per device for the life of
+ * 80 MiB device region that the library holds per device for the life of
  * the process; it calls no hipMalloc / hipFree.  A frame whose buffers do
  * not fit fails with BL_AMD_ERROR_DATA_TOO_LARGE before anything is
  * composited.  Every call on a device shares the region and leaves it dirty

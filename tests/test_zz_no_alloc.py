@@ -68,3 +68,23 @@ def test_noalloc_replay_rejects_a_frame_larger_than_its_region(amd):
     assert r == E_DATA_TOO_LARGE
     assert (img.download() == 0x12345678).all()
     ctx.end()
+
+
+def test_noalloc_replay_takes_the_long_curves_it_took(amd):
+    # frames just below what 64 MiB held at 20 bytes a segment and 88 a piece
+    # (three a quad), above what it holds at 24 and 72
+    n = 26400
+    rng = np.random.default_rng(1)
+    sc = S.Scene(3000, 800, S.FMT_A8, 0)
+    sc.set_comp_op(S.COMP_OP_PLUS)
+    sc.set_fill_style_rgba32(0x01FFFFFF)
+    for k in range(8):
+        pts = rng.random((2 * (n // 8) + 2, 2)) * [3000.0, 800.0]
+        pts[-2:] = pts[0]
+        sc.set_fill_rule(k & 1)
+        sc.fill_path([S.CMD_MOVE] + [S.CMD_QUAD, S.CMD_ON] * (n // 8) + [S.CMD_CLOSE], pts)
+    (p_ref, st), (p_na, st_na) = _both(amd, sc)
+    binned = 16 * st["binned"]
+    assert 272 * n + 20 * st["segments"] + binned < 64 << 20 < 216 * n + 24 * st["segments"] + binned
+    assert (p_ref == p_na).all()
+    assert st_na["segments"] == st["segments"]
