@@ -1524,6 +1524,37 @@ __device__ __forceinline__ void apply_n(const FrameDev& f, const FrameScratch& s
   pipe::composite32_n<N>(op, d, sp, mm, fetch >= kFetchPatternNN);
 }
 
+// Words px .. px + N - 1 of a row; those past its end stay as they are.
+template<int N>
+__device__ __forceinline__ void load_words(const uint8_t* rowp, int px, int w, uint32_t v[N]) {
+  const uint32_t* r32 = (const uint32_t*)rowp;
+  if (N == 4 && px + 3 < w && (((uintptr_t)(r32 + px)) & 15) == 0) {
+    const uint4 q = *(const uint4*)(r32 + px);
+    const uint32_t u[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+    for (int k = 0; k < N; k++) v[k] = u[k];
+  }
+  else {
+#pragma unroll
+    for (int k = 0; k < N; k++) if (px + k < w) v[k] = r32[px + k];
+  }
+}
+
+template<int N, bool kStream>
+__device__ __forceinline__ void store_words(uint8_t* rowp, int px, int w, const uint32_t v[N]) {
+  uint32_t* r32 = (uint32_t*)rowp;
+  if (N == 4 && px + 3 < w && (((uintptr_t)(r32 + px)) & 15) == 0) {
+    typedef uint32_t words4 __attribute__((ext_vector_type(4)));
+    const words4 q = {v[0], v[1 % N], v[2 % N], v[3 % N]};
+    if (kStream) __builtin_nontemporal_store(q, (words4*)(r32 + px));
+    else *(words4*)(r32 + px) = q;
+  }
+  else {
+#pragma unroll
+    for (int k = 0; k < N; k++) if (px + k < w) r32[px + k] = v[k];
+  }
+}
+
 // Destination pixels px .. px + N - 1 of a row, as pairs (A8: neighbouring
 // pixels in d[k].rb); zero outside the canvas.
 template<int N>
@@ -1545,17 +1576,7 @@ __device__ __forceinline__ void load_px(const uint8_t* rowp, int px, int w, bool
     for (int k = 0; k < (N + 1) / 2; k++) d[k].rb = pipe::u16x2{(uint16_t)v[2 * k], (uint16_t)(2 * k + 1 < N ? v[2 * k + 1 < N ? 2 * k + 1 : 0] : 0u)};
     return;
   }
-  const uint32_t* r32 = (const uint32_t*)rowp;
-  if (N == 4 && px + 3 < w && (((uintptr_t)(r32 + px)) & 15) == 0) {
-    const uint4 q = *(const uint4*)(r32 + px);
-    const uint32_t u[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-    for (int k = 0; k < N; k++) v[k] = u[k];
-  }
-  else {
-#pragma unroll
-    for (int k = 0; k < N; k++) if (px + k < w) v[k] = r32[px + k];
-  }
+  load_words<N>(rowp, px, w, v);
 #pragma unroll
   for (int k = 0; k < N; k++) d[k] = pipe::px_of(v[k]);
 }
@@ -1578,20 +1599,10 @@ __device__ __forceinline__ void store_px(uint8_t* rowp, int px, int w, bool a8, 
     }
     return;
   }
-  uint32_t* r32 = (uint32_t*)rowp;
   uint32_t v[N];
 #pragma unroll
   for (int k = 0; k < N; k++) v[k] = pipe::px_bits(d[k]);
-  if (N == 4 && px + 3 < w && (((uintptr_t)(r32 + px)) & 15) == 0) {
-    typedef uint32_t words4 __attribute__((ext_vector_type(4)));
-    const words4 q = {v[0], v[1 % N], v[2 % N], v[3 % N]};
-    if (kStream) __builtin_nontemporal_store(q, (words4*)(r32 + px));
-    else *(words4*)(r32 + px) = q;
-  }
-  else {
-#pragma unroll
-    for (int k = 0; k < N; k++) if (px + k < w) r32[px + k] = v[k];
-  }
+  store_words<N, kStream>(rowp, px, w, v);
 }
 
 // Rows strip * 4N .. + 4N - 1 of the analytic tile with header `slot`: the
@@ -2041,16 +2052,15 @@ __global__ __launch_bounds__(kQueueBuckets) void k_tile_scatter(FrameDev f, Fram
 // canvas's first command is an opaque colour over the whole group the
 // destination isn't read at all.
 //
-// Instances: solid SRC_OVER / SRC_COPY aligned boxes on 32-bit canvases
-// (fast), other solid styles, and every style.  Measured against one thread
-// per 16 pixels of a row with records in LDS, 4K canvases: four with three
-// translucent layers each 72 -> 40 us (fresh; 54 with the layers composited per
-// pixel), four with an image, a half-size one at a fraction or scaled and 24
-// sprites 422 -> 119, two with a colour through a mask 70 -> 43 and two with a
+// Kernels: solid SRC_OVER / SRC_COPY aligned boxes on 32-bit canvases (one of
+// its own, k_render_box_fast), other solid styles, and every style.  Measured
+// against one thread per 16 pixels of a row with records in LDS, 4K canvases:
+// four with an image, a half-size one at a fraction or scaled and 24 sprites
+// 422 -> 119 us, two with a colour through a mask 70 -> 43 and two with a
 // gradient through another above it 117 -> 48.  What is left there: the vector
 // instructions of the composite, and at 4 waves per SIMD the latency of the
 // header, list and source loads.  Streaming stores took 3 to 6 % off.
-enum BoxClass { kBoxFast, kBoxSolid, kBoxGeneral };
+enum BoxClass { kBoxSolid, kBoxGeneral };
 
 template<int kClass, bool kDither>
 __device__ __forceinline__ void render_box(const FrameDev& f, const FrameScratch& s, uint32_t n) {
@@ -2058,18 +2068,15 @@ __device__ __forceinline__ void render_box(const FrameDev& f, const FrameScratch
   const uint32_t slot = xcd_tile(blockIdx.x);
   if (slot >= n) return;
   // headers: the fast bands' groups first, then the solid ones, then the
-  // general ones.  n is at most the number of all groups: a fast group's header
-  // is loaded together with the counts.
+  // general ones
   const uint32_t n_fast = s.fgroup_off[f.n_bands], n_solid = s.sgroup_off[f.n_bands];
-  const uint32_t count_of = kClass == kBoxFast ? n_fast : kClass == kBoxSolid ? n_solid : s.ggroup_off[f.n_bands];
-  const uint32_t failed = s.flags ? *s.flags : 0u;   // pool overflow: nothing is composited
-  const uint32_t before = kClass == kBoxFast ? 0u : kClass == kBoxSolid ? n_fast : n_fast + n_solid;
-  if (kClass != kBoxFast && (slot >= count_of || failed)) return;
+  if (slot >= (kClass == kBoxSolid ? n_solid : s.ggroup_off[f.n_bands])) return;
+  if (s.flags && *s.flags) return;   // pool overflow: nothing is composited
+  const uint32_t before = kClass == kBoxSolid ? n_fast : n_fast + n_solid;
   const pipe::CPtr<uint32_t> h = pipe::cptr((const uint32_t*)(s.group_hdr + 2 * ((size_t)before + slot)));
   const uint32_t lb = h[1], le = h[2], where = h[3], shape = h[7];
   const uint64_t ptr = ((uint64_t)h[5] << 32) | h[4];
   const int64_t stride = (int32_t)h[6];
-  if (slot >= count_of || failed) return;
   const int lane = threadIdx.x & 63;
   const int row0 = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) * kRows;
   const int rows = min((int)((shape >> 16) & 0x1Fu) - row0, kRows);   // the wave's rows inside the canvas
@@ -2077,7 +2084,7 @@ __device__ __forceinline__ void render_box(const FrameDev& f, const FrameScratch
   const uint32_t tc0 = (where & 0xFFFFu) * kGroupTiles;
   const int X0 = (int)tc0 * kTileW, w = X0 + (int)(shape & 0xFFFFu);
   const int Y = (int)(where >> 16) * kTileH + row0;
-  const bool a8 = kClass != kBoxFast && ((shape >> 21) & 1u);
+  const bool a8 = (shape >> 21) & 1u;
   const bool fresh = (shape >> 22) & 1u;
   const int px = X0 + lane * 4;
   const int xr = min(X0 + (int)kGroupTiles * kTileW, w);   // right end of the group's pixels
@@ -2102,7 +2109,7 @@ __device__ __forceinline__ void render_box(const FrameDev& f, const FrameScratch
   }
   // While the pixels of a fresh group are one value, that value alone is
   // composited.
-  bool one = kClass == kBoxFast ? fresh : fresh && !a8;
+  bool one = fresh && !a8;
   pipe::Px value[1] = {pipe::px_of(0u)};
   auto spread = [&]() {
     if (!one) return;
@@ -2137,7 +2144,7 @@ __device__ __forceinline__ void render_box(const FrameDev& f, const FrameScratch
 
       uint32_t pm[kRows];
       bool full = false;   // one mask, alpha, for every pixel of the group
-      if (kClass == kBoxFast || (meta & 3u) == kCmdBoxA) {
+      if ((meta & 3u) == kCmdBoxA) {
         // a box that goes past the canvas's right edge of the group takes
         // every lane: those pixels are neither counted nor stored, and a whole
         // wave under one mask is cheaper
@@ -2152,7 +2159,7 @@ __device__ __forceinline__ void render_box(const FrameDev& f, const FrameScratch
         if (!c) continue;
         npix += c * (uint32_t)(rb - ra);
         touched |= row_bits;
-        if ((kClass == kBoxFast || (fetch == kFetchSolid && !a8)) && op <= kOpSrcOver && full) {
+        if (fetch == kFetchSolid && !a8 && op <= kOpSrcOver && full) {
           if (one && row_bits == (1u << rows) - 1u) {
             pipe::composite32_flat<1>(op, value, st, alpha);
             continue;
@@ -2184,8 +2191,7 @@ __device__ __forceinline__ void render_box(const FrameDev& f, const FrameScratch
       // Sources that are colours or texels as they lie in memory: the four
       // rows together.
       const uint32_t fmt = (meta >> kMetaFmt) & 3u;
-      if (kClass == kBoxFast ||
-          (!a8 && (fetch == kFetchSolid || (kClass == kBoxGeneral && pipe::fetches_rows(fetch, fmt))))) {
+      if (!a8 && (fetch == kFetchSolid || (kClass == kBoxGeneral && pipe::fetches_rows(fetch, fmt)))) {
         uint32_t src[kRows][4];
 #pragma unroll
         for (int r = 0; r < kRows; r++)
@@ -2214,29 +2220,27 @@ __device__ __forceinline__ void render_box(const FrameDev& f, const FrameScratch
         }
         continue;
       }
-      if constexpr (kClass != kBoxFast) {
-        // the rest a row at a time: the fetchers are long
+      // the rest a row at a time: the fetchers are long
 #pragma unroll 1
-        for (int r = ra; r < rb; r++) {
-          pipe::Px t[4];
-          uint32_t tp = 0;
+      for (int r = ra; r < rb; r++) {
+        pipe::Px t[4];
+        uint32_t tp = 0;
 #pragma unroll
-          for (int q = 0; q < kRows; q++) {
-            if (r != q) continue;
-            tp = pm[q];
+        for (int q = 0; q < kRows; q++) {
+          if (r != q) continue;
+          tp = pm[q];
 #pragma unroll
-            for (int k = 0; k < 4; k++) t[k] = d[q][k];
-          }
-          uint32_t m[4];
+          for (int k = 0; k < 4; k++) t[k] = d[q][k];
+        }
+        uint32_t m[4];
 #pragma unroll
-          for (int k = 0; k < 4; k++) m[k] = (tp >> (8 * k)) & 0xFFu;
-          apply_n<4, kDither>(f, s, meta, cmd, st, a8, 0u, Y + r, px, m, t);
+        for (int k = 0; k < 4; k++) m[k] = (tp >> (8 * k)) & 0xFFu;
+        apply_n<4, kDither>(f, s, meta, cmd, st, a8, 0u, Y + r, px, m, t);
 #pragma unroll
-          for (int q = 0; q < kRows; q++) {
-            if (r != q) continue;
+        for (int q = 0; q < kRows; q++) {
+          if (r != q) continue;
 #pragma unroll
-            for (int k = 0; k < 4; k++) d[q][k] = t[k];
-          }
+          for (int k = 0; k < 4; k++) d[q][k] = t[k];
         }
       }
     }
@@ -2248,8 +2252,109 @@ __device__ __forceinline__ void render_box(const FrameDev& f, const FrameScratch
   if (lane == 0) count_pixels(s, npix);
 }
 
-__global__ __launch_bounds__(kTileThreads) void k_render_box_fast(FrameDev f, FrameScratch s, uint32_t n) {
-  render_box<kBoxFast, false>(f, s, n);
+// Bands of solid SRC_OVER / SRC_COPY aligned boxes on 32-bit canvases, the pure
+// compositing load, where nothing but loads in flight matters: pixels stay
+// words (16 registers a lane) and are taken apart for one command at a time, so
+// that eight waves fit a SIMD.  Ten 4K canvases with one SRC_OVER layer over
+// what they hold: 116 us, 5.7 TB/s; 132 with the pixels as pairs throughout
+// (five waves), 123 with records in LDS.  Four 4K canvases of three translucent
+// layers over an opaque first fill: 31 us against 41 and 73.
+__global__ __launch_bounds__(kTileThreads, 8) void k_render_box_fast(FrameDev f, FrameScratch s, uint32_t n) {
+  constexpr int kRows = 4;
+  const uint32_t slot = xcd_tile(blockIdx.x);
+  if (slot >= n) return;
+  // n is at most the number of all groups: the header, the first in the buffer,
+  // is loaded together with the count and the pool flag
+  const uint32_t n_groups = s.fgroup_off[f.n_bands], failed = s.flags ? *s.flags : 0u;
+  const pipe::CPtr<uint32_t> h = pipe::cptr((const uint32_t*)(s.group_hdr + 2 * (size_t)slot));
+  const uint32_t lb = h[1], le = h[2], where = h[3], shape = h[7];
+  const uint64_t ptr = ((uint64_t)h[5] << 32) | h[4];
+  const int64_t stride = (int32_t)h[6];
+  if (slot >= n_groups || failed) return;
+  const int lane = threadIdx.x & 63;
+  const int row0 = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) * kRows;
+  const int rows = min((int)((shape >> 16) & 0x1Fu) - row0, kRows);   // the wave's rows inside the canvas
+  if (rows <= 0) return;
+  const int X0 = (int)((where & 0xFFFFu) * kGroupTiles) * kTileW, w = X0 + (int)(shape & 0xFFFFu);
+  const int px = X0 + lane * 4;
+  const int xr = min(X0 + (int)kGroupTiles * kTileW, w);   // right end of the group's pixels
+  uint8_t* const base = (uint8_t*)ptr + row0 * stride - (int64_t)X0 * 4;
+  const bool fresh = (shape >> 22) & 1u;
+
+  uint32_t d[kRows][4];
+#pragma unroll
+  for (int r = 0; r < kRows; r++) {
+#pragma unroll
+    for (int k = 0; k < 4; k++) d[r][k] = 0u;
+    if (!fresh && r < rows) load_words<4>(base + r * stride, px, w, d[r]);
+  }
+  // While the pixels of a fresh group are one value, that value alone is
+  // composited.
+  bool one = fresh;
+  uint32_t value = 0u;
+  auto spread = [&]() {
+    if (!one) return;
+    one = false;
+#pragma unroll
+    for (int r = 0; r < kRows; r++)
+#pragma unroll
+      for (int k = 0; k < 4; k++) d[r][k] = value;
+  };
+
+  uint32_t npix = 0, touched = 0;   // touched: bit r, row r
+  for (uint32_t chunk = lb; chunk < le; chunk += 64u) {
+    // up to 64 commands in the lanes
+    const uint32_t li = chunk + (uint32_t)lane;
+    uint32_t box_x = 0, box_meta = 0, style = 0;
+    bool on = false;
+    if (li < le) {
+      const uint4 ent = s.list_ent[li];
+      box_x = ent.y;
+      box_meta = ent.w;
+      style = s.list_style[li];
+      on = (int)(box_x & 0xFFFFu) < xr && (int)(box_x >> 16) > X0 && (int)((box_meta >> kMetaRow0) & 31u) < row0 + rows &&
+           (int)((box_meta >> kMetaRow1) & 31u) > row0 && ((box_meta >> kMetaAlpha) & 0xFFu);
+    }
+    for (uint64_t bits = __ballot(on); bits; bits &= bits - 1ull) {
+      const uint32_t p = (uint32_t)__builtin_ctzll(bits);
+      const uint32_t xs = lane_value(box_x, p), meta = lane_value(box_meta, p), color = lane_value(style, p);
+      const uint32_t alpha = (meta >> kMetaAlpha) & 0xFFu, op = (meta >> kMetaOp) & 7u;
+      const int x0 = (int)(xs & 0xFFFFu), x1 = (int)(xs >> 16);
+      const int ra = max((int)((meta >> kMetaRow0) & 31u) - row0, 0);
+      const int rb = min((int)((meta >> kMetaRow1) & 31u) - row0, rows);   // rows ra .. rb - 1 (not empty)
+      const uint32_t row_bits = (1u << rb) - (1u << ra);
+      touched |= row_bits;
+      npix += (uint32_t)((min(x1, xr) - max(x0, X0)) * (rb - ra));
+      const bool full = x0 <= X0 && x1 >= xr;
+      if (one && full && row_bits == (1u << rows) - 1u) {
+        pipe::Px v[1] = {pipe::px_of(value)};
+        pipe::composite32_flat<1>(op, v, color, alpha);
+        value = pipe::px_bits(v[0]);
+        continue;
+      }
+      spread();
+      // a box over the whole group takes every lane: pixels right of the canvas
+      // aren't stored
+      bool in[4];
+#pragma unroll
+      for (int k = 0; k < 4; k++) in[k] = full || (px + k >= x0 && px + k < x1);
+#pragma unroll
+      for (int r = 0; r < kRows; r++) {
+        if (!((row_bits >> r) & 1u)) continue;
+        pipe::Px v[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) v[k] = pipe::px_of(d[r][k]);
+        pipe::composite32_flat<4>(op, v, color, alpha);
+#pragma unroll
+        for (int k = 0; k < 4; k++) d[r][k] = in[k] ? pipe::px_bits(v[k]) : d[r][k];
+      }
+    }
+  }
+  spread();
+#pragma unroll
+  for (int r = 0; r < kRows; r++)
+    if ((touched >> r) & 1u) store_words<4, true>(base + r * stride, px, w, d[r]);
+  if (lane == 0) count_pixels(s, npix);
 }
 
 __global__ __launch_bounds__(kTileThreads, 3) void k_render_box_solid(FrameDev f, FrameScratch s, uint32_t n) {
