@@ -1,4 +1,4 @@
-// What a tile group of a box-only band starts from.
+// Which kernel takes a band, and what its tile groups start from.
 #pragma once
 
 #include <stdint.h>
@@ -7,6 +7,20 @@
 #include "raster_device.h"
 
 namespace b2amd {
+
+// The kernels in the order of their counts: analytic fills go to the tile
+// kernel, box fills to the compositor of solid SRC_OVER / SRC_COPY aligned boxes
+// on 32-bit canvases, of other solid ones, or of all.
+enum BandClass : uint32_t { kBandTiles = 0, kBandFast = 1, kBandSolid = 2, kBandGeneral = 3, kBandEmpty = 4 };
+
+// `listed`: commands in the band's list.  A band without any belongs to no
+// kernel: the fast compositor, which what follows would give it to, reads words,
+// four times the bytes that a row of an A8 canvas has.
+B2AMD_HD BandClass band_class(uint32_t listed, bool analytic, bool nonsolid, bool slow) {
+  if (listed == 0u) return kBandEmpty;
+  if (analytic) return kBandTiles;
+  return nonsolid ? kBandGeneral : slow ? kBandSolid : kBandFast;
+}
 
 // Whether the canvas's first command copies an opaque colour over all of the
 // canvas's pixels [x0, x1) x [y0, y1), so that what they held doesn't matter.

@@ -999,7 +999,7 @@ __device__ __forceinline__ ScanVal<2> cell_value(const FrameScratch& s, uint64_t
 // The class of band b: analytic fills present (a non-empty binned range) ->
 // its tiles go to k_render; otherwise its tile groups go to k_render_box_fast
 // (solid SRC_OVER / SRC_COPY aligned boxes only), or to k_render_box, the
-// solid or the general instance.
+// solid or the general instance, or, without any command, to none.
 __device__ __forceinline__ ScanVal<4> band_value(const FrameDev& f, const FrameScratch& s, uint64_t b, uint64_t n) {
   ScanVal<4> x{{0u, 0u, 0u, 0u}};
   if (b >= n) return x;
@@ -1010,10 +1010,10 @@ __device__ __forceinline__ ScanVal<4> band_value(const FrameDev& f, const FrameS
   }
   const DevCanvas& cv = f.canvases[lo];
   const uint64_t row_base = cv.mat_base + (b - cv.band_base) * cv.n_cmds;
-  if (s.mat_off[row_base + cv.n_cmds] != s.mat_off[row_base]) x.v[0] = cv.tiles_x;
-  else if (s.band_nonsolid[b]) x.v[3] = cv.groups_x;
-  else if (s.band_slow[b]) x.v[2] = cv.groups_x;
-  else x.v[1] = cv.groups_x;
+  const BandClass c = band_class(s.list_off[row_base + cv.n_cmds] - s.list_off[row_base],
+                                 s.mat_off[row_base + cv.n_cmds] != s.mat_off[row_base], s.band_nonsolid[b] != 0u, s.band_slow[b] != 0u);
+#pragma unroll
+  for (uint32_t k = 0; k < 4u; k++) x.v[k] = c == k ? (k == kBandTiles ? cv.tiles_x : cv.groups_x) : 0u;
   return x;
 }
 

@@ -1,5 +1,5 @@
-// Checks which tile groups start from an opaque colour
-// (blend2d_amd/csrc/group_device.h, compiled here for the host).  The command
+// Checks which kernel takes a band and which tile groups start from an opaque
+// colour (blend2d_amd/csrc/group_device.h, compiled here for the host).  The command
 // and style tables end where a page without access begins, and the command
 // behind the last one, where there is room for one, is a stale one whose style
 // lies far outside its table: a canvas that recorded nothing must not lead to
@@ -89,6 +89,14 @@ int main() {
   expect("empty canvas before stale memory", starts_opaque(none, cmds, styles, 0, 0, 256, 16), false);
   none.cmd_base = 2;
   expect("empty canvas at the end of the table", starts_opaque(none, cmds, styles, 0, 0, 256, 16), false);
+
+  // bands: every class, and none without a command
+  expect("paths", band_class(3, true, false, false) == kBandTiles, true);
+  expect("paths over a gradient", band_class(3, true, true, true) == kBandTiles, true);
+  expect("solid boxes", band_class(1, false, false, false) == kBandFast, true);
+  expect("solid boxes on A8", band_class(1, false, false, true) == kBandSolid, true);
+  expect("gradient boxes", band_class(1, false, true, true) == kBandGeneral, true);
+  expect("no commands", band_class(0, false, false, false) == kBandEmpty, true);
 
   printf("mismatches %d\n", bad);
   return bad ? 1 : 0;

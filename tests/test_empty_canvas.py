@@ -1,9 +1,11 @@
-"""Batches in which a context recorded nothing.  The tile groups of such a
-canvas have no first command to look at: the command behind the last one is
-whatever an earlier, larger frame left there, and its style may lie outside the
-style table.  On the CPU the rule is compiled for the host with tables that end
-at a page without access (tests/native/group_fresh_check.cpp); without its look
-at the command count, planted in a copy, the check dies or fails."""
+"""Canvases and bands that no command touches, and batches in which a context
+recorded nothing.  A band without commands goes to no kernel: the compositor of
+words would read past the end of an A8 canvas.  An empty canvas has no first
+command to look at: the command behind the last one is whatever an earlier,
+larger frame left there, and its style may lie outside the style table.  On the
+CPU both rules are compiled for the host with tables that end at a page without
+access (tests/native/group_fresh_check.cpp); without the look at the counts,
+taken out of a copy, the check dies or fails."""
 import os
 import shutil
 import subprocess
@@ -40,11 +42,32 @@ def test_groups_of_an_empty_canvas_read_no_command(tmp_path):
     assert res.returncode == 0 and "mismatches 0" in res.stdout, res.stderr
 
 
-def test_without_the_command_count_the_check_fails(tmp_path):
+@pytest.mark.parametrize("rule", ["if (cv.n_cmds == 0u) return false;", "if (listed == 0u) return kBandEmpty;"])
+def test_without_a_look_at_the_counts_the_check_fails(tmp_path, rule):
     text = open(os.path.join(CSRC, "group_device.h")).read()
-    planted = text.replace("if (cv.n_cmds == 0u) return false;", "")
+    planted = text.replace(rule, "")
     assert planted != text
     assert _check(tmp_path, planted).returncode != 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt", [S.FMT_A8, S.FMT_PRGB32])
+def test_bands_without_commands_go_to_no_kernel(fmt):
+    import blend2d_amd as amd
+    if amd.lib().bl_amd_device_count() < 1:
+        pytest.skip("no HIP device")
+    sc = S.Scene(256, 256, fmt, 0x21)
+    sc.set_fill_style_rgba32(0xC0FF8040)
+    sc.fill_polygon([(20.0, 40.0), (200.0, 50.0), (90.0, 90.0)])
+    img = amd.BLImage(sc.width, sc.height, sc.format)
+    img.fill_raw(sc.clear_value)
+    ctx = amd.BLContext(img)
+    assert amd.replay_into(ctx, sc, []) == []
+    ctx.flush()
+    assert ctx.last_stats()["render_kernels"] == 1     # the tile kernel alone
+    want, _ = checkers.render_oracle(sc)
+    assert np.array_equal(img.download(), want)
+    ctx.end()
 
 
 @pytest.mark.gpu
