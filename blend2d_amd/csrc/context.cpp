@@ -931,19 +931,28 @@ void Runner::resolve_schedule(uint32_t n_a, uint32_t n_binned, bool allow_queue,
     else if (force_schedule != BL_AMD_SCHEDULE_AUTO) { sched = force_schedule; wgs = force_wgs; }
     else if (g_schedule != BL_AMD_SCHEDULE_AUTO) { sched = g_schedule; wgs = g_queue_wgs; }
     else {
-      // A shape never tuned: longest tiles first when the tiles are a few
-      // rounds of workgroups, where a long one left for the end holds up the
-      // frame; one workgroup per tile for a frame smaller than one round
-      // (strips share out its tiles) or so large that the tail is nothing and
-      // sorting scatters the tiles of a band over the chip.  Render stage ms,
-      // grid against sorted queue: 256 tiles 0.76 / 1.02, 1024 tiles (1000
-      // polygons) 1.01 / 0.90, 2040 (cubics 1080p) 1.98 / 1.84, 8100 (pattern
-      // shapes) 1.22 / 1.21, 15 600 (glyph canvases) 1.77 / 1.51, 170 000
-      // (uneven canvases) 1.94 / 2.43.  Tiles of few segments (40 gradient
-      // panels: 25 a tile) are over before their sorting pays.
+      // A shape never tuned: longest tiles first where a long one left for the
+      // end would hold up the frame.  Render stage ms, grid against sorted queue:
+      //   glyph canvases (330 to 1260 segments a tile) 3700 tiles 0.185 / 0.138,
+      //     16 000 1.80 / 1.47, 32 000 3.33 / 2.97, 65 000 6.40 / 5.93, 97 000
+      //     9.45 / 8.91; with 130 a tile 0.24 / 0.27 and (63 000) 0.87 / 1.01
+      //   polygons 1024 tiles (160 a tile) 1.05 / 0.97, 1536 (110) 1.17 / 1.02,
+      //     2040 (86) 1.35 / 1.35, 4590 (280) 12.0 / 11.5
+      //   cubics 2040 tiles (1870 a tile) 2.04 / 1.85, 8160 7.19 / 7.02, 24 500
+      //     20.9 / 21.2, 65 000 54.5 / 56.5; (125) 1536 0.14 / 0.15
+      //   uneven canvases (4 to 30 a tile) 14 000 0.13 / 0.21, 177 000 1.42 / 2.09
+      // Sorting takes about 25 us and 3 ns a tile, which tiles of few segments
+      // don't pay back (64 a tile within two rounds of workgroups, where the
+      // tail is much of the frame, 256 beyond); and it scatters the tiles of a
+      // band, which read one list, over the chip: a loss in large frames of wide
+      // bands, nothing to bands of four tiles and less.
       auto it = g_tuned.find(shape_key());
       if (it != g_tuned.end()) { sched = it->second.schedule; wgs = it->second.wgs; }
-      else if (strips_for(n_a) == 1 && n_a <= 32768 && n_binned / 64 >= n_a) { sched = BL_AMD_SCHEDULE_QUEUE_HEURISTIC; wgs = 4; }
+      else if (strips_for(n_a) == 1 && n_binned / (n_a <= 2048u ? 64u : 256u) >= n_a &&
+               (n_a <= 16384u || n_a <= 4ull * f.n_bands)) {
+        sched = BL_AMD_SCHEDULE_QUEUE_HEURISTIC;
+        wgs = 4;
+      }
     }
   }
   if (sched == BL_AMD_SCHEDULE_QUEUE_LEARNED && g_tile_model.empty()) sched = BL_AMD_SCHEDULE_QUEUE_HEURISTIC;
@@ -954,12 +963,13 @@ void Runner::resolve_schedule(uint32_t n_a, uint32_t n_binned, bool allow_queue,
 // tiles is rendered with less than one pixel quad per thread: a tile split in
 // strips of 8 or 4 rows has two or four times the waves to hide latency with.
 // The strips repeat the walk over the band's segments, which costs more than
-// it hides once the tiles fill the chip.  Measured on 1000 polygons (render
-// stage ms for 1 / 2 / 4 strips): 64 tiles 1.17 / 0.82 / 0.73, 256 tiles
-// 1.01 / 0.82 / 0.89, 512 tiles 1.12 / 1.02 / 1.22, 1024 tiles
-// 1.33 / 1.47 / 1.94 (before the XCDs shared out the tiles evenly).
+// it hides once the tiles fill the chip.  Render stage ms for 1 / 2 / 4 strips
+// (256 CUs): 1000 polygons on 64 tiles 1.16 / 0.80 / 0.72, 256 1.03 / 0.77 / 0.73,
+// 384 1.02 / 0.78 / 0.77, 512 1.02 / 0.85 / 0.95, 768 1.00 / 0.92 / 1.19, 896
+// 1.03 / 1.04 / 1.33; 2000 cubics on 384 tiles 1.39 / 1.01 / 0.94, 512
+// 0.97 / 0.74 / 0.80, 768 0.70 / 0.60 / 0.71, 960 0.58 / 0.61 / 0.73.
 uint32_t Runner::strips_for(uint32_t n_a) const {
-  return n_a * 2ull <= cus ? 4u : n_a <= cus * 2ull ? 2u : 1u;
+  return n_a * 2ull <= cus * 3ull ? 4u : n_a <= cus * 3ull ? 2u : 1u;
 }
 
 uint32_t Runner::render_stage(FrameScratch& s, uint32_t n_a, uint32_t n_f, uint32_t n_s, uint32_t n_g, uint32_t n_binned,

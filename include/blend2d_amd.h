@@ -423,8 +423,8 @@ BLAmdResult bl_amd_cost_model_train(const float* features, const float* targets,
  *                    runs as QUEUE_HEURISTIC);
  *   AUTO (default)   the schedule the autotuner picked for frames of this
  *                    shape (tile, command and canvas counts, each by its
- *                    power of two), else by a rule on the tile and segment
- *                    counts QUEUE_HEURISTIC or GRID.
+ *                    power of two), else by a rule on the tile, segment and
+ *                    band counts QUEUE_HEURISTIC or GRID.
  * bl_amd_context_replay_noalloc always runs GRID. */
 enum { BL_AMD_SCHEDULE_GRID = 0, BL_AMD_SCHEDULE_QUEUE = 1, BL_AMD_SCHEDULE_QUEUE_HEURISTIC = 2,
        BL_AMD_SCHEDULE_QUEUE_LEARNED = 3, BL_AMD_SCHEDULE_AUTO = 4 };

@@ -33,6 +33,10 @@ int g_later_from = 1 << 30;
 struct Pass { uint32_t seg_stride, clip_stride; };
 std::vector<Pass> g_passes;
 FrameScratch g_s{};
+// Analytic tiles and binned segments that the scans report (0: no tiles, every
+// segment in one band), and how the tiles were launched.
+uint32_t g_tiles = 0, g_binned = 0, g_strips = 0;
+bool g_queue = false;
 
 uint32_t region_segs() {
   return g_segs + (g_clip <= g_s.clip_stride ? g_clip_segs : 0u) + ((int)g_passes.size() >= g_later_from ? g_later : 0u);
@@ -117,17 +121,20 @@ void launch_report(const FrameScratch& s, uint32_t* report, hipStream_t) {
     report[kReportCursors + r] = n;
     report[kReportClip + r] = g_clip;
   }
-  report[kCounterBinned] = n * s.seg_regions;
+  report[kCounterBinned] = g_tiles ? g_binned : n * s.seg_regions;
+  report[kCounterTiles] = g_tiles;
   report[kCounterList] = 1;
 }
 void launch_bin_count(const FrameDev&, const FrameScratch&, uint64_t, hipStream_t) {}
 void launch_scans(const FrameDev&, const FrameScratch&, hipStream_t) {}
 void launch_setup(const FrameDev&, const FrameScratch&, hipStream_t) {}
 void launch_bin_scatter(const FrameDev&, const FrameScratch&, uint64_t, hipStream_t) {}
-void launch_render(const FrameDev&, const FrameScratch&, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, hipStream_t) {}
+void launch_render(const FrameDev&, const FrameScratch&, uint32_t n_a, uint32_t strips, uint32_t, uint32_t, uint32_t, hipStream_t) {
+  if (n_a) g_strips = strips;
+}
 void launch_tile_features(const FrameDev&, const FrameScratch&, uint32_t, hipStream_t) {}
 void launch_tile_queue(const FrameDev&, const FrameScratch&, uint32_t, const float*, hipStream_t) {}
-void launch_render_queue(const FrameDev&, const FrameScratch&, uint32_t, uint32_t, hipStream_t) {}
+void launch_render_queue(const FrameDev&, const FrameScratch&, uint32_t, uint32_t, hipStream_t) { g_queue = true; }
 void launch_fill_u32(uint32_t*, uint32_t, size_t, hipStream_t) {}
 void launch_gradient_luts(const lut::Job*, const lut::Stop*, uint32_t, uint32_t*, hipStream_t) {}
 hipError_t noalloc_scratch(int, void**, size_t*) { return hipErrorNotSupported; }
@@ -152,8 +159,8 @@ constexpr uint32_t kLines = 200000;   // sixteen regions of 12 500
 struct Frame {
   BLAmdImage* img = nullptr;
   BLAmdContext* ctx = nullptr;
-  Frame() {
-    EXPECT(bl_amd_image_create(&img, 640, 480, BL_AMD_FORMAT_PRGB32) == 0);
+  explicit Frame(int w = 640, int h = 480) {
+    EXPECT(bl_amd_image_create(&img, w, h, BL_AMD_FORMAT_PRGB32) == 0);
     EXPECT(bl_amd_context_create(&ctx) == 0);
     EXPECT(bl_amd_context_begin(ctx, img) == 0);
   }
@@ -258,13 +265,50 @@ void other_device() {
     }
 }
 
+// How a frame never tuned runs its analytic tiles, on 256 CUs.
+void schedules() {
+  const struct { int w, h; uint32_t tiles, per_tile, strips; } cases[] = {
+    {640, 480, 1, 1000, 4},        {1024, 1024, 384, 1000, 4},   {1024, 1024, 385, 1000, 2},
+    {1024, 1024, 768, 1000, 2},    {1024, 1024, 769, 1000, 0},   {1024, 1024, 769, 63, 1},
+    {2048, 2048, 2048, 64, 0},     {2048, 2048, 2049, 255, 1},   {2048, 2048, 2049, 256, 0},
+    {8192, 8192, 16384, 256, 0},   {8192, 8192, 16385, 4000, 1}, {512, 65535, 16385, 4000, 1},
+    {256, 65535, 16384, 256, 0},
+  };
+  set_needs(12000, 0, 0);
+  for (const auto& c : cases) {
+    Frame fr(c.w, c.h);
+    g_tiles = c.tiles;
+    g_binned = c.tiles * c.per_tile;
+    g_segs = g_binned / 16 / 20 + 1;
+    g_strips = 0;
+    g_queue = false;
+    EXPECT(fr.flush() == 0);
+    if (g_queue != (c.strips == 0) || g_strips != c.strips)
+      fprintf(stderr, "%u tiles of %u segments: queue %d strips %u\n", c.tiles, c.per_tile, g_queue, g_strips);
+    EXPECT(g_queue == (c.strips == 0) && g_strips == c.strips);
+  }
+  // two canvases of bands of four tiles
+  Frame a(256, 65535), b(256, 65535);
+  BLAmdBatch* batch = nullptr;
+  EXPECT(bl_amd_batch_create(&batch) == 0 && bl_amd_batch_add(batch, a.ctx) == 0 && bl_amd_batch_add(batch, b.ctx) == 0);
+  const double xy[6] = {1, 1, 200, 3, 100, 90};
+  EXPECT(bl_amd_context_fill_polygon_d(a.ctx, xy, 3) == 0 && bl_amd_context_fill_polygon_d(b.ctx, xy, 3) == 0);
+  g_tiles = 32000;
+  g_binned = 256 * 32000;
+  g_segs = 4000;
+  g_queue = false;
+  EXPECT(bl_amd_batch_flush(batch) == 0);
+  EXPECT(g_queue);
+  bl_amd_batch_destroy(batch);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
   const std::map<std::string, void (*)()> cases = {
     {"enough", enough},           {"more_segments", more_segments}, {"more_clip_items", more_clip_items},
     {"tight_device", tight_device}, {"too_tight", too_tight},       {"counts_differ", counts_differ},
-    {"other_device", other_device}};
+    {"other_device", other_device}, {"schedules", schedules}};
   const auto it = argc > 1 ? cases.find(argv[1]) : cases.end();
   if (it == cases.end()) return 2;
   it->second();

@@ -10,7 +10,8 @@ import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 HIP_INCLUDE = "/opt/rocm/include"
-CASES = ["enough", "more_segments", "more_clip_items", "tight_device", "too_tight", "counts_differ", "other_device"]
+CASES = ["enough", "more_segments", "more_clip_items", "tight_device", "too_tight", "counts_differ", "other_device",
+         "schedules"]
 
 
 @pytest.fixture(scope="module")

@@ -30,7 +30,7 @@ def _cmp(amd, sc):
     assert mx == 0, f"max diff {mx}, mean {mean}, {n} channels differ"
 
 
-# 64 x 16 pixel tiles: 1, 4 and 72 (four strips), 130 and 510 (two), 792 (one)
+# 64 x 16 pixel tiles: 1, 4, 72 and 130 (four strips), 510 (two), 792 (one)
 @pytest.mark.parametrize("w,h", [(17, 1), (65, 17), (511, 130), (640, 207), (1025, 480), (1100, 700)])
 @pytest.mark.parametrize("fmt", [S.FMT_PRGB32, S.FMT_XRGB32, S.FMT_A8])
 def test_tile_forms(amd, w, h, fmt):
