@@ -831,7 +831,7 @@ uint32_t Runner::execute_pool(Stats& stats, uint32_t mode) {
   s.seg_regions = edge_plan(f.n_src).regions;
   if (!reserve_clip(s)) return kErrOOM;
 
-  launch_frame_init(f, s, true, stream);
+  launch_frame_init(f, s, stream);
 
   // Pool sizes.
   uint64_t want_segs, want_bins;
@@ -1135,7 +1135,7 @@ uint32_t Runner::execute_exact(Stats& stats, ScratchArena* arena, const ExactPla
   uint32_t n_segs = 0, max_region = 0, max_clip = 0;
   bool some_failed = false;
   if (graph) {
-    launch_frame_init(f, s, true, stream);
+    launch_frame_init(f, s, stream);
     launch_edges(f, s, stream);
     n_segs = known->n_segs;
     some_failed = known->some_failed != 0;
@@ -1161,7 +1161,7 @@ uint32_t Runner::execute_exact(Stats& stats, ScratchArena* arena, const ExactPla
       clip.release();
       s.seg_stride = s.clip_stride = 0;
     }
-    launch_frame_init(f, s, true, stream);
+    launch_frame_init(f, s, stream);
     while (n_src) {   // a frame of box fills only has no edges: no round trip
       launch_edges(f, s, stream);
       launch_report(s, host_readback, stream);
@@ -1182,12 +1182,12 @@ uint32_t Runner::execute_exact(Stats& stats, ScratchArena* arena, const ExactPla
         // more pieces cross the clip box than the list holds: their segments
         // are not counted yet
         if (!take_clip(max_clip)) return kErrFit;
-        launch_frame_init(f, s, true, stream);
+        launch_frame_init(f, s, stream);
         continue;
       }
       if (max_region > s.seg_stride || arena) {
         if (!take_segs(max_region)) return kErrFit;
-        launch_frame_init(f, s, true, stream);
+        launch_frame_init(f, s, stream);
         launch_edges(f, s, stream);
       }
       break;

@@ -61,7 +61,6 @@ __device__ __forceinline__ uint32_t fxf(const Clip& c, P p) { return fx0(c, p) |
 __device__ __forceinline__ uint32_t fyf(const Clip& c, P p) { return fy0(c, p) | fy1(c, p); }
 __device__ __forceinline__ uint32_t fxy(const Clip& c, P p) { return fxf(c, p) | fyf(c, p); }
 
-
 // Emitter receives stored segments: y0 < y1, sign = 1 when the source went up.
 template<typename Emit>
 struct Builder {
@@ -368,21 +367,6 @@ struct Builder {
     return true;
   }
 
-  __device__ void flatten_safe(Mono& m, const P* src, uint32_t sign, P* stack) {
-    mbegin(m, src, sign);
-    asign = sign;
-    if (is_ltr(m)) bound_ltr(m); else bound_rtl(m);
-    open_at(mfirst(m).x, mfirst(m).y);
-    for (;;) {
-      if (!is_flat(m)) {
-        if (m.sp != kLimit) { Step s; msplit(m, s); mpush(m, s, stack); continue; }
-      }
-      add_line(mlast(m).x, mlast(m).y);
-      if (m.sp == 0) break;
-      mpop(m, stack);
-    }
-  }
-
   __device__ void flatten_unsafe(Mono& m, const P* src, uint32_t sign, P* stack) {
     mbegin(m, src, sign);
     asign = sign;
@@ -648,19 +632,6 @@ RTL_AddLine:
     out[1] = P{tp.x - cp.x, tp.y - cp.y};
     out[2] = tp;
   }
-  __device__ int split_quad(const P* cv, P* out) {
-    double ts[3];
-    const int n = cuts_quad(cv, ts);
-    if (n == 0) { out[0] = cv[0]; out[1] = cv[1]; out[2] = cv[2]; return 1; }
-    P at = cv[0];
-    double t_cut = 0.0;
-    for (int i = 0; i < n; i++, out += 2) {
-      piece_quad(cv, t_cut, ts[i], i + 1 == n, at, out);
-      at = out[2];
-      t_cut = ts[i];
-    }
-    return n;
-  }
 
   // The same for a cubic (`ts` holds 8); a parameter may repeat, and the
   // piece that would be empty is skipped.
@@ -710,33 +681,13 @@ RTL_AddLine:
     out[2] = P{tp.x - cp2.x, tp.y - cp2.y};
     out[3] = tp;
   }
-  __device__ int split_cubic(const P* cv, P* out) {
-    double ts[8];
-    const int n = cuts_cubic(cv, ts);
-    if (n == 0) { out[0] = cv[0]; out[1] = cv[1]; out[2] = cv[2]; out[3] = cv[3]; return 1; }
-    P at = cv[0];
-    double t_cut = 0.0;
-    int pieces = 0;
-    for (int i = 0; i < n; i++) {
-      if (ts[i] == t_cut) continue;
-      piece_cubic(cv, t_cut, ts[i], i + 1 == n, at, out);
-      at = out[3];
-      out += 3;
-      pieces++;
-      t_cut = ts[i];
-    }
-    return pieces;
-  }
 
-  // quad_to / cubic_to of one source curve (edgebuilder_p.h:1618-1890): its
-  // monotonic pieces are flattened independently; `any`: a control point lies
-  // outside the clip box.
-  __device__ void curve_piece(const P* sp, int npts, uint32_t any, P* stack) {
+  // One monotonic piece of quad_to / cubic_to of a curve that leaves the clip
+  // box (edgebuilder_p.h:1618-1890); pieces are flattened independently.
+  __device__ void curve_piece(const P* sp, int npts, P* stack) {
     Mono m;
     m.n = npts;
-    const uint32_t sign = sp[0].y > sp[npts - 1].y;
-    if (any) flatten_unsafe(m, sp, sign, stack);
-    else flatten_safe(m, sp, sign, stack);
+    flatten_unsafe(m, sp, sp[0].y > sp[npts - 1].y, stack);
   }
 };
 

@@ -122,9 +122,8 @@ constexpr uint32_t kMetaOp = 2, kMetaAlpha = 5, kMetaEvenOdd = 13, kMetaFetch = 
 
 size_t scan_tmp_words(void);
 
-// Counters, failure bits and bounds; with `cells` also the cell counts, box
-// marks and band flags.
-void launch_frame_init(const FrameDev& f, const FrameScratch& s, bool cells, hipStream_t st);
+// Counters, failure bits, bounds, cell counts, box marks and band flags.
+void launch_frame_init(const FrameDev& f, const FrameScratch& s, hipStream_t st);
 // Writes what the host reads of the counters to pinned memory (kReportWords).
 void launch_report(const FrameScratch& s, uint32_t* report, hipStream_t st);
 

@@ -74,9 +74,9 @@ void launch_fill_u32(uint32_t* p, uint32_t v, size_t n, hipStream_t st) {
 }
 
 // Everything a frame starts from, in one launch: counters and cursors, command
-// failure bits and bounds, and (cells) the (band, command) counts, presence
-// flags and band flags.
-__global__ void k_frame_init(FrameDev f, FrameScratch s, bool cells) {
+// failure bits and bounds, the (band, command) counts, presence flags and band
+// flags.
+__global__ void k_frame_init(FrameDev f, FrameScratch s) {
   const size_t i0 = (size_t)blockIdx.x * blockDim.x + threadIdx.x, step = (size_t)gridDim.x * blockDim.x;
   for (size_t i = i0; i < kCounterWords; i += step) s.counters[i] = 0u;
   for (size_t i = i0; i < f.n_cmds; i += step) {
@@ -85,7 +85,6 @@ __global__ void k_frame_init(FrameDev f, FrameScratch s, bool cells) {
     const DevCanvas& cv = f.canvases[f.cmds[i].canvas];
     s.cmd_bin[i] = CmdBin{(uint32_t)cv.mat_base + (uint32_t)i - cv.cmd_base, cv.n_cmds, cv.bands};
   }
-  if (!cells) return;
   for (size_t i = i0; i < f.n_mat; i += step) {
     s.mat_cnt[i] = 0u;
     s.mat_pres[i] = 0u;
@@ -96,9 +95,9 @@ __global__ void k_frame_init(FrameDev f, FrameScratch s, bool cells) {
   }
 }
 
-void launch_frame_init(const FrameDev& f, const FrameScratch& s, bool cells, hipStream_t st) {
-  const uint64_t n = std::max<uint64_t>({kCounterWords, f.n_cmds, cells ? f.n_mat : 0, cells ? f.n_bands : 0});
-  hipLaunchKernelGGL(k_frame_init, dim3((unsigned)std::min<uint64_t>((n + 255) / 256, 4096)), dim3(256), 0, st, f, s, cells);
+void launch_frame_init(const FrameDev& f, const FrameScratch& s, hipStream_t st) {
+  const uint64_t n = std::max<uint64_t>({kCounterWords, f.n_cmds, f.n_mat, f.n_bands});
+  hipLaunchKernelGGL(k_frame_init, dim3((unsigned)std::min<uint64_t>((n + 255) / 256, 4096)), dim3(256), 0, st, f, s);
 }
 
 // The counters the host reads, into pinned memory: one small launch instead of
@@ -712,7 +711,7 @@ __global__ __launch_bounds__(64) void k_edges_clip(FrameDev f, FrameScratch s) {
       if (it.n == 2) b.line(ip[0], ip[1]);
       else {
         edge::P stack[edge::Builder<ClipEmit>::kLimit * 4];
-        b.curve_piece(ip, (int)it.n, 1u, stack);
+        b.curve_piece(ip, (int)it.n, stack);
       }
       if (b.invalid) fail_cmd(s, cmd, b.invalid);
     }

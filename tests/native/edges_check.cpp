@@ -81,7 +81,7 @@ int cut(const P cv[4], int n, P out[8][4]) {
 uint32_t build(Sink& out, const Clip& clip, const P p[4], int n) {
   P stack[B::kLimit * 4];
   B b(out, clip, out.tol_sq);
-  b.curve_piece(p, n, 1u, stack);
+  b.curve_piece(p, n, stack);
   return b.invalid;
 }
 

@@ -98,7 +98,7 @@ hipError_t hipMemsetD32(hipDeviceptr_t p, int v, size_t n) { for (size_t i = 0; 
 namespace b2amd {
 size_t scan_tmp_words(void) { return 16; }
 EdgePlan edge_plan(uint32_t n_src) { return EdgePlan{8, 1, n_src >= 8192 ? kSegRegions : 1u}; }
-void launch_frame_init(const FrameDev&, const FrameScratch&, bool, hipStream_t) {}
+void launch_frame_init(const FrameDev&, const FrameScratch&, hipStream_t) {}
 void launch_edges(const FrameDev&, const FrameScratch& s, hipStream_t) {
   g_s = s;
   g_passes.push_back(Pass{s.seg_stride, s.clip_stride});
