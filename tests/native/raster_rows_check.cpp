@@ -6,7 +6,8 @@
 // coverage prefix sum at every pixel of the tile (backdrop + tile cells)
 // must equal the sum of the oracle's cells up to that pixel.
 //
-//   raster_rows_check <segments> <seed>     exit status 0 when all agree
+//   raster_rows_check <segments> <seed> [<width> <height>]     exit status 0 when all agree
+// Of a segment of more than 64 rows, the end rows and 40 between are compared.
 #include <stdint.h>
 #include <stdio.h>
 #include <stdlib.h>
@@ -22,9 +23,8 @@ extern "C" int orc_raster_segment(int32_t x0, int32_t y0, int32_t x1, int32_t y1
 
 namespace {
 
-constexpr int kW = 300;       // canvas width in pixels
-constexpr int kH = 40;        // canvas height in pixels
-constexpr int kStride = kW + 8;
+int kW = 300;       // canvas width in pixels
+int kH = 40;        // canvas height in pixels
 
 struct Gen {
   std::mt19937_64 rng;
@@ -45,8 +45,13 @@ struct Gen {
 int main(int argc, char** argv) {
   const long n = argc > 1 ? atol(argv[1]) : 20000;
   const uint64_t seed = argc > 2 ? strtoull(argv[2], nullptr, 10) : 1;
+  if (argc > 4) {
+    kW = atoi(argv[3]);
+    kH = atoi(argv[4]);
+  }
+  const int kStride = kW + 8;
   Gen g(seed);
-  std::vector<uint32_t> cells((size_t)kStride * kH);
+  std::vector<uint32_t> cells((size_t)kStride * kH, 0u);
   long bad = 0, rows_checked = 0;
   for (long i = 0; i < n; i++) {
     int x0, y0, x1, y1;
@@ -76,35 +81,44 @@ int main(int argc, char** argv) {
     if (y0 == y1) continue;
     if (y0 > y1) { std::swap(y0, y1); std::swap(x0, x1); }
     const uint32_t sign = (uint32_t)g.uni(0, 1);
-    std::fill(cells.begin(), cells.end(), 0u);
+    struct Clear {   // the rows the segment touched
+      std::vector<uint32_t>& c;
+      size_t a, b;
+      ~Clear() { std::fill(c.begin() + a, c.begin() + b, 0u); }
+    } clear{cells, (size_t)(y0 >> 8) * kStride, (size_t)(((y1 - 1) >> 8) + 1) * kStride};
     if (!orc_raster_segment(x0, y0, x1, y1, sign, cells.data(), kStride, kH)) continue;
     b2amd::ras::Edge e;
     if (!b2amd::ras::edge_init(e, x0, y0, x1, y1)) { bad++; continue; }
     const int32_t sgn = sign ? -1 : 1;
-    int lefts[8] = {0, 64, 128, 192, 256, g.uni(0, kW - 1), g.uni(0, kW - 1), std::max(0, (x0 >> 8) - g.uni(0, 64))};
-    for (int li = 0; li < 8; li++) {
-      const int xl = lefts[li];
-      const int width = li < 6 ? 64 : g.uni(1, 64);
-      // row by row, in chunks of 1..4 rows
-      std::vector<uint32_t> tile((size_t)(e.row1 - e.row0 + 1) * 64, 0u), bdr(e.row1 - e.row0 + 1, 0u);
-      for (int r = e.row0; r <= e.row1;) {
-        const int last = std::min(e.row1, r + g.uni(0, 3));
-        for (int row = r; row <= last; row++) {
-          bdr[row - e.row0] += b2amd::ras::emit_row(e, row, xl, width, sgn, [&](int32_t k, uint32_t v) {
-            if (k < 0 || k >= width) { bad++; return; }
-            tile[(size_t)(row - e.row0) * 64 + k] += v;
-          });
-        }
-        r = last + 1;
-      }
-      for (int r = e.row0; r <= e.row1; r++) {
-        const uint32_t* row = &cells[(size_t)r * kStride];
-        uint32_t want = 0;
-        for (int x = 0; x < xl && x < kStride; x++) want += row[x];
-        uint32_t got = bdr[r - e.row0];
+    // the rows compared, with the oracle's prefix sums
+    std::vector<int> rows;
+    if (e.row1 - e.row0 < 64)
+      for (int r = e.row0; r <= e.row1; r++) rows.push_back(r);
+    else {
+      rows = {e.row0, e.row0 + 1, e.row1 - 1, e.row1};
+      for (int k = 0; k < 40; k++) rows.push_back(g.uni(e.row0, e.row1));
+    }
+    std::vector<uint32_t> prefix(kStride);
+    for (int r : rows) {
+      const uint32_t* row = &cells[(size_t)r * kStride];
+      uint32_t sum = 0;
+      for (int x = 0; x < kStride; x++) prefix[x] = sum += row[x];
+      // tiles all over the canvas, and those around the row's first cell
+      int first = 0;
+      while (first < kW && !row[first]) first++;
+      const int lefts[8] = {0, std::min(64, kW - 1), std::min(256, kW - 1), first / 64 * 64, g.uni(0, kW - 1), g.uni(0, kW - 1),
+                            std::max(0, (x0 >> 8) - g.uni(0, 64)), std::max(0, first - g.uni(0, 64))};
+      for (int li = 0; li < 8; li++) {
+        const int xl = lefts[li];
+        const int width = li < 6 ? 64 : g.uni(1, 64);
+        uint32_t tile[64] = {};
+        uint32_t got = b2amd::ras::emit_row(e, r, xl, width, sgn, [&](int32_t k, uint32_t v) {
+          if (k < 0 || k >= width) { bad++; return; }
+          tile[k] += v;
+        });
         for (int k = 0; k < width && xl + k < kStride; k++) {
-          want += row[xl + k];
-          got += tile[(size_t)(r - e.row0) * 64 + k];
+          got += tile[k];
+          const uint32_t want = prefix[xl + k];
           if (want != got) {
             if (bad < 10)
               fprintf(stderr, "mismatch: seg (%d,%d)-(%d,%d) sign %u row %d tile %d+%d pixel %d: want %d got %d\n",

@@ -5,7 +5,7 @@ golden canvases): tests/native/raster_rows_check.cpp compares the coverage
 prefix sum of every pixel of every row of random and boundary-hugging
 segments (vertical, near-vertical, flat, on pixel boundaries, both
 directions and signs, 45-degree and very steep ones) for tiles at many
-offsets.  Two planted mistakes in a
+offsets, on small canvases and on some of the longest sides.  Two planted mistakes in a
 copy of the emitter (the rounding term of the row-boundary x, and the
 modulo-256 crossing of steep edges) must make it fail."""
 import os
@@ -36,8 +36,8 @@ def _build(tmp_path, emitter_text=None):
     return exe
 
 
-def _run(exe, n, seed):
-    res = subprocess.run([str(exe), str(n), str(seed)], capture_output=True, text=True)
+def _run(exe, n, seed, *size):
+    res = subprocess.run([str(exe), str(n), str(seed), *map(str, size)], capture_output=True, text=True)
     m = re.search(r"mismatches (\d+)", res.stdout)
     assert m, res.stdout + res.stderr
     return int(m.group(1)), res
@@ -47,6 +47,13 @@ def _run(exe, n, seed):
 def test_row_emitter_matches_the_rasterizer(tmp_path, seed):
     exe = _build(tmp_path)
     bad, res = _run(exe, 60000, seed)
+    assert bad == 0 and res.returncode == 0, res.stderr
+
+
+# long sides: coordinates of 24 bits, dividends of up to 41
+@pytest.mark.parametrize("w,h,n", [(65535, 24, 2500), (24, 65535, 2500), (9000, 4000, 1200)])
+def test_row_emitter_on_large_canvases(tmp_path, w, h, n):
+    bad, res = _run(_build(tmp_path), n, 5, w, h)
     assert bad == 0 and res.returncode == 0, res.stderr
 
 
