@@ -75,7 +75,7 @@ constexpr uint32_t kMaxItemSegments = 1u << 22;
 // control points of up to 1e308 on canvases up to 65535 pixels a side)
 constexpr uint32_t kMaxItemSplits = 1u << 16;
 
-// Source geometry unit processed by one edge-builder thread.
+// Source segments, as the edge builder's lanes take them.
 enum SrcKind : uint32_t {
   kSrcLine = 0,
   kSrcQuad = 1,

@@ -311,9 +311,10 @@ typedef struct BLAmdStats {
                               fills), 2 k_render_box_solid (solid box fills only), 4 k_render_box,
                               8 k_render_box_fast (solid SRC_OVER / SRC_COPY aligned boxes only) */
   double render_ms;    /* device time of the render stage (k_render, k_render_box_solid, k_render_box) */
-  double total_ms;     /* host wall time of the device stages */
+  double total_ms;     /* host wall time of the device stages; in a flush also of what is left of the
+                          frame's transfer and gradient tables, which they wait for */
   double merge_ms;     /* flush: host time merging the batch's recorded frames (0 for one context) */
-  double upload_ms;    /* flush: host time packing and uploading the frame (0 for a replay) */
+  double upload_ms;    /* flush: host time packing the frame and issuing its transfer (0 for a replay) */
   double pack_ms;      /* flush: the part of upload_ms spent packing the frame into staging memory */
   uint32_t schedule;   /* BL_AMD_SCHEDULE_* the analytic tiles ran with (AUTO resolved) */
   uint32_t queue_wgs;  /* queue schedules: workgroups per CU of the persistent grid (0 for GRID) */

@@ -1,7 +1,8 @@
 """The sizing MLP: the numpy checker pinned by finite differences (CPU), the
 GPU forward / gradient / Adam kernels against it, training on logged exact
-counts, and learned sizing end to end (identical pixels, fewer host round
-trips and no counting pass, fewer fallbacks than history sizing)."""
+counts, and learned sizing end to end (identical pixels, as many host round
+trips as exact sizing and the edges built once, fewer fallbacks than history
+sizing)."""
 import numpy as np
 import pytest
 
@@ -164,7 +165,7 @@ def test_learned_sizing_keeps_pixels_and_skips_the_counting_pass(amd, trained):
         history = stats[amd.SIZING_HISTORY][1]
         # 3 host round trips per frame either way (exact: segment count,
         # binned count, end; learned: predicted totals, render-grid counts,
-        # end), but learned sizing runs no counting pass of the edge builder
+        # end), but learned sizing never runs the edge builder twice
         assert all(s["syncs"] == 3 for s in exact_sts)
         ok = [s for s in learned if not s["fallback"]]
         assert len(ok) >= len(learned) - 1
