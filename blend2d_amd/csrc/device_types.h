@@ -64,16 +64,16 @@ enum CmdFail : uint32_t {
   // raster/rastercontextops.cpp:38-45).
   kFailInvalidGeometry = 1,
   // One monotonic piece of a curve flattened to more than kMaxItemSegments
-  // segments or took more than kMaxItemSplits splits (control points
-  // astronomically far apart): the fill is dropped and reported as
-  // BL_ERROR_OUT_OF_MEMORY instead of being flattened on to the subdivision
-  // limit, or for ever.
+  // segments, or came to the subdivision limit or discarded halves more than
+  // kMaxItemOdd times (control points astronomically far apart): the fill is
+  // dropped and reported as BL_ERROR_OUT_OF_MEMORY instead of being flattened
+  // on to the limit, or for ever.
   kFailTooManySegments = 2,
 };
 constexpr uint32_t kMaxItemSegments = 1u << 22;
-// (pieces that end at all took up to about 1000, over millions of curves with
-// control points of up to 1e308 on canvases up to 65535 pixels a side)
-constexpr uint32_t kMaxItemSplits = 1u << 16;
+// (pieces that end at all took up to about 1000, over millions of curves with control
+// points of up to 1e308 on canvases up to 65535 pixels a side)
+constexpr uint32_t kMaxItemOdd = 1u << 16;
 
 // Source segments, as the edge builder's lanes take them.
 enum SrcKind : uint32_t {

@@ -71,10 +71,10 @@ struct Builder {
   uint32_t asign;
   uint32_t invalid;     // CmdFail bits
   uint32_t n_out;       // segments emitted so far
-  uint32_t n_split;     // nodes that weren't flat so far
+  uint32_t n_odd;       // halves discarded and nodes at the subdivision limit so far
 
   __device__ Builder(Emit& e, const Clip& clip, double t)
-      : out(e), c(clip), tol_sq(t), ax(0), ay(0), asign(0), invalid(0), n_out(0), n_split(0) {}
+      : out(e), c(clip), tol_sq(t), ax(0), ay(0), asign(0), invalid(0), n_out(0), n_odd(0) {}
 
   // Past the segment budget nothing more is emitted and is_flat() holds for
   // every piece, so the flattening loops only unwind their stacks.
@@ -263,16 +263,17 @@ struct Builder {
     P f = mfirst(m), l = mlast(m);
     for (int i = 1; i < m.n - 1; i++) { m.p[i].x = dclamp(m.p[i].x, l.x, f.x); m.p[i].y = dclamp(m.p[i].y, f.y, l.y); }
   }
-  // Points that overflow while they are halved, or that a cut made infinite or
-  // NaN, can give nodes that no number of splits makes flat: past the budget
-  // of splits every node counts as flat and the fill fails.
-  __device__ __forceinline__ bool is_flat(const Mono& m) {
+  __device__ __forceinline__ bool is_flat(const Mono& m) const {
     double value, limit;
     flatness(m, tol_sq, value, limit);
-    if (value <= limit || (invalid & kFailTooManySegments)) return true;
-    if (n_split++ < kMaxItemSplits) return false;
-    invalid |= kFailTooManySegments;
-    return true;
+    return (invalid & kFailTooManySegments) || value <= limit;
+  }
+  // Points that overflow while they are halved, or that a cut made infinite or
+  // NaN, can give nodes that no number of splits makes flat.  Their walk keeps
+  // coming to the subdivision limit, or discards half after half: both are
+  // counted, and past the budget every node counts as flat and the fill fails.
+  __device__ __forceinline__ void count_odd() {
+    if (n_odd++ == kMaxItemOdd) invalid |= kFailTooManySegments;
   }
   // Squared distance of the control points from the chord, and the most that
   // counts as flat (both times the chord's squared length).
@@ -337,7 +338,8 @@ struct Builder {
     }
     m.sp++;
   }
-  __device__ __forceinline__ static void mdiscard(Mono& m, const Step& s) {
+  __device__ __forceinline__ void mdiscard(Mono& m, const Step& s) {
+    count_odd();
     if (m.n == 3) { m.p[0] = s.p012; m.p[1] = s.p12; }
     else { m.p[0] = s.p0123; m.p[1] = s.p123; m.p[2] = s.p23; }
   }
@@ -399,6 +401,7 @@ struct Builder {
             msplit(m, s);
             if (step_mid(m, s).y <= c.y0) { mdiscard(m, s); continue; }
             if (m.sp != kLimit) { mpush(m, s, stack); continue; }
+            count_odd();
           }
           if (mlast(m).y > c.y0) {
             out = mlast(m).x < c.x0;
@@ -424,6 +427,7 @@ struct Builder {
               msplit(m, s);
               if (step_mid(m, s).x <= c.x0) { mdiscard(m, s); continue; }
               if (m.sp != kLimit) { mpush(m, s, stack); continue; }
+              count_odd();
             }
             if (mlast(m).x > c.x0) {
 LTR_BeforeX0_Clip:
@@ -455,6 +459,7 @@ LTR_BeforeX0_Pop:
               }
               msplit(m, s);
               if (m.sp != kLimit) { mpush(m, s, stack); continue; }
+              count_odd();
             }
 LTR_AddLine:
             out = mlast(m).x > c.x1;
@@ -495,6 +500,7 @@ LTR_AddLine:
             msplit(m, s);
             if (step_mid(m, s).y <= c.y0) { mdiscard(m, s); continue; }
             if (m.sp != kLimit) { mpush(m, s, stack); continue; }
+            count_odd();
           }
           if (mlast(m).y > c.y0) {
             out = mlast(m).x > c.x1;
@@ -520,6 +526,7 @@ LTR_AddLine:
               msplit(m, s);
               if (step_mid(m, s).x >= c.x1) { mdiscard(m, s); continue; }
               if (m.sp != kLimit) { mpush(m, s, stack); continue; }
+              count_odd();
             }
             if (mlast(m).x < c.x1) {
 RTL_AfterX1_Clip:
@@ -551,6 +558,7 @@ RTL_AfterX1_Pop:
               }
               msplit(m, s);
               if (m.sp != kLimit) { mpush(m, s, stack); continue; }
+              count_odd();
             }
 RTL_AddLine:
             out = mlast(m).x < c.x0;

@@ -404,8 +404,8 @@ __device__ __forceinline__ bool share_halves(edge::CurveWalk<B>& w, uint32_t* gi
 // monotonic pieces of a curve: its walk is long and branchy, and k_edges_clip
 // gives every piece a lane.  A piece inside the box is finite and at most 65535
 // pixels across, and each split cuts its distance from its chord to a quarter,
-// so it is flat after about ten: the subdivision, split and segment limits of
-// the general builder cannot be reached here.
+// so it is flat after about ten: the limits of the general builder cannot be
+// reached here.
 //
 // Each lane stages up to four segments in LDS; a flush writes them lane by
 // lane, so the segments of a contour stay together (binning gathers equal

@@ -2,7 +2,7 @@
 are cut or halved.  tests/native/edges_check.cpp compiles the device edge
 builder for the host and compares every way a piece can take with the general
 builder; two mistakes planted in a copy -- pieces that aren't finite taken as
-inside the canvas, and no budget of splits -- must make it fail or run out of
+inside the canvas, and no budget for those that never get flat -- must make it fail or run out of
 time.  The reference subdivides such a piece to its recursion limit, which takes
 hours, so those that give up have no reference pixels: the fill fails with
 BL_ERROR_OUT_OF_MEMORY and the others are drawn."""
@@ -49,9 +49,9 @@ def test_pieces_that_are_not_finite_taken_as_inside_are_caught(tmp_path):
     assert _check(tmp_path, 1, 1, 10, edges=planted).returncode != 0
 
 
-def test_a_missing_budget_of_splits_is_caught(tmp_path):
+def test_a_missing_budget_is_caught(tmp_path):
     text = open(os.path.join(CSRC, "device_types.h")).read()
-    planted = text.replace("kMaxItemSplits = 1u << 16", "kMaxItemSplits = 0xFFFFFFFFu")
+    planted = text.replace("kMaxItemOdd = 1u << 16", "kMaxItemOdd = 0xFFFFFFFFu")
     assert planted != text
     assert _check(tmp_path, 60000, 1, 2, types=planted).returncode != 0
 
